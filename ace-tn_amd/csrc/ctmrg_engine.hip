@@ -134,27 +134,26 @@ const double* orthonormalize(Ctx& c, double* Y, int64_t m, int64_t q, bool steer
   const int* any = c.launch ? dead + q : nullptr;
   // Gram matrix and inverse factor of src, then dst = src Rinv (or += with acc)
   auto pass = [&](const double* src, double* dst, double shift, double rank_tol, int* dead_out,
-                  const int* only_if, const int* run_if, bool acc) {
+                  const int* run_if, bool acc) {
     GemmDesc gg = dense_desc(qi, qi, mi, true, q, false, q, q);
     gg.run_if = run_if;
     gemm(c, gg, src, src, G);
-    if (c.launch) chol_rinv(G, Rinv, qi, shift, rank_tol, c.st, scr, dead_out, only_if);
+    if (c.launch) chol_rinv(G, Rinv, qi, shift, rank_tol, c.st, scr, dead_out, run_if, !c.mixed);
     GemmDesc gr = dense_desc(mi, qi, qi, false, q, false, q, q, 1.0, acc ? 1.0 : 0.0);
     gr.run_if = run_if;
     gemm(c, gr, src, Rinv, dst);
   };
   // pass 0: shifted (Y -> Yt)
-  pass(Y, Yt, 11.0 * ((double)m * q + (double)q * (q + 1)) * u, 0.0, nullptr, nullptr, nullptr,
-       false);
+  pass(Y, Yt, 11.0 * ((double)m * q + (double)q * (q + 1)) * u, 0.0, nullptr, nullptr, false);
   if (single) return Yt;
   // pass 1: plain with rank guard (Yt -> Y); dropped columns come out zero
-  pass(Yt, Y, 0.0, 1e-14, dead, nullptr, nullptr, false);
+  pass(Yt, Y, 0.0, 1e-14, dead, nullptr, false);
   if (!c.recover) {
     // ACETN_HIP_RF_FAST: dropped columns refilled at random, then the two
     // plain passes (all skipped on the device when none was dropped)
     if (c.launch) refill_dead_columns(Y, m, qi, dead, 0x243F6A8885A308D3ull, c.st);
-    pass(Y, Yt, 0.0, 1e-14, nullptr, dead, any, false);
-    pass(Yt, Y, 0.0, 1e-14, nullptr, dead, any, false);
+    pass(Y, Yt, 0.0, 1e-14, nullptr, any, false);
+    pass(Yt, Y, 0.0, 1e-14, nullptr, any, false);
     return Y;
   }
   // recovery levels; ``prev`` flags the columns still dropped (level 0: the
@@ -170,7 +169,7 @@ const double* orthonormalize(Ctx& c, double* Y, int64_t m, int64_t q, bool steer
     GemmDesc gg = dense_desc(qi, qi, mi, true, q, false, q, q);
     gg.run_if = on;
     gemm(c, gg, Y, Y, G);
-    if (c.launch) chol_rinv(G, Rinv, qi, 0.0, 1e-14, c.st, scr, nullptr, prev);
+    if (c.launch) chol_rinv(G, Rinv, qi, 0.0, 1e-14, c.st, scr, nullptr, on, !c.mixed);
     GemmDesc gt = dense_desc(qi, qi, mi, true, q, false, q, q);
     gt.run_if = on;
     gemm(c, gt, Y, Yt, T);                                   // Y^T Yt
@@ -186,15 +185,15 @@ const double* orthonormalize(Ctx& c, double* Y, int64_t m, int64_t q, bool steer
     // factorise the projected columns and add the ones with rank back: the
     // other columns of Yt are zero (their Rinv columns too), the dropped
     // ones of Y are zero, so Y += Yt Rinv fills exactly the recovered ones
-    pass(Yt, Y, 0.0, 1e-14, next, prev, on, true);
+    pass(Yt, Y, 0.0, 1e-14, next, on, true);
     if (c.launch) still_dead(next, prev, qi, c.st);
     prev = next;
     next = (next == flags_a) ? flags_b : flags_a;
   }
   if (c.launch) refill_dead_columns(Y, m, qi, prev, 0x243F6A8885A308D3ull, c.st);
   // two plain passes over the whole basis (Y -> Yt -> Y)
-  pass(Y, Yt, 0.0, 1e-14, nullptr, dead, any, false);
-  pass(Yt, Y, 0.0, 1e-14, nullptr, dead, any, false);
+  pass(Y, Yt, 0.0, 1e-14, nullptr, any, false);
+  pass(Yt, Y, 0.0, 1e-14, nullptr, any, false);
   return Y;
 }
 

@@ -229,11 +229,15 @@ void gaussian_sketch(double* out, int64_t n, int64_t q, uint64_t seed, uint64_t 
 // (row-major, ld=q), write the upper-triangular inverse factor Rinv (q x q,
 // row-major) with G + shift*I = R^T R.  Columns whose pivot falls below
 // rank_tol * max(diag G) are marked dead: their rows/cols of Rinv are zero.
-// ``only_if_dead`` (device, q ints): when given and all zero, the kernel
-// skips the factorisation and writes Rinv = I (completion passes).
+// ``run_if`` (device flag): when given and zero, the kernel skips the
+// factorisation and writes Rinv = I (completion passes).
+// ``tiles``: the register-tile kernel; off in mixed precision, where the last
+// bits of the basis decide how its bf16 pieces round: the same spectrum to
+// rounding, but boundary tensors that move by 5e-4 (they are resolved to about
+// 1e-7 s_0 / s_k there), so that path keeps the kernel it has always had.
 void chol_rinv(const double* G, double* Rinv, int q, double shift_rel, double rank_tol,
                hipStream_t s, double* gscratch, int* dead_out = nullptr,
-               const int* only_if_dead = nullptr);
+               const int* run_if = nullptr, bool tiles = true);
 // Replace the columns flagged in ``dead`` (device, q ints) of Y (m x q,
 // row-major) by N(0,1) Philox vectors.
 void refill_dead_columns(double* Y, int64_t m, int q, const int* dead, uint64_t seed,

@@ -74,21 +74,12 @@ __global__ __launch_bounds__(LA_NT) void chol_rinv_kernel(const double* __restri
                                                           double* __restrict__ Rinv, int q,
                                                           double shift_rel, double rank_tol,
                                                           double* gscratch, int use_lds,
-                                                          int* dead_out, const int* only_if_dead) {
+                                                          int* dead_out, const int* run_if) {
   extern __shared__ double lds[];
   double* S = kLds ? lds : gscratch;
-  if (only_if_dead) {
-    // completion pass: nothing to do unless an earlier pass refilled a column
-    __shared__ int any;
-    if (threadIdx.x == 0) any = 0;
-    __syncthreads();
-    for (int i = threadIdx.x; i < q; i += LA_NT)
-      if (only_if_dead[i]) any = 1;
-    __syncthreads();
-    if (!any) {
-      for (int e = threadIdx.x; e < q * q; e += LA_NT) Rinv[e] = (e / q == e % q) ? 1.0 : 0.0;
-      return;
-    }
+  if (run_if && *run_if == 0) {
+    for (int e = threadIdx.x; e < q * q; e += LA_NT) Rinv[e] = (e / q == e % q) ? 1.0 : 0.0;
+    return;
   }
   __shared__ double s_red[LA_NT / 64];
   __shared__ double s_trace, s_dmax;
@@ -296,23 +287,15 @@ __global__ __launch_bounds__(CB_NT) void chol_rinv_blk_kernel(const double* __re
                                                               double* __restrict__ Rinv, int q,
                                                               double shift_rel, double rank_tol,
                                                               int* dead_out,
-                                                              const int* only_if_dead) {
+                                                              const int* run_if) {
   extern __shared__ double T[];  // upper tiles
   __shared__ int dead[kCbMaxQ];
   __shared__ double xbuf[32];
   __shared__ double s_red[CB_WAVES][2];
-  __shared__ int any;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  if (only_if_dead) {
-    if (tid == 0) any = 0;
-    __syncthreads();
-    for (int i = tid; i < q; i += CB_NT)
-      if (only_if_dead[i]) any = 1;
-    __syncthreads();
-    if (!any) {
-      for (int e = tid; e < q * q; e += CB_NT) Rinv[e] = (e / q == e % q) ? 1.0 : 0.0;
-      return;
-    }
+  if (run_if && *run_if == 0) {
+    for (int e = tid; e < q * q; e += CB_NT) Rinv[e] = (e / q == e % q) ? 1.0 : 0.0;
+    return;
   }
   double tr = 0.0, dm = 0.0;
   for (int i = tid; i < q; i += CB_NT) {
@@ -430,6 +413,221 @@ __global__ __launch_bounds__(CB_NT) void chol_rinv_blk_kernel(const double* __re
   for (int e = tid; e < q * q; e += CB_NT) {
     const int a = e / q, b = e % q;
     Rinv[e] = (a <= b) ? T[cb_tile(a >> 4, b >> 4) + (a & 15) * CB_LD + (b & 15)] : 0.0;
+  }
+}
+
+// Matrix-core variant for q <= kCtMaxQ, one workgroup: the matrix is cut into
+// 16 x 16 tiles; the off-diagonal ones stay in the waves' registers
+// (accumulator layout) from load to store, and only the diagonal tiles and the
+// current tile row are in LDS.  The factor and its inverse come out of one
+// elimination of [G + shift I | I], which turns the right half into Z = R^-T:
+// with Z_kk = R_kk^-T of the diagonal tile,
+//   panel:     R_kI = Z_kk A_kI (I > k),   Z_kJ = Z_kk Z_kJ (J < k)
+//   trailing:  A_JI -= R_kJ^T R_kI (k < J <= I),  Z_IJ -= R_kI^T Z_kJ (J <= k < I)
+// Tile A(J, I) is dead once row J has been the panel, just when Z(I, J) comes
+// into being, so both live in one slot: Q(Q-1)/2 slots dealt in column order
+// over all waves but the last, which keeps each step's active slots spread
+// evenly.  The bound is latency: per tile row one diagonal factorisation and
+// two barriers.  The last wave updates and factors the next diagonal tile
+// while the others run the trailing update.  Measured against the other
+// kernels here (tiles in LDS with a separate inverse phase up to q = 176,
+// element by element from global memory above): q = 22 10 us against 21,
+// q = 66 24 against 51, q = 146 58 against 120, q = 176 66 against 137,
+// q = 272 144 against 6050.
+constexpr int kCtMaxQ = 272;          // 17 tile rows: 136 slots, 10 a wave (80 VGPRs)
+constexpr int kCtMaxT = kCtMaxQ / 16;
+
+__device__ __forceinline__ double lane_value(double x, int lane) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x), lane),
+                          __builtin_amdgcn_readlane(__double2loint(x), lane));
+}
+
+// One wave: Cholesky of the diagonal tile D (LDS, symmetric) with the rank
+// guard, column j of D in lane j and column j of I in lane 16 + j (the upper
+// half-wave repeats both), rows in registers; the row operations that reduce
+// D to R turn I into Z = R^-T, written to Zs.  dead[c] flags the dead pivots,
+// whose rows of R and rows and columns of Z are zero.
+__device__ __forceinline__ void ct_factor_diag(const double* D, double* Zs, int lane,
+                                               double thresh, int* dead) {
+  // opaque, or the comparisons below are hoisted out of the caller's loop and
+  // held in scalar registers
+  asm volatile("" : "+v"(lane));
+  const int j = lane & 15;
+  const bool id = (lane & 16) != 0;
+  double x[16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) x[i] = id ? (i == j ? 1.0 : 0.0) : D[i * CB_LD + j];
+#pragma unroll
+  for (int c = 0; c < 16; ++c) {
+    const double d = lane_value(x[c], c);
+    const bool dd = !(d > thresh) || !isfinite(d);
+    const double r = dd ? 0.0 : rsqrt(d);
+    x[c] *= r;
+#pragma unroll
+    for (int i = c + 1; i < 16; ++i) x[i] = fma(-lane_value(x[c], i), x[c], x[i]);
+    if (lane == 0) dead[c] = dd ? 1 : 0;
+  }
+  if (lane >= 16 && lane < 32) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) Zs[i * CB_LD + j] = x[i];
+  }
+}
+
+template <int NW, int NS>
+__global__ __launch_bounds__(64 * NW) void chol_rinv_tile_kernel(
+    const double* __restrict__ G, double* __restrict__ Rinv, int q, double shift_rel,
+    double rank_tol, int* dead_out, const int* run_if) {
+  constexpr int NT = 64 * NW, NO = NW - 1;  // waves with slots
+  __shared__ double pan[kCtMaxT][CB_TS];    // the panel: R_kI (I > k), Z_kJ (J < k)
+  __shared__ double dg[kCtMaxT][CB_TS];     // diagonal tiles
+  __shared__ double zk[2][CB_TS];           // Z_kk of this tile row and of the next
+  __shared__ int dead[kCtMaxQ];
+  __shared__ double s_red[NW][2];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  if (run_if && *run_if == 0) {
+    for (int e = tid; e < q * q; e += NT) Rinv[e] = (e / q == e % q) ? 1.0 : 0.0;
+    return;
+  }
+  double tr = 0.0, dm = 0.0;
+  for (int i = tid; i < q; i += NT) {
+    const double gii = G[(int64_t)i * q + i];
+    tr += gii;
+    dm = fmax(dm, gii);
+  }
+  for (int o = 32; o > 0; o >>= 1) { tr += __shfl_down(tr, o); dm = fmax(dm, __shfl_down(dm, o)); }
+  if (lane == 0) { s_red[wave][0] = tr; s_red[wave][1] = dm; }
+  const int Q = (q + 15) / 16;
+  const int m = lane & 15, kq = lane >> 4;
+  __syncthreads();
+  double t0 = 0.0, t1 = 0.0;
+#pragma unroll
+  for (int w = 0; w < NW; ++w) { t0 += s_red[w][0]; t1 = fmax(t1, s_red[w][1]); }
+  const double shift = shift_rel * t0;
+  const double thresh = rank_tol * (t1 + shift);
+  for (int e = tid; e < Q * 256; e += NT) {
+    const int I = e >> 8, x = (e >> 4) & 15, y = e & 15;
+    const int lo = 16 * I + min(x, y), hi = 16 * I + max(x, y);
+    const double v = hi < q ? G[(int64_t)lo * q + hi] : (x == y ? 1.0 : 0.0);  // padding: identity
+    dg[I][x * CB_LD + y] = v + (x == y && hi < q ? shift : 0.0);
+  }
+  __syncthreads();
+
+  auto wave_sync = [&] {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+  // dg[I] -= R_kI^T R_kI
+  auto update_diag = [&](int I) {
+    cb_d4 v;
+    double* D = dg[I];
+    const double* P = pan[I];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] = D[(kq + 4 * r) * CB_LD + m];
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      const double p = P[(4 * ks + kq) * CB_LD + m];
+      v = __builtin_amdgcn_mfma_f64_16x16x4f64(-p, p, v, 0, 0, 0);
+    }
+    wave_sync();
+#pragma unroll
+    for (int r = 0; r < 4; ++r) D[(kq + 4 * r) * CB_LD + m] = v[r];
+  };
+  // The two kinds of waves run loops of their own with the same barriers (two
+  // per tile row): the factorisation's registers then do not add to the slots'.
+  if (wave == NO) {
+    for (int k = 0; k < Q; ++k) {
+      if (k > 0) update_diag(k);
+      double* Zs = zk[k & 1];
+      wave_sync();
+      ct_factor_diag(dg[k], Zs, lane, thresh, dead + 16 * k);
+      wave_sync();
+      for (int e = lane; e < 256; e += 64) {
+        const int a = 16 * k + (e >> 4), b = 16 * k + (e & 15);
+        if (a < q && b < q) Rinv[(int64_t)a * q + b] = Zs[(e & 15) * CB_LD + (e >> 4)];
+      }
+      __syncthreads();
+      __syncthreads();
+    }
+  } else {
+    // this wave's slots: tile (J, I), J < I, of slot t = I (I - 1) / 2 + J, packed J | I << 8
+    int ji[NS];
+    cb_d4 acc[NS];
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      const int t = s * NO + wave;
+      int I = 1;
+      while (I * (I + 1) / 2 <= t) ++I;
+      const int J = t - I * (I - 1) / 2;
+      ji[s] = I < Q ? (J | I << 8) : (255 | 255 << 8);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int a = min(16 * J + kq + 4 * r, q - 1), b = 16 * I + m;
+        const double g = G[(int64_t)a * q + min(b, q - 1)];
+        acc[s][r] = b < q ? g : 0.0;
+      }
+      // one slot at a time here and below: interleaving the slots costs more
+      // registers than the 128 a wave has
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    for (int k = 0; k < Q; ++k) {
+      __syncthreads();
+      const double* Z = zk[k & 1];
+      // keeps the compiler from holding every slot's addresses across the loop
+#pragma unroll
+      for (int s = 0; s < NS; ++s) asm volatile("" : "+s"(ji[s]));
+      // panel: the slots of tile row / column k
+#pragma unroll
+      for (int s = 0; s < NS; ++s) {
+        const int J = ji[s] & 255, I = ji[s] >> 8;
+        if (I == k || J == k) {
+          cb_d4 v = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+          for (int ks = 0; ks < 4; ++ks)
+            v = __builtin_amdgcn_mfma_f64_16x16x4f64(Z[m * CB_LD + 4 * ks + kq], acc[s][ks], v, 0, 0, 0);
+          double* P = pan[I == k ? J : I];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) P[(kq + 4 * r) * CB_LD + m] = v[r];
+          // A(k, I) is done with: the slot starts over as Z(I, k)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) acc[s][r] = 0.0;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      __syncthreads();
+      // Z(k, J), J < k, is final: Rinv(J, k) = Z(k, J)^T
+      for (int e = tid; e < k * 256; e += 64 * NO) {
+        const int J = e >> 8, a = (e >> 4) & 15, b = e & 15;
+        if (16 * k + b < q) Rinv[(int64_t)(16 * J + a) * q + 16 * k + b] = pan[J][b * CB_LD + a];
+      }
+#pragma unroll
+      for (int s = 0; s < NS; ++s) {
+        const int J = ji[s] & 255, I = ji[s] >> 8;
+        if (I > k && I < Q) {
+          const double* A = pan[J > k ? J : I];
+          const double* B = J > k ? pan[I] : (J == k ? Z : pan[J]);
+#pragma unroll
+          for (int ks = 0; ks < 4; ++ks)
+            acc[s] = __builtin_amdgcn_mfma_f64_16x16x4f64(-A[(4 * ks + kq) * CB_LD + m],
+                                                          B[(4 * ks + kq) * CB_LD + m], acc[s], 0, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      for (int I = k + 2 + wave; I < Q; I += NO) update_diag(I);
+    }
+  }
+  // below the diagonal tiles
+  for (int e = tid; e < q * q; e += NT)
+    if ((e / q) >> 4 > (e % q) >> 4) Rinv[e] = 0.0;
+  if (dead_out) {
+    int anyd = 0;
+    for (int i = tid; i < q; i += NT) {
+      dead_out[i] = dead[i];
+      anyd |= dead[i];
+    }
+    anyd = __syncthreads_or(anyd);
+    if (tid == 0) dead_out[q] = anyd;
   }
 }
 
@@ -1171,7 +1369,7 @@ void gaussian_sketch(double* out, int64_t n, int64_t q, uint64_t seed, uint64_t 
 }
 
 void chol_rinv(const double* G, double* Rinv, int q, double shift_rel, double rank_tol,
-               hipStream_t s, double* gscratch, int* dead_out, const int* only_if_dead) {
+               hipStream_t s, double* gscratch, int* dead_out, const int* run_if, bool tiles) {
   ACETN_REQUIRE(q >= 1 && q <= 512, "chol_rinv: q out of range");
   // q^3/3 (factor) + q^3/6 (inverse)
   hipEvent_t e0 = kernel_timing_begin(s);
@@ -1180,6 +1378,22 @@ void chol_rinv(const double* G, double* Rinv, int q, double shift_rel, double ra
     ~End() { if (e0) kernel_timing_end(e0, s, kKCholesky, f, 0.0); }
   } timing_end{e0, s, 0.5 * (double)q * q * q};
   const size_t pb = packed_bytes(q);
+  // fewest waves that hold the slots in registers: a small matrix pays for
+  // every wave at each barrier
+#define ACETN_CT(NW, NS)                                                                        \
+  hipLaunchKernelGGL((chol_rinv_tile_kernel<NW, NS>), dim3(1), dim3(64 * NW), 0, s, G, Rinv, q, \
+                     shift_rel, rank_tol, dead_out, run_if)
+  if (tiles && q <= kCtMaxQ) {
+    const int Q = (q + 15) / 16, slots = Q * (Q - 1) / 2;
+    if (slots <= 2) ACETN_CT(2, 2);
+    else if (slots <= 12) ACETN_CT(4, 4);
+    else if (slots <= 28) ACETN_CT(8, 4);
+    else if (slots <= 60) ACETN_CT(16, 4);
+    else ACETN_CT(16, 10);
+    ACETN_HIP_CHECK(hipGetLastError());
+    return;
+  }
+#undef ACETN_CT
   if (q <= kCbMaxQ) {
     const int Q = (q + 15) / 16;
     const size_t tb = sizeof(double) * (size_t)CB_TS * Q * (Q + 1) / 2;
@@ -1190,7 +1404,7 @@ void chol_rinv(const double* G, double* Rinv, int q, double shift_rel, double ra
       attr = true;
     }
     hipLaunchKernelGGL(chol_rinv_blk_kernel, dim3(1), dim3(CB_NT), tb, s, G, Rinv, q, shift_rel,
-                       rank_tol, dead_out, only_if_dead);
+                       rank_tol, dead_out, run_if);
     ACETN_HIP_CHECK(hipGetLastError());
     return;
   }
@@ -1198,10 +1412,10 @@ void chol_rinv(const double* G, double* Rinv, int q, double shift_rel, double ra
   ACETN_REQUIRE(use_lds || gscratch != nullptr, "chol_rinv: scratch required");
   if (use_lds)
     hipLaunchKernelGGL(chol_rinv_kernel<true>, dim3(1), dim3(LA_NT), pb, s, G, Rinv, q, shift_rel,
-                       rank_tol, gscratch, use_lds, dead_out, only_if_dead);
+                       rank_tol, gscratch, use_lds, dead_out, run_if);
   else
     hipLaunchKernelGGL(chol_rinv_kernel<false>, dim3(1), dim3(LA_NT), 0, s, G, Rinv, q, shift_rel,
-                       rank_tol, gscratch, use_lds, dead_out, only_if_dead);
+                       rank_tol, gscratch, use_lds, dead_out, run_if);
   ACETN_HIP_CHECK(hipGetLastError());
 }
 
