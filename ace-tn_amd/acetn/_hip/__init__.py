@@ -188,6 +188,8 @@ def _declare(lib):
         "acetn_hip_svd_workspace": (c_size, [c_i64, c_i64]),
         "acetn_hip_svd": (ctypes.c_int, [c_vp, c_i64, c_i64, c_i64, c_vp, c_vp,
                                          ctypes.POINTER(ctypes.c_int32), c_vp, c_size, c_vp]),
+        "acetn_hip_gram_svd_workspace": (c_size, [c_i64, c_i64]),
+        "acetn_hip_gram_svd": (ctypes.c_int, [c_vp, c_i64, c_i64, c_vp, c_vp, c_vp, c_size, c_vp]),
         "acetn_hip_eigh_workspace": (c_size, [c_i64]),
         "acetn_hip_eigh": (ctypes.c_int, [c_vp, c_i64, c_vp, c_vp, c_vp, c_size, c_vp]),
         "acetn_hip_orthonormalize_workspace": (c_size, [c_i64, c_i64]),
@@ -479,6 +481,20 @@ def eigh(G):
     ws = workspace(nb, G.device)
     check(lib().acetn_hip_eigh(ptr(G), q, ptr(w), ptr(V), ptr(ws), ws.numel(), stream_handle()))
     return w, V
+
+
+def gram_svd(BT):
+    """The SVD behind the projectors, of B given as BT = B^T (n x q, device
+    FP64): (eigenvalues of B B^T, descending; left singular vectors)."""
+    n, q = BT.shape
+    BT = BT.contiguous()
+    w = torch.empty(q, dtype=torch.float64, device=BT.device)
+    U = torch.empty(q, q, dtype=torch.float64, device=BT.device)
+    nb = lib().acetn_hip_gram_svd_workspace(n, q)
+    ws = workspace(nb, BT.device)
+    check(lib().acetn_hip_gram_svd(ptr(BT), n, q, ptr(w), ptr(U), ptr(ws), ws.numel(),
+                                   stream_handle()))
+    return w, U
 
 
 def rsvd_product(ops, q, niter, mid_qr, seed, stream_id):

@@ -116,6 +116,11 @@ void quarter_tensor(Ctx& c, const acetn_site* s, int k, double* Q, bool f32 = fa
 // precision: the next orthonormalisation restores that).
 constexpr int kRecoverLevels = 3;
 
+// Sketch width from which the projector SVD is preconditioned through the
+// tridiagonal form: its twenty launches cost a small matrix more than the two
+// Jacobi solves take (0.15 ms at q = 22).
+constexpr int kTridiagMinQ = 48;
+
 const double* orthonormalize(Ctx& c, double* Y, int64_t m, int64_t q, bool steer = false) {
   SplitScope sc(c, 0);
   const bool single = steer && c.mixed;
@@ -198,26 +203,86 @@ const double* orthonormalize(Ctx& c, double* Y, int64_t m, int64_t q, bool steer
 }
 
 // ---------------------------------------------------------------------------
-// Singular values / left vectors of B (q x n) given as BT = B^T (n x q):
-// two passes of Gram + Jacobi (the second on the rotated, nearly diagonal
-// Gram matrix restores absolute accuracy eps*s0 for the small values).
+// Singular values / left vectors of B (q x n) given as BT = B^T (n x q).
 // Outputs: w (q, descending eigenvalues of B B^T), UB (q x q).
+//
+// Two passes over the Gram matrix: the first only preconditions (a basis W
+// close to the eigenvectors), the second works on the rotated, nearly diagonal
+// Gram matrix S = (B^T W)^T (B^T W), whose entries are accurate relative to
+// their rows and columns, which restores absolute accuracy eps*s0 for the
+// small values.
+//   * W comes from the tridiagonal form (|G w - l w| ~ eps |G|); vectors of
+//     clustered eigenvalues, which come out independent but not orthogonal,
+//     are orthonormalised by a Cholesky factor of H = W^T W (identity otherwise);
+//   * two refinement steps (I + E_1)(I + E_2), quadratically convergent in the
+//     residual and in W's orthogonality, both on q x q matrices;
+//   * a Jacobi solve of what is left, to 1e-14: nothing but one scan of S
+//     unless there are clusters.
+// A matrix that the tridiagonal route does not serve (judge_basis, on the
+// device: graded spectra, large clusters) is preconditioned by a Jacobi pass on
+// the Gram matrix instead and solved by another to full precision.
+// The eigensolver's kernels, one pair, D=6, chi=144 (q = 146): a Jacobi pass as
+// preconditioner and one to full precision behind it (``signs``, mixed) take
+// 2.45 ms with their replays, this 0.55 ms (tridiagonal form 209 us, vectors
+// 105, a dozen q x q products and the scan); D=4, chi=64: 0.70 against 0.25 ms.
+// ``signs``: the caller hands the vectors out without a sign gauge of its own,
+// so they keep the signs of the Jacobi rotations.  Mixed precision keeps the
+// Jacobi passes too (see chol_rinv's ``tiles``).
 // ---------------------------------------------------------------------------
-void small_svd(Ctx& c, const double* BT, int64_t n, int64_t q, double* w, double* UB) {
+void small_svd(Ctx& c, const double* BT, int64_t n, int64_t q, double* w, double* UB,
+               bool signs = false) {
   SplitScope sc(c, 0);
+  const int qi = (int)q, ni = (int)n;
   double* G = c.take((size_t)q * q);
   double* W1 = c.take((size_t)q * q);
   double* W2 = c.take((size_t)q * q);
   double* w1 = c.take((size_t)q);
   double* B2T = c.take((size_t)n * q);
-  double* rot = c.take(jacobi_rot_elems((int)q));
-  mm(c, (int)q, (int)q, (int)n, true, BT, q, false, BT, q, G, q);
-  // pass 1 only preconditions (pass 2 converges quadratically from ~1e-9)
-  if (c.launch) jacobi_eigh(G, w1, W1, rot, (int)q, c.st, 1e-9);
-  mm(c, (int)n, (int)q, (int)q, false, BT, q, false, W1, q, B2T, q);
-  mm(c, (int)q, (int)q, (int)n, true, B2T, q, false, B2T, q, G, q);
-  if (c.launch) jacobi_eigh(G, w, W2, rot, (int)q, c.st);
-  mm(c, (int)q, (int)q, (int)q, false, W1, q, false, W2, q, UB, q);
+  double* rot = c.take(jacobi_rot_elems(qi));
+  // the refinement's matrices (in every layout, so that one workspace query
+  // serves all modes)
+  double* X = c.take((size_t)q * q);
+  double* H = c.take((size_t)q * q);
+  double* F = c.take((size_t)q * q);
+  double* T = c.take((size_t)q * q);
+  double* S1 = c.take((size_t)q * q);
+  double* H1 = c.take((size_t)q * q);
+  double* F2 = c.take((size_t)q * q);
+  int* robust = c.take_int(2);
+  double* scr = c.take(std::max(tridiag_scratch_elems(qi), (size_t)q * (q + 1) / 2));
+  mm(c, qi, qi, ni, true, BT, q, false, BT, q, G, q);
+  if (q < kTridiagMinQ || q > kTridiagMaxQ || c.mixed || signs) {
+    // the first pass only preconditions (the second converges quadratically from ~1e-9)
+    if (c.launch) jacobi_eigh(G, w1, W1, rot, qi, c.st, 1e-9);
+    mm(c, ni, qi, qi, false, BT, q, false, W1, q, B2T, q);
+    mm(c, qi, qi, ni, true, B2T, q, false, B2T, q, G, q);
+    if (c.launch) jacobi_eigh(G, w, W2, rot, qi, c.st);
+    mm(c, qi, qi, qi, false, W1, q, false, W2, q, UB, q);
+    return;
+  }
+  if (c.launch) tridiag_vectors(G, X, w1, qi, scr, c.st);
+  mm(c, qi, qi, qi, false, X, q, true, X, q, H, q);
+  if (c.launch) chol_rinv(H, T, qi, 0.0, 1e-14, c.st, scr, nullptr, nullptr, true, 1e-4);
+  mm(c, qi, qi, qi, true, X, q, false, T, q, W1, q);
+  mm(c, qi, qi, qi, true, W1, q, false, W1, q, H, q);
+  if (c.launch) {
+    judge_basis(w1, H, qi, robust, c.st);
+    jacobi_eigh(G, w, W1, rot, qi, c.st, 1e-9, robust, -1.0);
+  }
+  mm(c, ni, qi, qi, false, BT, q, false, W1, q, B2T, q);
+  mm(c, qi, qi, ni, true, B2T, q, false, B2T, q, G, q);      // S
+  if (c.launch) refine_eigenvectors(G, H, qi, F, robust, 1e-4, c.st);
+  mm(c, qi, qi, qi, false, G, q, false, F, q, T, q);
+  mm(c, qi, qi, qi, true, F, q, false, T, q, S1, q);         // S_1 = F^T S F
+  mm(c, qi, qi, qi, false, H, q, false, F, q, T, q);
+  mm(c, qi, qi, qi, true, F, q, false, T, q, H1, q);         // H_1 = F^T H F
+  if (c.launch) refine_eigenvectors(S1, H1, qi, F2, robust, 1e-8, c.st);
+  mm(c, qi, qi, qi, false, S1, q, false, F2, q, T, q);
+  mm(c, qi, qi, qi, true, F2, q, false, T, q, G, q);         // S_2
+  mm(c, qi, qi, qi, false, F, q, false, F2, q, T, q);
+  mm(c, qi, qi, qi, false, W1, q, false, T, q, X, q);
+  if (c.launch) jacobi_eigh(G, w, W2, rot, qi, c.st, 2.2e-16, robust, 1e-14);
+  mm(c, qi, qi, qi, false, X, q, false, W2, q, UB, q);
 }
 
 // ---------------------------------------------------------------------------
@@ -283,7 +348,7 @@ void rsvd_product(Ctx& c, int r, const double* const* ops, const int64_t* dims, 
   }
   const double* Qm = orthonormalize(c, Y, m, q);
   apply_t(Qm, Z);                              // Z = M^T Q = B^T
-  small_svd(c, Z, n, q, w, UB);
+  small_svd(c, Z, n, q, w, UB, true);
   if (c.launch) count_kept(w, (int)q, (int)q, 0.0, S, cd, c.st);  // S = sqrt(max(w, 0))
   mm(c, (int)m, (int)q, (int)q, false, Qm, q, false, UB, q, U, q);
   mm(c, (int)n, (int)q, (int)q, false, Z, q, false, UB, q, V, q);
@@ -1466,6 +1531,21 @@ int acetn_hip_svd(const double* M, int64_t rows, int64_t cols, int64_t ldc, doub
     ACETN_HIP_CHECK(hipMemcpyAsync(info, scr, sizeof(info), hipMemcpyDeviceToHost, st));
     ACETN_HIP_CHECK(hipStreamSynchronize(st));
     if (host_sweeps) *host_sweeps = info[1] ? info[0] : -info[0];
+  });
+}
+
+size_t acetn_hip_gram_svd_workspace(int64_t n, int64_t q) {
+  size_t r = 0;
+  guarded([&] { r = measure([&](Ctx& c) { small_svd(c, nullptr, n, q, nullptr, nullptr); }); });
+  return r;
+}
+
+int acetn_hip_gram_svd(const double* BT, int64_t n, int64_t q, double* w, double* U, void* ws,
+                       size_t ws_bytes, void* stream) {
+  return guarded([&] {
+    ACETN_REQUIRE(BT && w && U, "gram_svd: null pointer");
+    ACETN_REQUIRE(q >= 1 && q <= 510 && n >= 1 && n < (int64_t(1) << 31), "gram_svd: bad shape");
+    execute(ws, ws_bytes, stream, [&](Ctx& c) { small_svd(c, BT, n, q, w, U); });
   });
 }
 

@@ -231,13 +231,15 @@ void gaussian_sketch(double* out, int64_t n, int64_t q, uint64_t seed, uint64_t 
 // rank_tol * max(diag G) are marked dead: their rows/cols of Rinv are zero.
 // ``run_if`` (device flag): when given and zero, the kernel skips the
 // factorisation and writes Rinv = I (completion passes).
+// ``near_identity``: Rinv = I also when |G - I| <= near_identity everywhere
+// (tiles only).
 // ``tiles``: the register-tile kernel; off in mixed precision, where the last
 // bits of the basis decide how its bf16 pieces round: the same spectrum to
 // rounding, but boundary tensors that move by 5e-4 (they are resolved to about
 // 1e-7 s_0 / s_k there), so that path keeps the kernel it has always had.
 void chol_rinv(const double* G, double* Rinv, int q, double shift_rel, double rank_tol,
                hipStream_t s, double* gscratch, int* dead_out = nullptr,
-               const int* run_if = nullptr, bool tiles = true);
+               const int* run_if = nullptr, bool tiles = true, double near_identity = -1.0);
 // Replace the columns flagged in ``dead`` (device, q ints) of Y (m x q,
 // row-major) by N(0,1) Philox vectors.
 void refill_dead_columns(double* Y, int64_t m, int q, const int* dead, uint64_t seed,
@@ -254,9 +256,30 @@ void still_dead(int* still, const int* dead, int q, hipStream_t s);
 // the recorded rotations (see jacobi_rot_elems).
 // ``tol``: a pair is rotated while |g_pq| > tol * sqrt(g_pp g_qq); 2.2e-16
 // gives a converged decomposition, a looser value a preconditioning one.
+// ``robust`` (device flag): when given, the solve runs with tolerance tol if it
+// is set and otherwise with tol_else, or not at all (w and V are left alone)
+// when tol_else < 0.
 void jacobi_eigh(double* G, double* w, double* V, double* rot, int q, hipStream_t s,
-                 double tol = 2.2e-16);
+                 double tol = 2.2e-16, const int* robust = nullptr, double tol_else = 0.0);
 size_t jacobi_rot_elems(int q);
+
+// Approximate eigenvectors of the positive semidefinite G (q x q, row-major),
+// row j of X (q x q) the one of the j-th largest eigenvalue: |G x - w x| ~ eps |G|,
+// unit norm, orthogonal except inside clusters of eigenvalues, where they are
+// a well-conditioned random basis of the cluster's subspace (tridiag.hip).
+constexpr int kTridiagMaxQ = 464;
+// lam: the eigenvalues, descending, in units of G's largest diagonal entry.
+void tridiag_vectors(const double* G, double* X, double* lam, int q, double* scratch,
+                     hipStream_t s);
+size_t tridiag_scratch_elems(int q);
+// F = I + E, one refinement step of the basis X with S = X^T G X and
+// H = X^T X (all q x q): X F has the errors of X squared, pairs that call for
+// a rotation above ``most`` left out.  F = I when *robust.
+void refine_eigenvectors(const double* S, const double* H, int q, double* F, const int* robust,
+                         double most, hipStream_t s);
+// *robust <- whether the basis with H = X^T X and eigenvalues lam (descending)
+// should be given up for a Jacobi preconditioner.
+void judge_basis(const double* lam, const double* H, int q, int* robust, hipStream_t s);
 
 // One-sided (Hestenes) Jacobi SVD of the rows x cols matrix M whose column j
 // is stored contiguously at Mc + j * ldc (M(i, j) = Mc[j * ldc + i]),

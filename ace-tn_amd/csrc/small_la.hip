@@ -476,7 +476,7 @@ __device__ __forceinline__ void ct_factor_diag(const double* D, double* Zs, int 
 template <int NW, int NS>
 __global__ __launch_bounds__(64 * NW) void chol_rinv_tile_kernel(
     const double* __restrict__ G, double* __restrict__ Rinv, int q, double shift_rel,
-    double rank_tol, int* dead_out, const int* run_if) {
+    double rank_tol, int* dead_out, const int* run_if, double near_identity) {
   constexpr int NT = 64 * NW, NO = NW - 1;  // waves with slots
   __shared__ double pan[kCtMaxT][CB_TS];    // the panel: R_kI (I > k), Z_kJ (J < k)
   __shared__ double dg[kCtMaxT][CB_TS];     // diagonal tiles
@@ -485,7 +485,14 @@ __global__ __launch_bounds__(64 * NW) void chol_rinv_tile_kernel(
   __shared__ double s_red[NW][2];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  if (run_if && *run_if == 0) {
+  bool skip = run_if && *run_if == 0;
+  if (near_identity >= 0.0) {
+    int off = 0;
+    for (int e = tid; e < q * q; e += NT)
+      off |= !(fabs(G[e] - (e / q == e % q ? 1.0 : 0.0)) <= near_identity);
+    skip = skip || !__syncthreads_or(off);
+  }
+  if (skip) {
     for (int e = tid; e < q * q; e += NT) Rinv[e] = (e / q == e % q) ? 1.0 : 0.0;
     return;
   }
@@ -761,7 +768,12 @@ __global__ __launch_bounds__(JAC_NT) void jacobi_kernel(const double* __restrict
                                                         double* __restrict__ w,
                                                         double* __restrict__ rot, int* info,
                                                         double* gscratch, int use_lds,
-                                                        double tol) {
+                                                        double tol, const int* robust,
+                                                        double tol_else) {
+  if (robust && *robust == 0) {
+    if (tol_else < 0.0) return;
+    tol = tol_else;
+  }
   extern __shared__ double lds[];
   double* S = kLds ? lds : gscratch;
   __shared__ double cs_c[256], cs_s[256];
@@ -872,7 +884,8 @@ __device__ __forceinline__ void rep_wave_sync() {
 
 __global__ __launch_bounds__(64 * kRepWaves) void jacobi_vectors_kernel(
     const double* __restrict__ rot, const int* __restrict__ info, int q, double* __restrict__ w,
-    double* __restrict__ V, const double* __restrict__ wraw) {
+    double* __restrict__ V, const double* __restrict__ wraw, const int* robust) {
+  if (robust && *robust == 0) return;
   extern __shared__ double lds[];  // kRepWaves rows x n, then one rotation chunk
   __shared__ int perm[512];
   constexpr int NT = 64 * kRepWaves;
@@ -978,7 +991,12 @@ __device__ __forceinline__ int bj_global(int li, int I, int J) {
 __global__ __launch_bounds__(BJE_NT) void jacobi_blk_kernel(const double* __restrict__ Gin, int q,
                                                            double* __restrict__ w,
                                                            double* __restrict__ vrec, int* info,
-                                                           double tol) {
+                                                           double tol, const int* robust,
+                                                           double tol_else) {
+  if (robust && *robust == 0) {
+    if (tol_else < 0.0) return;
+    tol = tol_else;
+  }
   extern __shared__ double S[];  // 8 x 8 blocks of the upper triangle
   __shared__ double Vs[kBjMaxPairs][16 * BJ_LD];
   __shared__ double Ws[kBjMaxPairs][16 * BJ_LD];
@@ -1190,7 +1208,8 @@ __global__ __launch_bounds__(BJE_NT) void jacobi_blk_kernel(const double* __rest
 // sorted by descending eigenvalue (ties: lower index first).
 __global__ __launch_bounds__(BJ_NT) void jacobi_blk_vectors_kernel(
     const double* __restrict__ vrec, const int* __restrict__ info, int q, double* __restrict__ w,
-    double* __restrict__ V, const double* __restrict__ wraw) {
+    double* __restrict__ V, const double* __restrict__ wraw, const int* robust) {
+  if (robust && *robust == 0) return;
   __shared__ double Vt[16][kBjMaxQ + 1];
   __shared__ int perm[kBjMaxQ];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -1369,7 +1388,8 @@ void gaussian_sketch(double* out, int64_t n, int64_t q, uint64_t seed, uint64_t 
 }
 
 void chol_rinv(const double* G, double* Rinv, int q, double shift_rel, double rank_tol,
-               hipStream_t s, double* gscratch, int* dead_out, const int* run_if, bool tiles) {
+               hipStream_t s, double* gscratch, int* dead_out, const int* run_if, bool tiles,
+               double near_identity) {
   ACETN_REQUIRE(q >= 1 && q <= 512, "chol_rinv: q out of range");
   // q^3/3 (factor) + q^3/6 (inverse)
   hipEvent_t e0 = kernel_timing_begin(s);
@@ -1382,7 +1402,7 @@ void chol_rinv(const double* G, double* Rinv, int q, double shift_rel, double ra
   // every wave at each barrier
 #define ACETN_CT(NW, NS)                                                                        \
   hipLaunchKernelGGL((chol_rinv_tile_kernel<NW, NS>), dim3(1), dim3(64 * NW), 0, s, G, Rinv, q, \
-                     shift_rel, rank_tol, dead_out, run_if)
+                     shift_rel, rank_tol, dead_out, run_if, near_identity)
   if (tiles && q <= kCtMaxQ) {
     const int Q = (q + 15) / 16, slots = Q * (Q - 1) / 2;
     if (slots <= 2) ACETN_CT(2, 2);
@@ -1456,7 +1476,10 @@ size_t jacobi_rot_elems(int q) {
   return jacobi_record_elems(q) + (size_t)q + 8 + (size_t)n * (n + 1) / 2;
 }
 
-void jacobi_eigh(double* G, double* w, double* V, double* rot, int q, hipStream_t s, double tol) {
+void jacobi_eigh(double* G, double* w, double* V, double* rot, int q, hipStream_t s, double tol,
+                 const int* robust, double tol_else) {
+  // the replay runs whenever the solve does
+  const int* vrun = tol_else < 0.0 ? robust : nullptr;
   ACETN_REQUIRE(q >= 1 && q <= 510, "jacobi_eigh: q out of range");
   hipEvent_t e0 = kernel_timing_begin(s);
   struct End {
@@ -1479,10 +1502,11 @@ void jacobi_eigh(double* G, double* w, double* V, double* rot, int q, hipStream_
                                           (int)(sizeof(double) * kNmax * (kNmax + 1) / 2 * 64)));
       attr = true;
     }
-    hipLaunchKernelGGL(jacobi_blk_kernel, dim3(1), dim3(BJE_NT), lds, s, G, q, wraw, rot, info, tol);
+    hipLaunchKernelGGL(jacobi_blk_kernel, dim3(1), dim3(BJE_NT), lds, s, G, q, wraw, rot, info, tol,
+                       robust, tol_else);
     ACETN_HIP_CHECK(hipGetLastError());
     hipLaunchKernelGGL(jacobi_blk_vectors_kernel, dim3((8 * N + 15) / 16), dim3(BJ_NT), 0, s, rot,
-                       info, q, w, V, wraw);
+                       info, q, w, V, wraw, vrun);
     ACETN_HIP_CHECK(hipGetLastError());
     return;
   }
@@ -1492,18 +1516,18 @@ void jacobi_eigh(double* G, double* w, double* V, double* rot, int q, hipStream_
   const bool list = half * (half + 1) / 2 <= kJacList * JAC_NT;
   if (list && use_lds)
     hipLaunchKernelGGL((jacobi_kernel<true, true>), dim3(1), dim3(JAC_NT), pb, s, G, q, wraw, rot,
-                       info, gscr, use_lds, tol);
+                       info, gscr, use_lds, tol, robust, tol_else);
   else if (use_lds)
     hipLaunchKernelGGL((jacobi_kernel<false, true>), dim3(1), dim3(JAC_NT), pb, s, G, q, wraw, rot,
-                       info, gscr, use_lds, tol);
+                       info, gscr, use_lds, tol, robust, tol_else);
   else
     hipLaunchKernelGGL((jacobi_kernel<false, false>), dim3(1), dim3(JAC_NT), 0, s, G, q, wraw, rot,
-                       info, gscr, use_lds, tol);
+                       info, gscr, use_lds, tol, robust, tol_else);
   ACETN_HIP_CHECK(hipGetLastError());
   const int nblk = (q + kRepWaves - 1) / kRepWaves;
   const size_t lds = sizeof(double) * ((size_t)kRepWaves * n + (size_t)kRepPrefetch * 64 * kRepWaves);
   hipLaunchKernelGGL(jacobi_vectors_kernel, dim3(nblk), dim3(64 * kRepWaves), lds, s, rot, info, q,
-                     w, V, wraw);
+                     w, V, wraw, vrun);
   ACETN_HIP_CHECK(hipGetLastError());
 }
 

@@ -28,3 +28,46 @@ def test_orthonormalize_tile_edges(hip, q):
     for n in sorted({1, (q + 1) // 2, q}):
         P = Q[:, :n] - ref[:, :n] @ (ref[:, :n].T @ Q[:, :n])
         assert np.abs(P).max() <= 1e-12
+
+
+@pytest.mark.parametrize("case", ["separate", "pairs", "triples", "clusters", "equal", "graded",
+                                  "deficient"])
+@pytest.mark.parametrize("q", [1, 2, 9, 31, 32, 33, 65, 96, 130, 160, 193, 300])
+def test_gram_svd_spectra(hip, q, case):
+    """The Gram-matrix SVD behind the projectors at the edges of the
+    tridiagonal kernels' blocks, on spectra of every kind.  A Jacobi solve
+    takes each column through q - 1 rotations a sweep, each good to 3 eps, and
+    some twelve sweeps in its two passes: 36 eps q = 4e-15 q for the
+    orthonormality of the vectors, the same for the values in units of s_0
+    (sqrt(eps) where they vanish).  The projector onto each group of equal
+    values is compared where the values are resolved: eps s_0 / (s gap), with
+    gaps of 0.02 and more, times the q terms of its entries."""
+    i = np.arange(q)
+    s = np.exp(-7.0 * i / max(q, 2))
+    if case in ("pairs", "triples"):
+        n = 2 if case == "pairs" else 3
+        s = s[i // n * n]
+    elif case == "clusters":
+        s = s[i // 7 * 7] * (1.0 - 1e-9 * (i % 7))
+    elif case == "equal":
+        s = np.ones(q)
+    elif case == "graded":
+        s = np.exp(-23.0 * i / max(q, 2))
+    elif case == "deficient":
+        s = np.where(i < (q + 1) // 2, s, 0.0)
+    g = np.random.default_rng(100 * q + len(case))
+    U = np.linalg.qr(g.standard_normal((q, q)))[0]
+    V = np.linalg.qr(g.standard_normal((700, q)))[0]
+    w, UB = hip.gram_svd(torch.as_tensor(V @ (U * s).T, device="cuda"))
+    sv, UB = torch.sqrt(torch.clamp(w, min=0.0)).cpu().numpy(), UB.cpu().numpy()
+    tol = 4e-15 * q + 1e-15
+    assert np.abs(sv - s).max() <= (1.5e-8 * q if case == "deficient" else tol)
+    assert np.abs(UB.T @ UB - np.eye(q)).max() <= tol
+    new = np.concatenate([[True], s[1:] < s[:-1] * (1.0 - 1e-6)])
+    group = np.cumsum(new) - 1
+    for k in range(group[-1] + 1):
+        at = np.nonzero(group == k)[0]
+        if s[at[0]] < 1e-6:
+            continue
+        P, R = UB[:, at] @ UB[:, at].T, U[:, at] @ U[:, at].T
+        assert np.abs(P - R).max() <= 2.2e-16 * q / (0.02 * s[at[0]])
