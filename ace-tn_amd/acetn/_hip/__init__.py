@@ -409,6 +409,9 @@ PRECISIONS = {"fp64": 0, "mixed": 1}
 # OR-ed into a projector pair's precision code: the range finder refills
 # dropped columns at random (cheaper; identical unless the spectrum is graded)
 RF_FAST = 0x100
+# likewise: the range finder reports dropped columns (count -1) instead of
+# dealing with them, and the pair is begun again without this bit
+RF_TRUST = 0x200
 
 
 def precision_code(precision):
@@ -610,7 +613,7 @@ class ProjectorJob:
 
     def __init__(self, slot, sites, k, chi, oversampling, niter, cutoff, seed, stream_id,
                  precision="fp64", system="half-system", svd="rsvd", ws_key=None, graph=None,
-                 mark=False, rf_fast=False):
+                 mark=False, rf_fast=False, trust=False):
         """With ``graph`` = (stream_base, counts, index) the pair is enqueued in
         the capturable form (acetn_hip_projectors_begin_graph / _end_padded):
         the sketch stream is stream_id + stream_base[0] (an int64 device
@@ -622,7 +625,10 @@ class ProjectorJob:
         the eigensolver (acetn_hip_projectors_begin_mark).  ``rf_fast`` sets
         RF_FAST (for pairs whose previous spectrum was not graded); the
         ungraded test reads the spectrum: ``self.spec_host`` receives its q
-        computed values on the host by the time ``ready`` completes."""
+        computed values on the host by the time ``ready`` completes.
+        ``trust`` begins the pair without the launches that deal with dropped
+        columns (RF_TRUST); should there be any, ``finish`` begins it again
+        with them and waits, so the result is the same either way."""
         made = [make_site(*st) for st in sites]
         self.sv = [m[0] for m in made]
         self.keep = [m[1] for m in made]
@@ -660,27 +666,31 @@ class ProjectorJob:
         self.ws = slot_workspace(slot if ws_key is None else ("pair", ws_key), nb, self.dev)
         self.cd_host = torch.zeros(2, dtype=torch.int32, pin_memory=True)
         self.mark = None
+        self.begin_args = (niter, cutoff, seed, stream_id, nspec)
+        self._begin(RF_TRUST if trust else 0, mark)
+
+    def _begin(self, trust, mark=False):
+        niter, cutoff, seed, stream_id, nspec = self.begin_args
+        args = (self.arr, self.k, self.chi, self.p, niter, cutoff, seed, stream_id, self.system,
+                self.svd, self.prec | trust)
         with torch.cuda.stream(self.stream):
             # zero-filled on the pair's stream, ahead of the kernels that write it
             self.spec = torch.zeros(nspec, dtype=torch.float64, device=self.dev)
+            tail = (c_vp(self.cd_host.data_ptr()), ptr(self.spec), ptr(self.ws), self.ws.numel(),
+                    c_vp(self.stream.cuda_stream))
             if mark:
                 # the event object exists once recorded; the library records it
                 # again at the mark, and waits issued later refer to that record
                 self.mark = torch.cuda.Event()
                 self.mark.record(self.stream)
-                check(lib().acetn_hip_projectors_begin_mark(
-                    self.arr, k, chi, oversampling, niter, cutoff, seed, stream_id, self.system,
-                    self.svd, self.prec, c_vp(self.cd_host.data_ptr()), ptr(self.spec),
-                    ptr(self.ws), self.ws.numel(), c_vp(self.stream.cuda_stream),
-                    c_vp(self.mark.cuda_event)))
+                check(lib().acetn_hip_projectors_begin_mark(*args, *tail,
+                                                            c_vp(self.mark.cuda_event)))
             else:
-                check(lib().acetn_hip_projectors_begin(
-                    self.arr, k, chi, oversampling, niter, cutoff, seed, stream_id, self.system,
-                    self.svd, self.prec, c_vp(self.cd_host.data_ptr()), ptr(self.spec),
-                    ptr(self.ws), self.ws.numel(), c_vp(self.stream.cuda_stream)))
+                check(lib().acetn_hip_projectors_begin(*args, *tail))
             if self.svd == SVD_TYPES["rsvd"]:
-                q = chi + oversampling
-                self.spec_host = torch.empty(q, dtype=torch.float64, pin_memory=True)
+                q = self.chi + self.p
+                if self.spec_host is None:
+                    self.spec_host = torch.empty(q, dtype=torch.float64, pin_memory=True)
                 self.spec_host.copy_(self.spec[:q], non_blocking=True)
             # marks the truncation count's (and spectrum's) arrival in pinned
             # host memory
@@ -700,6 +710,10 @@ class ProjectorJob:
                     c_vp(self.stream.cuda_stream)))
             return P1, P2
         n = int(self.cd_host[0])
+        if n < 0:
+            self._begin(0)
+            self.ready.synchronize()
+            n = int(self.cd_host[0])
         with torch.cuda.stream(self.stream):
             P1 = torch.empty(self.rows, n, dtype=torch.float64, device=self.dev)
             P2 = torch.empty(self.rows, n, dtype=torch.float64, device=self.dev)

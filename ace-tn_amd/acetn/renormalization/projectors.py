@@ -9,6 +9,10 @@ from .. import _hip
 
 # s_{q-1} / s_0 at or above which a pair's spectrum counts as not graded
 UNGRADED = 1e-3
+# and from which the range finder is trusted not to drop a column: its Gram
+# matrices see the square of the ratio, the shift of their first pass (1e-9)
+# lifts it, and the rank guard (1e-14) then lies at 2e-6
+TRUSTED = 1e-5
 
 
 class SketchCounter:
@@ -43,6 +47,8 @@ class ProjectorCalculator:
         # pair (sites, k, system) -> its last spectrum was not graded, so the
         # next computation may take the range finder's fast path (RF_FAST)
         self.ungraded = {}
+        # the same pair -> s_{q-1} / s_0 of its last spectrum
+        self.span = {}
         self.set_calculate()
 
     def set_calculate(self):
@@ -112,7 +118,9 @@ class ProjectorCalculator:
                                     precision=self.precision, system=system,
                                     svd=self.svd_type, ws_key=ws_key, graph=graph,
                                     mark=mark,
-                                    rf_fast=graph is None and self.ungraded.get(key, False))
+                                    rf_fast=graph is None and self.ungraded.get(key, False),
+                                    trust=graph is None and
+                                    self.span.get(key, 1.0) >= TRUSTED)
             job.key = key
             started.append(job)
         return started
@@ -133,12 +141,13 @@ class ProjectorCalculator:
         D = ipeps.dims['bond']
 
         def finish(job):
+            P1, P2 = job.finish()
             if job.spec_host is not None:
                 # the range finder's CholeskyQR keeps every column when the
                 # q values span less than 1e-3 (margin 100 on its rank guard)
-                s = job.spec_host
-                self.ungraded[job.key] = bool(s[0] > 0 and s[-1] >= UNGRADED * s[0])
-            P1, P2 = job.finish()
+                s0, s1 = float(job.spec_host[0]), float(job.spec_host[-1])
+                self.span[job.key] = s1 / s0 if s0 > 0 else 0.0
+                self.ungraded[job.key] = bool(s0 > 0 and s1 >= UNGRADED * s0)
             # the kept count: a device scalar for a captured pair (written on
             # every replay)
             cd = P1.shape[1] if job.graph is None else job.graph[1][job.graph[2]]

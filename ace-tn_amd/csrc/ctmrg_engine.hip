@@ -108,7 +108,8 @@ void quarter_tensor(Ctx& c, const acetn_site* s, int k, double* Q, bool f32 = fa
 // Householder QR, and unlike refilling every dropped column at random, this
 // keeps the directions the rounding-level content of those columns holds,
 // which after a power iteration are the next singular directions.  All of it
-// is skipped on the device when no column was dropped.
+// is skipped on the device when no column was dropped; when the caller is
+// prepared to start over (trust) none of it is launched and the drop reported.
 // ---------------------------------------------------------------------------
 // Returns the buffer that holds the basis: Y, or, for a basis that only steers
 // the power iteration in mixed precision (steer), the output of the single
@@ -118,7 +119,8 @@ constexpr int kRecoverLevels = 3;
 
 // Sketch width from which the projector SVD is preconditioned through the
 // tridiagonal form: its twenty launches cost a small matrix more than the two
-// Jacobi solves take (0.15 ms at q = 22).
+// Jacobi solves take (one iteration at D=2, chi=20, q = 22: 8.3 ms with the
+// line at 17, 6.6 ms with it here; full-system D=3, chi=35: 22.2 and 20.5 ms).
 constexpr int kTridiagMinQ = 48;
 
 const double* orthonormalize(Ctx& c, double* Y, int64_t m, int64_t q, bool steer = false) {
@@ -153,6 +155,10 @@ const double* orthonormalize(Ctx& c, double* Y, int64_t m, int64_t q, bool steer
   if (single) return Yt;
   // pass 1: plain with rank guard (Yt -> Y); dropped columns come out zero
   pass(Yt, Y, 0.0, 1e-14, dead, nullptr, false);
+  if (c.trust) {
+    if (c.launch) c.drops.add(any);
+    return Y;
+  }
   if (!c.recover) {
     // ACETN_HIP_RF_FAST: dropped columns refilled at random, then the two
     // plain passes (all skipped on the device when none was dropped)
@@ -494,7 +500,7 @@ void half_projectors(Ctx& c, const acetn_site* s1, const acetn_site* s4, int k, 
     c.launch = true;
     cD = out.cD_in;
   } else {
-    count_kept(w, (int)q, (int)chi, cutoff, s, cD_dev, c.st);
+    count_kept(w, (int)q, (int)chi, cutoff, s, cD_dev, c.st, c.drops);
     if (out.spectrum) ACETN_HIP_CHECK(hipMemcpyAsync(out.spectrum, s, sizeof(double) * q, hipMemcpyDeviceToDevice, c.st));
     if (phase == 1) {
       if (out.pinned_cD)
@@ -675,7 +681,7 @@ void general_projectors(Ctx& c, const acetn_site* const* st, int k, int system, 
     c.launch = true;
     cD = out.cD_in;
   } else {
-    count_kept(w, qi, (int)chi, cutoff, sv, cD_dev, c.st);
+    count_kept(w, qi, (int)chi, cutoff, sv, cD_dev, c.st, c.drops);
     if (out.spectrum) ACETN_HIP_CHECK(hipMemcpyAsync(out.spectrum, sv, sizeof(double) * q, hipMemcpyDeviceToDevice, c.st));
     if (phase == 1) {
       if (out.pinned_cD)
@@ -1319,6 +1325,8 @@ int acetn_hip_projectors_begin_graph(const acetn_site* const sites[4], int k, in
     check_precision(precision);
     ACETN_REQUIRE(dev_stream_base && dev_cD_new, "projectors_begin_graph: null device pointer");
     ACETN_REQUIRE(niter >= 0 && niter <= 16, "projectors: niter out of range");
+    ACETN_REQUIRE((precision & ACETN_HIP_RF_TRUST) == 0,
+                  "projectors_begin_graph: nothing reads the count, so RF_TRUST cannot be served");
     HalfOut o{nullptr, nullptr, nullptr, nullptr, 0, spectrum};
     o.stream_base = dev_stream_base;
     o.dev_cD = dev_cD_new;

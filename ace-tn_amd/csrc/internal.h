@@ -299,9 +299,21 @@ size_t jacobi_svd_scratch_elems(int rows, int cols);
 // With ``kept`` (a device count), the columns z >= kept[0] are written as zero.
 void scale_columns(const double* Ub, int q, const double* s, int cD, int mode, double* X,
                    hipStream_t st, const int* kept = nullptr);
-// cD_new = min(chi, #{s/s0 > cutoff}) with s = sqrt(max(w, 0)).
+// Device flags of the orthonormalisations of one range finder (2 niter + 1 at
+// most): nonzero where columns were dropped.
+constexpr int kMaxDropFlags = 40;
+struct DropFlags {
+  int n = 0;
+  const int* p[kMaxDropFlags];
+  void add(const int* f) {
+    ACETN_REQUIRE(n < kMaxDropFlags, "range finder: too many orthonormalisations");
+    p[n++] = f;
+  }
+};
+// cD_new = min(chi, #{s/s0 > cutoff}) with s = sqrt(max(w, 0)), or -1 when one
+// of the flags is set.
 void count_kept(const double* w, int q, int chi, double cutoff, double* s_out, int* cD_out,
-                hipStream_t st);
+                hipStream_t st, const DropFlags& drops = DropFlags());
 // Sign gauge of the projector pair (shared with the oracle).
 void fix_projector_gauge(double* P1, double* P2, int64_t rows1, int64_t rows2, int cD,
                          hipStream_t st);

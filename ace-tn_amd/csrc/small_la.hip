@@ -1275,7 +1275,7 @@ __global__ __launch_bounds__(BJ_NT) void jacobi_blk_vectors_kernel(
 
 // --------------------------------------------------------------------------
 __global__ void count_kept_kernel(const double* __restrict__ w, int q, int chi, double cutoff,
-                                  double* __restrict__ s_out, int* cD_out) {
+                                  double* __restrict__ s_out, int* cD_out, DropFlags drops) {
   __shared__ int cnt;
   if (threadIdx.x == 0) cnt = 0;
   __syncthreads();
@@ -1285,8 +1285,8 @@ __global__ void count_kept_kernel(const double* __restrict__ w, int q, int chi, 
     s_out[i] = si;
     if (s0 > 0.0 && si / s0 > cutoff) atomicAdd(&cnt, 1);
   }
-  __syncthreads();
-  if (threadIdx.x == 0) cD_out[0] = min(chi, cnt);
+  const int dropped = __syncthreads_or((int)threadIdx.x < drops.n && *drops.p[threadIdx.x] != 0);
+  if (threadIdx.x == 0) cD_out[0] = dropped ? -1 : min(chi, cnt);
 }
 
 __global__ void scale_columns_kernel(const double* __restrict__ Ub, int q,
@@ -1541,8 +1541,9 @@ void scale_columns(const double* Ub, int q, const double* s, int cD, int mode, d
 }
 
 void count_kept(const double* w, int q, int chi, double cutoff, double* s_out, int* cD_out,
-                hipStream_t st) {
-  hipLaunchKernelGGL(count_kept_kernel, dim3(1), dim3(256), 0, st, w, q, chi, cutoff, s_out, cD_out);
+                hipStream_t st, const DropFlags& drops) {
+  hipLaunchKernelGGL(count_kept_kernel, dim3(1), dim3(256), 0, st, w, q, chi, cutoff, s_out, cD_out,
+                     drops);
   ACETN_HIP_CHECK(hipGetLastError());
 }
 

@@ -67,6 +67,15 @@ enum { ACETN_HIP_FP64 = 0, ACETN_HIP_MIXED = 1 };
  * columns lose the small singular directions, so the default recovers them. */
 enum { ACETN_HIP_RF_FAST = 0x100 };
 
+/* Bit OR-ed into the ``precision`` of acetn_hip_projectors_begin[_mark] and
+ * the matching _end: the range finder does nothing about dropped columns but
+ * report them.  The truncation count then comes back as -1 (and nothing else
+ * of the pair is to be used): call begin again without the bit.  With any
+ * other count the result is bit for bit that of the call without it; the
+ * launches that only a dropped column would make use of (100 of 160 per pair)
+ * are saved. */
+enum { ACETN_HIP_RF_TRUST = 0x200 };
+
 /* Message of the last failed call on this thread ("" if none). */
 const char* acetn_hip_last_error(void);
 

@@ -71,3 +71,31 @@ def test_gram_svd_spectra(hip, q, case):
             continue
         P, R = UB[:, at] @ UB[:, at].T, U[:, at] @ U[:, at].T
         assert np.abs(P - R).max() <= 2.2e-16 * q / (0.02 * s[at[0]])
+
+
+@pytest.mark.parametrize("start", ["product", "random"])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_trusted_range_finder_starts_over(hip, start, precision):
+    """A pair begun without the launches that deal with dropped columns ends
+    with the bits of one begun with them: on a graded spectrum (columns are
+    dropped: the count comes back -1 and the pair starts over) and on one that
+    drops none (a count at once)."""
+    from oracle import ctmrg as oc
+    from test_hip_ctmrg import product_start, to_dev_site
+    D, chi = (4, 16) if start == "product" else (3, 9)
+    st = product_start(D, 5) if start == "product" else \
+        oc.make_state(oc.random_site_tensors(2, 2, D, 2, seed=41))
+    dsites = [to_dev_site(st[s]) for s in oc.plaquette(2, 2, 0, 1, 0)]
+    out, counts = [], []
+    for trust in (False, True):
+        job = hip.ProjectorJob(0, dsites, 0, chi, 2, 2, 1e-12, 21, 3, precision=precision,
+                               trust=trust)
+        job.ready.synchronize()
+        counts.append(int(job.cd_host[0]))
+        P1, P2 = job.finish()
+        torch.cuda.synchronize()
+        out.append((P1.cpu(), P2.cpu(), job.spec.cpu(), job.spec_host.clone()))
+    assert counts[0] > 0
+    assert counts[1] == (-1 if start == "product" else counts[0])
+    for a, b in zip(*out):
+        assert torch.equal(a, b)
