@@ -79,7 +79,9 @@ struct SplitScope {
   ~SplitScope() { c.split = saved; }
 };
 
-inline void gemm(Ctx& c, const GemmDesc& g, const double* A, const double* B, double* C) {
+inline void gemm(Ctx& c, const GemmDesc& gd, const double* A, const double* B, double* C) {
+  GemmDesc g = gd;
+  g.pipe = !c.mixed;
   if (!c.run) {
     c.gwork_need = std::max({c.gwork_need, gemm_f64_work_elems(g, 1), gemm_split_work_elems(g, 1)});
     return;

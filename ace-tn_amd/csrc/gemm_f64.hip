@@ -97,6 +97,7 @@ void kernel_timing_end(hipEvent_t e0, hipStream_t s, int cls, double flops, doub
 
 namespace {
 constexpr int BK = 16, NT = 256;
+constexpr double kPipeMinMacs = 5e7;
 
 __device__ __forceinline__ bool contiguous(const IdxMap& m) { return m.s0 == 1; }
 
@@ -304,6 +305,254 @@ __global__ void splitk_reduce_kernel(GemmDesc g, GemmBatch bt, int ksplit,
   }
 }
 
+// --------------------------------------------------------------------------
+// Large products with plainly strided operands: A contiguous along k or along
+// m (AM), B along n, all rows even and 16-byte aligned.  One workgroup of four
+// waves makes a 64 x 16 WN tile, 16 rows a wave, in k-tiles of 16; two
+// workgroups share a CU, so that one's barriers and stores fall into the
+// other's products (one workgroup of eight waves, in step at every barrier,
+// took 11 % longer; LDS and memory instructions dealt out between the matrix
+// instructions 10 % longer still).
+//
+// At these shapes the matrix cores are the bound (64 clocks a 16x16x4 product,
+// 128 flop a clock and CU), so everything else has to stay out of their way:
+//   * 16-byte loads, three k-tiles ahead in two sets of registers;
+//   * the operands of each product are read from LDS while the one before runs;
+//   * the k index is dealt so that a lane needs neighbouring k's in two
+//     successive products: 16-byte LDS reads of a k-contiguous A, whose 16-byte
+//     pieces are xor-ed over the banks, and rows of A (AM) and B padded so that
+//     two of the four k groups of a read cover the 64 banks;
+//   * the width in steps of 16 columns: 146 columns pay for 160, 66 for 80;
+//   * the number of k parts from the rounds of workgroups that result
+//     (pipe_ksplit), instead of a part count that leaves a last round nearly
+//     empty.
+// Measured with the reduction of the parts, back to back, against the 64- and
+// 128-row tiles of gemm_f64_kernel: 5184 x 146 x 5184 (the range finder at
+// D=6, chi=144) 205 us against 295 (its matrix-core floor is 110 us at 72
+// TFLOP/s: power holds the clock near 2.2 GHz, and the operands' way in costs
+// the rest), 2500 x 102 x 2500 47 against 74, 2592 x 74 x 2592 37 against 41,
+// 1024 x 66 x 1024 17 against 20.
+// --------------------------------------------------------------------------
+constexpr int PP_NW = 4, PP_NT = 64 * PP_NW, PP_BM = 16 * PP_NW, PP_BK = 16, PP_MAXWN = 10;
+typedef double pd2 __attribute__((ext_vector_type(2)));
+
+template <int WN, bool AM>
+__global__ __launch_bounds__(PP_NT, 2) void gemm_f64_pipe_kernel(GemmDesc g, const double* __restrict__ A,
+                                                                 const double* __restrict__ B,
+                                                                 double* __restrict__ C, int ksplit,
+                                                                 double* __restrict__ work) {
+  constexpr int BN = 16 * WN, LDB = BN + 8;
+  constexpr int LDA = PP_BM + 8;                        // AM: row of k
+  constexpr int SA = AM ? PP_BK * LDA : PP_BM * PP_BK;  // doubles per buffer
+  constexpr int SB = PP_BK * LDB;
+  constexpr int NB = (8 * PP_BK * WN + PP_NT - 1) / PP_NT;  // 16-byte pieces of B per thread
+  __shared__ __align__(16) double sA[2][SA];
+  __shared__ __align__(16) double sB[2][SB];
+  if (g.run_if && *g.run_if == 0) return;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int m16 = lane & 15, kq = lane >> 4;
+  const int m0 = blockIdx.y * PP_BM, n0 = blockIdx.x * BN, kpart = blockIdx.z;
+  const int64_t lda = AM ? g.ak.s0 : g.am.s0, ldb = g.bk.s0;
+  const int ktiles = (g.K + PP_BK - 1) / PP_BK;
+  const int per = (ktiles + ksplit - 1) / ksplit;
+  const int kbeg = kpart * per * PP_BK;
+  const int kend = min(g.K, kbeg + per * PP_BK);
+  const int nst = kend > kbeg ? (kend - kbeg + PP_BK - 1) / PP_BK : 0;
+
+  // this thread's pieces: (row, piece) of A and (k, piece) of B; rows and
+  // columns past the edge are clamped (their results are never stored)
+  int ax[2], ay[2], bx[NB], by[NB];
+  const double* ap[2];
+  const double* bp[NB];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int x = tid + PP_NT * i;
+    ax[i] = AM ? x / (PP_BM / 2) : x >> 3;  // k, or m
+    ay[i] = AM ? x % (PP_BM / 2) : x & 7;   // piece of m, or of k
+    ap[i] = AM ? A + (int64_t)min(m0 + 2 * ay[i], (g.M - 1) & ~1)
+               : A + (int64_t)min(m0 + ax[i], g.M - 1) * lda;
+  }
+#pragma unroll
+  for (int i = 0; i < NB; ++i) {
+    const int x = min(tid + PP_NT * i, 8 * PP_BK * WN - 1);
+    bx[i] = x / (8 * WN);
+    by[i] = x % (8 * WN);
+    bp[i] = B + min(n0 + 2 * by[i], (g.N - 1) & ~1);
+  }
+  struct Regs {
+    pd2 a[2], b[NB];
+  };
+  // piece i of k-tile st: the two of A, then those of B
+  constexpr int NP = 2 + NB;
+  auto load = [&](int st, Regs& r, int i) {
+    const int k0 = kbeg + st * PP_BK;
+    if (i >= 2) {
+      r.b[i - 2] = *reinterpret_cast<const pd2*>(
+          bp[i - 2] + (int64_t)min(k0 + bx[i - 2], kend - 1) * ldb);
+    } else if (AM) {
+      const int k = k0 + ax[i];
+      r.a[i] = *reinterpret_cast<const pd2*>(ap[i] + (int64_t)min(k, kend - 1) * lda);
+    } else {
+      r.a[i] = *reinterpret_cast<const pd2*>(ap[i] + min(k0 + 2 * ay[i], (kend - 1) & ~1));
+    }
+  };
+  auto store = [&](int st, const Regs& r, int i) {
+    if (i >= 2) {
+      *reinterpret_cast<pd2*>(&sB[st & 1][bx[i - 2] * LDB + 2 * by[i - 2]]) = r.b[i - 2];
+      return;
+    }
+    const int k = kbeg + st * PP_BK + (AM ? ax[i] : 2 * ay[i]);
+    const int at = AM ? ax[i] * LDA + 2 * ay[i] : ax[i] * PP_BK + 2 * (ay[i] ^ (ax[i] & 7));
+    pd2 v = r.a[i];
+    // past the last k (B's rows are repeated there)
+    if (k >= kend) v.x = 0.0;
+    if (AM ? k >= kend : k + 1 >= kend) v.y = 0.0;
+    *reinterpret_cast<pd2*>(&sA[st & 1][at]) = v;
+  };
+  d4 acc[WN];
+#pragma unroll
+  for (int j = 0; j < WN; ++j) acc[j] = d4{0.0, 0.0, 0.0, 0.0};
+  // operands of the four products of a k-tile, two sets of registers in turn:
+  // product x = 2 t + h takes k = 8 t + 2 kq + h
+  pd2 a[2];
+  double b[2][WN];
+  const int row = 16 * wave + m16;
+  auto fetch_a = [&](int buf, int x) {
+    const int k = 8 * (x >> 1) + 2 * kq + (x & 1);
+    if (AM) {
+      if (x & 1) a[x >> 1].y = sA[buf][k * LDA + row];
+      else a[x >> 1].x = sA[buf][k * LDA + row];
+    } else if ((x & 1) == 0) {
+      a[x >> 1] = *reinterpret_cast<const pd2*>(
+          &sA[buf][row * PP_BK + 2 * ((2 * x + kq) ^ (row & 7))]);
+    }
+  };
+  auto fetch_b = [&](int buf, int x, int j) {
+    b[x & 1][j] = sB[buf][(8 * (x >> 1) + 2 * kq + (x & 1)) * LDB + 16 * j + m16];
+  };
+  Regs r0, r1;
+  if (nst > 0) {
+#pragma unroll
+    for (int i = 0; i < NP; ++i) load(0, r0, i);
+    if (nst > 1) {
+#pragma unroll
+      for (int i = 0; i < NP; ++i) load(1, r1, i);
+    }
+#pragma unroll
+    for (int i = 0; i < NP; ++i) store(0, r0, i);
+    if (nst > 2) {
+#pragma unroll
+      for (int i = 0; i < NP; ++i) load(2, r0, i);
+    }
+    __syncthreads();
+    fetch_a(0, 0);
+#pragma unroll
+    for (int j = 0; j < WN; ++j) fetch_b(0, 0, j);
+  }
+  // k-tile st: its buffer is complete, its first operands are in registers,
+  // k-tile st + 1 is in ``next`` and st + 2 on its way.  Each product's operands
+  // are read while the one before runs; the barrier stands ahead of the last
+  // product, which hides the waves' skew and the first reads of the next buffer.
+  auto tile = [&](int st, Regs& next) {
+    const int buf = st & 1;
+    if (st + 1 < nst) {
+#pragma unroll
+      for (int i = 0; i < NP; ++i) store(st + 1, next, i);
+    }
+    if (st + 3 < nst) {
+#pragma unroll
+      for (int i = 0; i < NP; ++i) load(st + 3, next, i);
+    }
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+      if (x == 3) __syncthreads();
+      if (x < 3 || st + 1 < nst) {
+        const int to = x < 3 ? buf : buf ^ 1;
+        fetch_a(to, (x + 1) & 3);
+#pragma unroll
+        for (int j = 0; j < WN; ++j) fetch_b(to, (x + 1) & 3, j);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      const double v = x & 1 ? a[x >> 1].y : a[x >> 1].x;
+#pragma unroll
+      for (int j = 0; j < WN; ++j)
+        acc[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(v, b[x & 1][j], acc[j], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  for (int st = 0; st < nst; st += 2) {
+    tile(st, r1);
+    if (st + 1 < nst) tile(st + 1, r0);
+  }
+#pragma unroll
+  for (int j = 0; j < WN; ++j)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int m = m0 + 16 * wave + kq + 4 * r, n = n0 + 16 * j + m16;
+      if (m >= g.M || n >= g.N) continue;
+      const double v = acc[j][r];
+      if (ksplit == 1) {
+        const int64_t off = imap(g.cm, m) + imap(g.cn, n);
+        C[off] = (g.beta != 0.0) ? g.alpha * v + g.beta * C[off] : g.alpha * v;
+      } else {
+        work[((int64_t)kpart * g.M + m) * g.N + n] = v;
+      }
+    }
+}
+
+bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
+
+// Shapes the pipelined kernel takes over: plainly strided as above (rows of even
+// length: no 16-byte piece reaches past one), and large enough that 64-row tiles and a few k parts fill the chip: below 5e7 products
+// (324 x 38 x 324 has 4e6) a call is launches and latency either way.
+bool pipe_shape(const GemmDesc& g, int count) {
+  if (!g.pipe || count != 1) return false;
+  if (g.am.n0 > 0 || g.ak.n0 > 0 || g.bk.n0 > 0 || g.bn.n0 > 0) return false;
+  const bool am = g.am.s0 == 1 && g.ak.s0 != 1;
+  if (!am && g.ak.s0 != 1) return false;
+  const int64_t lda = am ? g.ak.s0 : g.am.s0, alen = am ? g.M : g.K;
+  if (g.bn.s0 != 1 || ((lda | alen | g.bk.s0 | g.N) & 1)) return false;
+  return g.M >= 96 && g.N >= 17 && g.K >= 32 &&
+         (double)g.M * g.N * g.K >= kPipeMinMacs;
+}
+int pipe_wn(const GemmDesc& g) {
+  const int nt = (g.N + 16 * PP_MAXWN - 1) / (16 * PP_MAXWN);
+  return ((g.N + nt - 1) / nt + 15) / 16;
+}
+// k parts: the fewest estimated microseconds of rounds of workgroups (two a CU,
+// 512 WN clocks a k-tile for the pair) and of the partial sums' way through
+// memory (about 4 TB/s, written and read).
+int pipe_ksplit(const GemmDesc& g) {
+  const int wn = pipe_wn(g), kt = (g.K + PP_BK - 1) / PP_BK;
+  const int64_t tiles = (int64_t)((g.M + PP_BM - 1) / PP_BM) * ((g.N + 16 * wn - 1) / (16 * wn));
+  const double stage = 512.0 * wn / 2400.0, fixed = 5.0;
+  int best = 1;
+  double t_best = 0.0;
+  for (int ks = 1; ks <= 64 && (ks == 1 || kt / ks >= 6); ++ks) {
+    const int per = (kt + ks - 1) / ks;
+    if (ks > 1 && (ks - 1) * per >= kt) continue;  // an empty part
+    const double rounds = (double)((tiles * ks + 2048 / PP_NW - 1) / (2048 / PP_NW));
+    double t = rounds * (per * stage + fixed);
+    if (ks > 1) t += 4.0 + 2.0 * ks * g.M * (double)g.N * 8.0 / 4e6;
+    if (ks == 1 || t < t_best) {
+      best = ks;
+      t_best = t;
+    }
+  }
+  return best;
+}
+
+template <int WN>
+void launch_pipe(const GemmDesc& g, const double* A, const double* B, double* C, int ks,
+                 double* work, hipStream_t s) {
+  const dim3 grid((g.N + 16 * WN - 1) / (16 * WN), (g.M + PP_BM - 1) / PP_BM, ks);
+  ACETN_REQUIRE(grid.y <= 65535 && grid.z <= 65535, "gemm_f64: grid too large");
+  if (g.am.s0 == 1 && g.ak.s0 != 1)
+    hipLaunchKernelGGL((gemm_f64_pipe_kernel<WN, true>), grid, dim3(PP_NT), 0, s, g, A, B, C, ks, work);
+  else
+    hipLaunchKernelGGL((gemm_f64_pipe_kernel<WN, false>), grid, dim3(PP_NT), 0, s, g, A, B, C, ks, work);
+}
+
 // Small-output, long-K products (M, N <= 8, e.g. the d^2 x d^2 reduced
 // density matrix summed over the whole environment): a 16 x 16 matrix-core
 // tile would be almost all padding, so each lane walks its own k indices and
@@ -447,7 +696,8 @@ void launch_gemm_wide(const GemmDesc& g, const GemmBatch& b, int ks, double* wor
 
 size_t gemm_f64_work_elems(const GemmDesc& g, int count) {
   if (dot_small_fits(g)) return (size_t)dot_small_wgs(g) * count * kDotMax * kDotMax;
-  const int ks = choose_ksplit(g, count);
+  int ks = choose_ksplit(g, count);
+  if (pipe_shape(g, count)) ks = std::max(ks, pipe_ksplit(g));
   return ks > 1 ? (size_t)ks * count * g.M * g.N : 0;
 }
 
@@ -498,6 +748,34 @@ void gemm_f64(const GemmDesc& g, const GemmBatch& b, double* work, size_t work_e
     }
   };
   const TuneKey key{0, g.M, g.N, g.K, (lin ? 1 : 0) | (b.count << 1)};
+  TuneChoice listed;
+  const bool in_table = autotune_lookup(key, &listed) && fits(listed.ks) && (listed.var == 0 || lin);
+  if (!in_table && pipe_shape(g, b.count) && aligned16(b.A[0]) && aligned16(b.B[0])) {
+    const int ks = pipe_ksplit(g);
+    if (ks == 1 || (work != nullptr && work_elems >= (size_t)ks * g.M * g.N)) {
+      hipEvent_t e0 = kernel_timing_begin(s);
+      switch (pipe_wn(g)) {
+        case 2: launch_pipe<2>(g, b.A[0], b.B[0], b.C[0], ks, work, s); break;
+        case 3: launch_pipe<3>(g, b.A[0], b.B[0], b.C[0], ks, work, s); break;
+        case 4: launch_pipe<4>(g, b.A[0], b.B[0], b.C[0], ks, work, s); break;
+        case 5: launch_pipe<5>(g, b.A[0], b.B[0], b.C[0], ks, work, s); break;
+        case 6: launch_pipe<6>(g, b.A[0], b.B[0], b.C[0], ks, work, s); break;
+        case 7: launch_pipe<7>(g, b.A[0], b.B[0], b.C[0], ks, work, s); break;
+        case 8: launch_pipe<8>(g, b.A[0], b.B[0], b.C[0], ks, work, s); break;
+        case 9: launch_pipe<9>(g, b.A[0], b.B[0], b.C[0], ks, work, s); break;
+        default: launch_pipe<10>(g, b.A[0], b.B[0], b.C[0], ks, work, s); break;
+      }
+      ACETN_HIP_CHECK(hipGetLastError());
+      kernel_timing_end(e0, s, kKGemmF64, 2.0 * g.M * g.N * (double)g.K,
+                        8.0 * ((double)g.M * g.K + (double)g.K * g.N + (double)g.M * g.N));
+      if (ks > 1) {
+        const int blocks = (int)std::min<int64_t>(((int64_t)g.M * g.N + 255) / 256, 2048);
+        hipLaunchKernelGGL(splitk_reduce_kernel, dim3(blocks, 1), dim3(256), 0, s, g, b, ks, work);
+        ACETN_HIP_CHECK(hipGetLastError());
+      }
+      return;
+    }
+  }
   if (autotune_should_tune(key, g, s)) {
     std::vector<TuneChoice> cands;
     const Tile tiles[8] = {{1, 5},    {2, 5},    {2, 2},    {4, 4},
@@ -524,8 +802,7 @@ void gemm_f64(const GemmDesc& g, const GemmBatch& b, double* work, size_t work_e
   if (!fits(ks)) ks = 1;
   const Tile t = choose_tile(g);
   TuneChoice ch{t.wm, t.wn, ks};
-  TuneChoice tuned;
-  if (autotune_lookup(key, &tuned) && fits(tuned.ks) && (tuned.var == 0 || lin)) ch = tuned;
+  if (in_table) ch = listed;
   launch_choice(ch);
 }
 

@@ -99,3 +99,21 @@ def test_trusted_range_finder_starts_over(hip, start, precision):
     assert counts[1] == (-1 if start == "product" else counts[0])
     for a, b in zip(*out):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("ta", [False, True])
+@pytest.mark.parametrize("N", [17, 18, 33, 50, 66, 82, 98, 114, 130, 146, 160, 162, 258, 322])
+def test_large_gemm_tile_edges(hip, N, ta):
+    """The pipelined FP64 product at every tile width, with remainders of rows,
+    columns and k (odd sizes among them) and one or several k parts, against
+    numpy: K terms of unit variance, 2 eps K at most in units of their
+    norms."""
+    g = np.random.default_rng(N)
+    for M, K in ((96, 32768 + 2 * N), (1030, 3000), (1031, 3001), (4098, 1234), (9000, 402)):
+        A = g.standard_normal((K, M) if ta else (M, K))
+        B = g.standard_normal((K, N))
+        C = hip.gemm(torch.as_tensor(A, device="cuda"), torch.as_tensor(B, device="cuda"),
+                     ta=ta).cpu().numpy()
+        exact = (A.T if ta else A) @ B
+        scale = np.linalg.norm(A, axis=0 if ta else 1)[:, None] * np.linalg.norm(B, axis=0)
+        assert np.all(np.abs(C - exact) <= 4.4e-16 * K * scale), (M, N, K)
