@@ -41,6 +41,30 @@ QuarterDims quarter_dims(const acetn_site* s, int k) {
   return q;
 }
 
+// E (n0 x n1 x in) -> its first two axes exchanged: an edge tensor as the operand
+// of a product over its first index (or as rows of its second) with one plain
+// stride, which the pipelined FP64 kernel needs.  The copy (6 MB and 5 us at D=6,
+// chi=144) is repaid many times over: the enlarged corner's last product takes
+// 225 us against 420 with the permutation folded into the operand loads.
+const double* swap_edge(Ctx& c, const double* E, int64_t n0, int64_t n1, int64_t in) {
+  double* T = c.take((size_t)n0 * n1 * in);
+  if (c.launch) permute3(E, T, n1, n0, in, in, n1 * in, 1, c.st);
+  return T;
+}
+
+// out[(m),(e,x)] = sum_a T[a][m] E[e][a][x] (T: na x M, E: ne x na x in)
+void corner_edge(Ctx& c, const double* T, int64_t M, const double* E, int64_t ne, int64_t na,
+                 int64_t in, double* out) {
+  GemmDesc g = gdesc((int)M, (int)(ne * in), (int)na, plain(1), plain(M), plain(in),
+                     grouped((int)in, 1, na * in), plain(ne * in), plain(1));
+  if (!c.mixed && gemm_f64_large(g.M, g.N, g.K)) {
+    E = swap_edge(c, E, ne, na, in);
+    g.bk = plain(ne * in);
+    g.bn = plain(1);
+  }
+  gemm(c, g, T, E, out);
+}
+
 // f32 (mixed precision only): T2 and Q are held in FP32, Q as a float array
 // of the same element count (the caller's split of Q into bf16 planes reads
 // FP32 either way)
@@ -56,19 +80,15 @@ void quarter_tensor(Ctx& c, const acetn_site* s, int k, double* Q, bool f32 = fa
   mm(c, (int)qd.ca, (int)(qd.cc * D2), (int)qd.cb, false, s->C[kk], qd.cb, false, s->E[kk],
      qd.cc * D2, T1, qd.cc * D2);
   // T2[(c,u,U),(e,l,L)] = sum_a T1[a,(c,u,U)] E[k+3][e,a,(l,L)]
-  GemmDesc g{};
-  g.M = (int)qd.N1; g.N = (int)qd.N2; g.K = (int)qd.ca;
-  g.am = plain(1); g.ak = plain(qd.N1);
-  g.bk = plain(D2); g.bn = grouped((int)D2, 1, qd.ca * D2);
-  g.cm = plain(qd.N2); g.cn = plain(1);
-  g.alpha = 1.0; g.beta = 0.0;
   if (f32 && c.launch) {
+    GemmDesc g = gdesc((int)qd.N1, (int)qd.N2, (int)qd.ca, plain(1), plain(qd.N1), plain(D2),
+                       grouped((int)D2, 1, qd.ca * D2), plain(qd.N2), plain(1));
     GemmBatch b{};
     b.count = 1;
     b.A[0] = T1; b.B[0] = s->E[(3 + kk) & 3]; b.C[0] = T2;
     gemm_split(g, b, c.split, DType::F64, DType::F64, DType::F32, c.gwork, c.gwork_elems, c.st);
   } else {
-    gemm(c, g, T1, s->E[(3 + kk) & 3], T2);
+    corner_edge(c, T1, qd.N1, s->E[(3 + kk) & 3], qd.ce, qd.ca, D2, T2);
   }
   if (!c.launch) return;
   int64_t ps[4];
@@ -807,6 +827,21 @@ void renormalize(Ctx& c, const acetn_site* s1, int k, const double* P1i, const d
     g.bk = plain(D2 * cf); g.bn = grouped((int)D2, cf, 1);
     g.cm = plain(D2 * cf); g.cn = plain(1);
     g.alpha = 1.0; g.beta = 0.0;
+    const double* Ea = s1->E[ke];
+    const double* Pb = Pf;
+    if (!c.mixed && gemm_f64_large(g.M, g.N, g.K)) {
+      // both operands with plain strides (route 1 reads E as it is)
+      if (!r1) {
+        Ea = swap_edge(c, Ea, xa, xb, D2);
+        g.am = plain(1); g.ak = plain(xa * D2);
+      } else {
+        g.am = plain(1);
+      }
+      double* Pp = c.take((size_t)xs * D2 * cf);
+      if (c.launch) permute3(Pf, Pp, xs, cf, D2, D2 * cf, 1, cf, c.st);
+      Pb = Pp;
+      g.bn = plain(1);
+    }
     // E_o[i][j][r][R] = Z[(c,r,R)][(f,q,Q)] . Ps[(f,q,Q)][last column]
     GemmDesc h{};
     h.M = (int)(cf * D2); h.N = (int)cs; h.K = (int)(xf * D2);
@@ -831,7 +866,7 @@ void renormalize(Ctx& c, const acetn_site* s1, int k, const double* P1i, const d
       b.A[0] = s1->E[ke]; b.B[0] = Pf; b.C[0] = T;
       gemm_split(g, b, c.split, DType::F64, DType::F64, DType::F32, c.gwork, c.gwork_elems, c.st);
     } else {
-      gemm(c, g, s1->E[ke], Pf, T);
+      gemm(c, g, Ea, Pb, T);
     }
     if (c.launch) {
       int64_t ps[4];
@@ -880,8 +915,7 @@ void site_rdm(Ctx& c, const acetn_site* s, double* rho) {
   // t1b[c][l][L][e][d][D] = sum_a t1a[a][(c,l,L)] e3[e][a][(d,D)]
   const int64_t N1 = c4 * D2, Ne = e3 * D2;
   double* t1b = c.take((size_t)N1 * Ne);
-  gemm(c, gdesc((int)N1, (int)Ne, (int)a0, plain(1), plain(N1), plain(D2),
-                grouped((int)D2, 1, a0 * D2), plain(Ne), plain(1)), t1a, s->E[2], t1b);
+  corner_edge(c, t1a, N1, s->E[2], e3, a0, D2, t1b);
   // t1c[c][l][e][d][U][R][P] = sum_{L,D} t1b[c][l][L][e][d][D] abar[L][U][R][D][P]
   const int64_t Mc = c4 * D * e3 * D, Nc = D2 * d;
   double* t1c = c.take((size_t)Mc * Nc);
@@ -914,8 +948,7 @@ void site_rdm(Ctx& c, const acetn_site* s, double* rho) {
   ACETN_REQUIRE(c1 == e2, "site rdm: e1/c2 mismatch");
   const int64_t Mb = b3 * D2, Na = a1 * D2;
   double* t3c = c.take((size_t)Mb * Na);
-  gemm(c, gdesc((int)Mb, (int)Na, (int)e2, plain(1), plain(Mb), plain(D2),
-                grouped((int)D2, 1, c1 * D2), plain(Na), plain(1)), t3b, t2, t3c);
+  corner_edge(c, t3b, Mb, t2, a1, e2, D2, t3c);
   // t4[r][u][l][d][P] = sum_{e,R,c,U} t3c[e][r][R][c][u][U] t1c[c][l][e][d][U][R][P]
   //   (t3c's leading index b plays e, its a plays c)
   ACETN_REQUIRE(b3 == e3 && a1 == c4, "site rdm: ring dimension mismatch");
@@ -960,8 +993,7 @@ void bond_halves(Ctx& c, const acetn_site* s1, const acetn_site* s2, int k, cons
   double* rt1 = c.take((size_t)c12a * Mr);
   mm(c, (int)c12a, (int)Mr, (int)c12b, false, s1->C[k1], c12b, false, s1->E[k1], Mr, rt1, Mr);
   double* rt2 = c.take((size_t)Mr * Nr);
-  gemm(c, gdesc((int)Mr, (int)Nr, (int)c12a, plain(1), plain(Mr), plain(D2),
-                grouped((int)D2, 1, c12a * D2), plain(Nr), plain(1)), rt1, s1->E[k], rt2);
+  corner_edge(c, rt1, Mr, s1->E[k], ne, c12a, D2, rt2);
   const int64_t Lr = ne * D2 * d2;                     // row length of t: (c,L,P,l,p)
   double* t = c.take((size_t)nc * D2 * Lr);
   if (c.launch) {
@@ -981,12 +1013,12 @@ void bond_halves(Ctx& c, const acetn_site* s1, const acetn_site* s2, int k, cons
   ACETN_REQUIRE(s1->E_dim[k2][0] == c13b, "bond rdm: c13/e13 mismatch");
   ACETN_REQUIRE(c13a == nc, "bond rdm: c13/e12 mismatch");
   const int64_t F = s1->E_dim[k2][1];
+  // r1a[f][a][D2]: written with a first, so that the product over (a,d,D) reads it plainly
   double* r1a = c.take((size_t)c13a * F * D2);
-  mm(c, (int)c13a, (int)(F * D2), (int)c13b, false, s1->C[k2], c13b, false, s1->E[k2], F * D2, r1a,
-     F * D2);
+  gemm(c, gdesc((int)c13a, (int)(F * D2), (int)c13b, plain(c13b), plain(1), plain(F * D2), plain(1),
+                plain(D2), grouped((int)D2, 1, nc * D2)), s1->C[k2], s1->E[k2], r1a);
   double* r1 = c.take((size_t)F * Lr);
-  gemm(c, gdesc((int)F, (int)Lr, (int)(nc * D2), plain(D2), grouped((int)D2, 1, F * D2), plain(Lr),
-                plain(1), plain(Lr), plain(1)), r1a, t, r1);
+  mm(c, (int)F, (int)Lr, (int)(nc * D2), false, r1a, nc * D2, false, t, Lr, r1, Lr);
   // ---------------- left half (site s2)
   const int64_t c21a = s2->C_dim[k][0], c21b = s2->C_dim[k][1];
   ACETN_REQUIRE(s2->E_dim[k][0] == c21b, "bond rdm: c21/e21 mismatch");
@@ -997,8 +1029,7 @@ void bond_halves(Ctx& c, const acetn_site* s1, const acetn_site* s2, int k, cons
   double* lt1 = c.take((size_t)c21a * Ml);
   mm(c, (int)c21a, (int)Ml, (int)c21b, false, s2->C[k], c21b, false, s2->E[k], Ml, lt1, Ml);
   double* lt2 = c.take((size_t)Ml * Nl);
-  gemm(c, gdesc((int)Ml, (int)Nl, (int)c21a, plain(1), plain(Ml), plain(D2),
-                grouped((int)D2, 1, c21a * D2), plain(Nl), plain(1)), lt1, s2->E[k3], lt2);
+  corner_edge(c, lt1, Ml, s2->E[k3], me, c21a, D2, lt2);
   const int64_t Ll = mc * D2 * d2;                     // row length of t2: (c,R,Q,r,q)
   double* t2 = c.take((size_t)me * D2 * Ll);
   if (c.launch) {
@@ -1019,11 +1050,12 @@ void bond_halves(Ctx& c, const acetn_site* s1, const acetn_site* s2, int k, cons
   ACETN_REQUIRE(s2->E_dim[k2][1] == c24a, "bond rdm: c24/e23 mismatch");
   const int64_t F2 = s2->E_dim[k2][0];
   double* r2a = c.take((size_t)me * F2 * D2);
+  // r2a[f][e][D2], as r1a
   gemm(c, gdesc((int)me, (int)(F2 * D2), (int)c24a, plain(1), plain(c24b), plain(D2),
-                grouped((int)D2, 1, c24a * D2), plain(F2 * D2), plain(1)), s2->C[k3], s2->E[k2], r2a);
+                grouped((int)D2, 1, c24a * D2), plain(D2), grouped((int)D2, 1, me * D2)), s2->C[k3],
+       s2->E[k2], r2a);
   double* r2 = c.take((size_t)F2 * Ll);
-  gemm(c, gdesc((int)F2, (int)Ll, (int)(me * D2), plain(D2), grouped((int)D2, 1, F2 * D2),
-                plain(Ll), plain(1), plain(Ll), plain(1)), r2a, t2, r2);
+  mm(c, (int)F2, (int)Ll, (int)(me * D2), false, r2a, me * D2, false, t2, Ll, r2, Ll);
   ACETN_REQUIRE(F == F2 && ne == mc, "bond network: halves do not close");
   out.r1 = r1;
   out.r2 = r2;

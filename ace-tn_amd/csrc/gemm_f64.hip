@@ -97,7 +97,6 @@ void kernel_timing_end(hipEvent_t e0, hipStream_t s, int cls, double flops, doub
 
 namespace {
 constexpr int BK = 16, NT = 256;
-constexpr double kPipeMinMacs = 5e7;
 
 __device__ __forceinline__ bool contiguous(const IdxMap& m) { return m.s0 == 1; }
 
@@ -503,8 +502,7 @@ __global__ __launch_bounds__(PP_NT, 2) void gemm_f64_pipe_kernel(GemmDesc g, con
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 // Shapes the pipelined kernel takes over: plainly strided as above (rows of even
-// length: no 16-byte piece reaches past one), and large enough that 64-row tiles and a few k parts fill the chip: below 5e7 products
-// (324 x 38 x 324 has 4e6) a call is launches and latency either way.
+// length: no 16-byte piece reaches past one) and large (gemm_f64_large).
 bool pipe_shape(const GemmDesc& g, int count) {
   if (!g.pipe || count != 1) return false;
   if (g.am.n0 > 0 || g.ak.n0 > 0 || g.bk.n0 > 0 || g.bn.n0 > 0) return false;
@@ -512,8 +510,7 @@ bool pipe_shape(const GemmDesc& g, int count) {
   if (!am && g.ak.s0 != 1) return false;
   const int64_t lda = am ? g.ak.s0 : g.am.s0, alen = am ? g.M : g.K;
   if (g.bn.s0 != 1 || ((lda | alen | g.bk.s0 | g.N) & 1)) return false;
-  return g.M >= 96 && g.N >= 17 && g.K >= 32 &&
-         (double)g.M * g.N * g.K >= kPipeMinMacs;
+  return gemm_f64_large(g.M, g.N, g.K);
 }
 int pipe_wn(const GemmDesc& g) {
   const int nt = (g.N + 16 * PP_MAXWN - 1) / (16 * PP_MAXWN);
@@ -693,6 +690,13 @@ void launch_gemm_wide(const GemmDesc& g, const GemmBatch& b, int ks, double* wor
                      ks, work);
 }
 }  // namespace
+
+// Large enough that 64-row tiles and a few k parts fill the chip: below 5e7
+// products (324 x 38 x 324 has 4e6) a call is launches and latency either way,
+// and 1024 x 66 x 1024 (7e7) takes 17 us against 20.
+bool gemm_f64_large(int64_t M, int64_t N, int64_t K) {
+  return M >= 96 && N >= 17 && K >= 32 && (double)M * N * K >= 5e7;
+}
 
 size_t gemm_f64_work_elems(const GemmDesc& g, int count) {
   if (dot_small_fits(g)) return (size_t)dot_small_wgs(g) * count * kDotMax * kDotMax;

@@ -104,6 +104,9 @@ struct GemmBatch {
 void gemm_f64(const GemmDesc& g, const GemmBatch& b, double* work, size_t work_elems,
               hipStream_t s);
 size_t gemm_f64_work_elems(const GemmDesc& g, int count);
+// whether a product of this size is worth plainly strided operands (the
+// pipelined kernel then takes it)
+bool gemm_f64_large(int64_t M, int64_t N, int64_t K);
 
 // Split-bf16 GEMM (v_mfma_f32_16x16x32_bf16, FP32 accumulation): operands
 // are rounded to FP32 and split into ``split`` bf16 pieces (2: "bf16x3",
@@ -321,6 +324,9 @@ void fix_projector_gauge(double* P1, double* P2, int64_t rows1, int64_t rows2, i
                          hipStream_t st);
 // x /= ||x||_F over n elements (two-pass, deterministic).
 void frobenius_normalize(double* x, int64_t n, double* scratch, hipStream_t st);
+// out (n0 x n1 x n2, contiguous) [i][j][k] = in[i s0 + j s1 + k s2].
+void permute3(const double* in, double* out, int64_t n0, int64_t n1, int64_t n2, int64_t s0,
+              int64_t s1, int64_t s2, hipStream_t st);
 // out[i] = sum of squares partials; used by tests for norms.
 void zero_fill(double* x, int64_t n, hipStream_t st);
 

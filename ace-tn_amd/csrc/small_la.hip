@@ -1372,6 +1372,16 @@ __global__ void zero_kernel(double* x, int64_t n) {
     x[i] = 0.0;
 }
 
+// out[i][j][k] (contiguous, n1 x n2 inner) = in[i s0 + j s1 + k s2]
+__global__ void permute3_kernel(const double* __restrict__ in, double* __restrict__ out,
+                                unsigned total, unsigned n1, unsigned n2, int64_t s0, int64_t s1,
+                                int64_t s2) {
+  for (unsigned e = blockIdx.x * blockDim.x + threadIdx.x; e < total; e += gridDim.x * blockDim.x) {
+    const unsigned k = e % n2, r = e / n2;
+    out[e] = in[r / n1 * s0 + r % n1 * s1 + k * s2];
+  }
+}
+
 size_t packed_bytes(int n) { return sizeof(double) * (size_t)n * (n + 1) / 2; }
 
 }  // namespace
@@ -1560,6 +1570,17 @@ void frobenius_normalize(double* x, int64_t n, double* scratch, hipStream_t st) 
   hipLaunchKernelGGL(sumsq_kernel, dim3(blocks), dim3(256), 0, st, x, n, scratch);
   ACETN_HIP_CHECK(hipGetLastError());
   hipLaunchKernelGGL(scale_by_norm_kernel, dim3(blocks), dim3(256), 0, st, x, n, scratch, blocks);
+  ACETN_HIP_CHECK(hipGetLastError());
+}
+
+void permute3(const double* in, double* out, int64_t n0, int64_t n1, int64_t n2, int64_t s0,
+              int64_t s1, int64_t s2, hipStream_t st) {
+  const int64_t total = n0 * n1 * n2;
+  if (total <= 0) return;
+  ACETN_REQUIRE(total < (int64_t(1) << 31), "permute3: tensor too large");
+  const int blocks = (int)std::min<int64_t>((total + 255) / 256, 4096);
+  hipLaunchKernelGGL(permute3_kernel, dim3(blocks), dim3(256), 0, st, in, out, (unsigned)total,
+                     (unsigned)n1, (unsigned)n2, s0, s1, s2);
   ACETN_HIP_CHECK(hipGetLastError());
 }
 
