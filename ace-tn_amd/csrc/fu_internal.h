@@ -5,7 +5,7 @@
 namespace acetn {
 
 constexpr int kQrMaxN = 32;   // Householder QR: at most 32 columns
-constexpr int kSvdMaxN = 32;  // one-sided Jacobi SVD: at most 64 x 32
+constexpr int kSvdMaxN = 32;  // one-sided Jacobi SVD: at most 32 x 32
 
 // out (contiguous, dims od[0..n-1]) = scale * in[sum_i idx_i * is[i]]
 struct PermDesc {
@@ -20,11 +20,26 @@ void permute_copy(const double* in, double* out, const PermDesc& p, double scale
 // W (m x n) scratch, Q (m x n, thin; may be null), R (n x n).
 void householder_qr(const double* A, int m, int n, double* W, double* Q, double* R, hipStream_t s);
 
-// One-sided Jacobi SVD, A (m x n, m <= 64, n <= 32) = U diag(s) V^T,
-// U (m x n), V (n x n), s descending.
-void svd_small(const double* A, int m, int n, double* U, double* sv, double* V, hipStream_t s);
+// One factorisation of a permuted tensor: element (i, c) of the m x n matrix is
+// A[(i / (rd0 rd1)) rs0 + (i / rd1 % rd0) rs1 + (i % rd1) rs2 + (c / cd) cs0 + (c % cd) cs1],
+// rd0 rd1 dividing m and cd dividing n.
+struct QrProblem {
+  const double* A;
+  double* Q;  // m x n, thin; may be null
+  double* R;  // n x n
+  int rd0, rd1, cd;
+  int64_t rs[3], cs[2];
+};
+// ``count`` (1 or 2) factorisations of the same shape side by side; M and W
+// (m x n) are scratch for shapes the register kernel does not hold.
+void householder_qr_pair(const QrProblem& a, const QrProblem& b, int count, int m, int n,
+                         double* M, double* W, hipStream_t s);
+
+// One-sided Jacobi SVD, A (n x n, n <= 32) = U diag(s) V^T, s descending (a
+// column of V at a vanishing singular value may be zero).
+void svd_small(const double* A, int n, double* U, double* sv, double* V, hipStream_t s);
 // ``count`` problems, matrices (A, U, V) ``stride`` doubles apart, sv n apart.
-void svd_small_batch(const double* A, int m, int n, double* U, double* sv, double* V, int count,
+void svd_small_batch(const double* A, int n, double* U, double* sv, double* V, int count,
                      int64_t stride, hipStream_t s);
 
 void lower_to_full(double* M, int n, hipStream_t s);

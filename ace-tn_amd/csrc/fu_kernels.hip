@@ -4,6 +4,7 @@
 // the persistent ALS solver, and a strided permute-copy.
 #include "internal.h"
 #include "fu_internal.h"
+#include "lanes.h"
 
 #include <algorithm>
 #include <cmath>
@@ -150,16 +151,174 @@ __global__ __launch_bounds__(QR_NT) void householder_qr_kernel(const double* __r
   }
 }
 
-// ---------------------------------------------------------------------------
-// One-sided (Hestenes) Jacobi SVD of a tiny dense m x n matrix (m <= 64,
-// n <= 32): A V = U S with S descending.  One wave per column pair (lane i
-// holds row i), round-robin pair ordering; a pair is rotated while
-// |a_p . a_q| > 1e-15 * ||a_p|| ||a_q||.
-// ---------------------------------------------------------------------------
-constexpr int SVD_NT = 1024;
+// The same factorisation with the whole matrix in registers, up to 64 NWV R
+// rows and NC columns, one workgroup per problem (one or two): row i is in
+// thread i mod 64 NWV.  A column costs one exchange: the products of column j
+// with itself and with all later ones are summed together (v^T W[:, c] =
+// W[j][c] + (sum_{i > j} W[i][j] W[i][c]) / (alpha - beta)), where the kernel
+// above makes three passes over memory and three block sums.  The input is
+// read through its permutation (rows of up to three digits, columns of two).
+// Latency-bound: 216 x 12 (D=6, d=2) 26 us the pair against 246 us each.
+template <int NC, int R, int NWV>
+__global__ __launch_bounds__(64 * NWV) void qr_reg_kernel(QrProblem p0, QrProblem p1, int m, int n) {
+  constexpr int NT = 64 * NWV;
+  __shared__ double part[2][NWV][NC], rowj[2][NC];
+  const QrProblem& p = blockIdx.x ? p1 : p0;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int kmax = min(m, n);
+  double w[R][NC];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int i = min(tid + NT * r, m - 1);
+    const int64_t ro = (int64_t)(i / (p.rd1 * p.rd0)) * p.rs[0] +
+                       (int64_t)(i / p.rd1 % p.rd0) * p.rs[1] + (int64_t)(i % p.rd1) * p.rs[2];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      const int cc = min(c, n - 1);
+      const double v = p.A[ro + (int64_t)(cc / p.cd) * p.cs[0] + (int64_t)(cc % p.cd) * p.cs[1]];
+      w[r][c] = (c < n && tid + NT * r < m) ? v : 0.0;
+    }
+  }
+  // sums of g over the workgroup: lane l gets that of value l mod 16; one
+  // barrier, buffers in turn
+  auto sum_all = [&](const double (&g)[NC], int buf) {
+    double k[NC / 4];
+    sum64_many<NC>(g, k);
+    const int at = lanes_of(lane);
+#pragma unroll
+    for (int t = 0; t < NC / 4; ++t)
+      if ((lane & 15) == t) part[buf][wave][4 * t + at] = k[t];
+    __syncthreads();
+    double s = 0.0;
+    const int c = min(lane & 15, NC - 1);
+#pragma unroll
+    for (int x = 0; x < NWV; ++x) s += part[buf][x][c];
+    return s;
+  };
+  double tau[NC];
+#pragma unroll
+  for (int j = 0; j < NC; ++j) {
+    tau[j] = 0.0;
+    if (j >= kmax) continue;
+    double g[NC];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) g[c] = 0.0;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const double x = tid + NT * r > j ? w[r][j] : 0.0;
+#pragma unroll
+      for (int c = j; c < NC; ++c) g[c] = fma(x, w[r][c], g[c]);
+    }
+    if (tid == j) {
+#pragma unroll
+      for (int c = j; c < NC; ++c) rowj[j & 1][c] = w[0][c];
+    }
+    const double gs = sum_all(g, j & 1);
+    const double row = rowj[j & 1][min(lane & 15, NC - 1)];
+    const double alpha = lane_value(row, j), xnorm2 = lane_value(gs, j);
+    double beta = alpha, t = 0.0, scal = 0.0;
+    if (xnorm2 > 0.0) {
+      beta = -copysign(sqrt(alpha * alpha + xnorm2), alpha);
+      t = (beta - alpha) / beta;
+      scal = 1.0 / (alpha - beta);
+    }
+    tau[j] = t;
+    const double wl = t * fma(scal, gs, row);
+    double v[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int i = tid + NT * r;
+      v[r] = i > j ? w[r][j] * scal : (i == j ? 1.0 : 0.0);
+      w[r][j] = i > j ? v[r] : (i == j ? beta : w[r][j]);
+    }
+#pragma unroll
+    for (int c = j + 1; c < NC; ++c) {
+      const double x = lane_value(wl, c);
+#pragma unroll
+      for (int r = 0; r < R; ++r) w[r][c] = fma(-v[r], x, w[r][c]);
+    }
+  }
+  // R (n x n, upper; rows beyond kmax are zero): row i is in thread i
+  if (tid < n) {
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+      if (c < n) p.R[tid * n + c] = (tid <= c && tid < kmax) ? w[0][c] : 0.0;
+  }
+  if (p.Q == nullptr) return;
+  // thin Q = H_0 ... H_{kmax-1} I[:, :kmax]  (m x kmax, leading dimension n)
+  double q[R][NC];
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+#pragma unroll
+    for (int c = 0; c < NC; ++c) q[r][c] = tid + NT * r == c ? 1.0 : 0.0;
+  int buf = kmax & 1;  // the factorisation's last buffer was the other one
+#pragma unroll
+  for (int j = NC - 1; j >= 0; --j) {
+    if (j >= kmax) continue;
+    const double t = tau[j];
+    if (t == 0.0) continue;
+    double g[NC], v[R];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) g[c] = 0.0;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int i = tid + NT * r;
+      v[r] = i > j ? w[r][j] : (i == j ? 1.0 : 0.0);
+#pragma unroll
+      for (int c = j; c < NC; ++c) g[c] = fma(v[r], q[r][c], g[c]);
+    }
+    const double wl = t * sum_all(g, buf);
+    buf ^= 1;
+#pragma unroll
+    for (int c = j; c < NC; ++c) {
+      const double x = lane_value(wl, c);
+#pragma unroll
+      for (int r = 0; r < R; ++r) q[r][c] = fma(-v[r], x, q[r][c]);
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+      if (c < n && tid + NT * r < m) p.Q[(int64_t)(tid + NT * r) * n + c] = c < kmax ? q[r][c] : 0.0;
+}
 
-__global__ __launch_bounds__(SVD_NT) void svd_small_kernel(const double* __restrict__ A, int m,
-                                                           int n, double* __restrict__ U,
+// ---------------------------------------------------------------------------
+// SVD of a tiny dense n x n matrix (n <= 32), A V = U S with S descending:
+// Householder QR of the columns in falling order of their norms, A P = Q R,
+// then one-sided (Hestenes) Jacobi on the columns of R^T, which the graded
+// rows of R leave in 6 - 8 sweeps where the columns of A itself take 8 to 19:
+// R^T W = Y S, so U = Q W and V = P Y.  Half a wave per column pair (lane i
+// holds row i), round-robin pair ordering; a pair is rotated while
+// |a_p . a_q| > 1e-15 * ||a_p|| ||a_q||.  Bound by instruction issue: one
+// barrier a round, the three inner products summed by lane exchanges without
+// LDS, the rotation by refined hardware reciprocals (24 x 24, graded: 114
+// us; 153 us with a wave a pair, 270 us without the factorisation as well,
+// 430 us with shuffles and full divisions).
+// ---------------------------------------------------------------------------
+constexpr int SVD_NT = 512;  // at most: half a wave for each of n / 2 pairs
+
+// the tangent of the rotation where squares would leave the range of a double
+__device__ __noinline__ double tiny_tangent(double dl, double ga) {
+  const double zeta = dl / (2.0 * ga);
+  return (zeta >= 0.0 ? 1.0 : -1.0) / (fabs(zeta) + sqrt(1.0 + zeta * zeta));
+}
+
+// order[]: 0..n-1 by falling nrm (the identity where NaNs leave ranks empty)
+__device__ __forceinline__ void falling_order(const double* nrm, int* order, int n) {
+  const int tid = threadIdx.x;
+  if (tid < n) order[tid] = tid;
+  __syncthreads();
+  if (tid < n) {
+    int rank = 0;
+    for (int j = 0; j < n; ++j) rank += (nrm[j] > nrm[tid]) || (nrm[j] == nrm[tid] && j < tid);
+    order[rank] = tid;
+  }
+  __syncthreads();
+}
+
+__global__ __launch_bounds__(SVD_NT) void svd_small_kernel(const double* __restrict__ A, int n,
+                                                           double* __restrict__ U,
                                                            double* __restrict__ s,
                                                            double* __restrict__ V,
                                                            int64_t batch_stride) {
@@ -169,79 +328,125 @@ __global__ __launch_bounds__(SVD_NT) void svd_small_kernel(const double* __restr
   U += blockIdx.x * batch_stride;
   V += blockIdx.x * batch_stride;
   s += (int64_t)blockIdx.x * n;
-  __shared__ double a[kSvdMaxN + 1][64];   // columns, padded to even count
-  __shared__ double v[kSvdMaxN + 1][kSvdMaxN + 1];
-  __shared__ double nrm[kSvdMaxN + 1];
-  __shared__ int order[kSvdMaxN + 1];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  constexpr int LD = kSvdMaxN + 1;
+  __shared__ double a[kSvdMaxN][LD];   // columns of A P, then of R^T
+  __shared__ double vh[kSvdMaxN][LD];  // columns of A, then the reflectors, zero above their one
+  __shared__ double v[kSvdMaxN][LD];   // columns of W
+  __shared__ double nrm[kSvdMaxN], tau[kSvdMaxN];
+  __shared__ int order[kSvdMaxN], perm[kSvdMaxN];
+  const int tid = threadIdx.x, lane = tid & 63, l = lane & 31, nt = blockDim.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // a unit (half a wave) has one pair and up to two columns, unit + {0, units}
+  const int unit = tid >> 5, units = nt >> 5;
   const int nn = n + (n & 1);
-  for (int e = tid; e < (kSvdMaxN + 1) * 64; e += SVD_NT) {
-    const int c = e / 64, r = e % 64;
-    a[c][r] = (c < n && r < m) ? A[r * n + c] : 0.0;
+  auto norms = [&](const double (*x)[LD]) {
+    for (int c0 = 0; c0 < n; c0 += units) {
+      const int c = c0 + unit;
+      const double y = x[min(c, n - 1)][l], ss = sum32(y * y);
+      if (l == 0 && c < n) nrm[c] = sqrt(ss);
+    }
+    __syncthreads();
+  };
+  for (int e = tid; e < kSvdMaxN * 32; e += nt) {
+    const int c = e & 31, r = e >> 5;
+    vh[c][r] = (c < n && r < n) ? A[r * n + c] : 0.0;
+    v[c][r] = (r == c) ? 1.0 : 0.0;
   }
-  for (int e = tid; e < (kSvdMaxN + 1) * (kSvdMaxN + 1); e += SVD_NT) {
-    const int r = e / (kSvdMaxN + 1), c = e % (kSvdMaxN + 1);
-    v[r][c] = (r == c) ? 1.0 : 0.0;
+  __syncthreads();
+  norms(vh);
+  falling_order(nrm, perm, n);
+  for (int c = unit; c < n; c += units) a[c][l] = vh[perm[c]][l];
+  // QR: the wave of column j + 1 prepares its reflector behind the update by
+  // reflector j
+  auto reflector = [&](int j) {
+    const double x = a[j][l];
+    const double xnorm2 = sum32(l > j ? x * x : 0.0), alpha = lane_value(x, j);
+    double beta = alpha, t = 0.0, scal = 0.0;
+    if (xnorm2 > 0.0) {
+      beta = -copysign(sqrt(alpha * alpha + xnorm2), alpha);
+      t = (beta - alpha) / beta;
+      scal = 1.0 / (alpha - beta);
+    }
+    vh[j][l] = l > j ? x * scal : (l == j ? 1.0 : 0.0);
+    a[j][l] = l > j ? 0.0 : (l == j ? beta : x);
+    if (lane == 0) tau[j] = t;
+  };
+  __syncthreads();  // vh read by all
+  if (wave == 0) reflector(0);
+  __syncthreads();
+  for (int j = 0; j + 1 < n; ++j) {
+    const double h = vh[j][l], t = tau[j];
+    for (int c0 = j + 1 >= units ? units : 0; c0 < n; c0 += units) {
+      const int c = c0 + unit;
+      const double x = a[min(c, n - 1)][l], y = fma(-t * sum32(h * x), h, x);
+      if (c > j && c < n) a[c][l] = y;
+    }
+    const int own = j + 1 >= units ? j + 1 - units : j + 1;
+    if (wave == own >> 1) reflector(j + 1);
+    __syncthreads();
   }
+  // a <- R^T: column c is row c of R
+  const int c1 = min(unit + units, n - 1);
+  const double t0 = a[l][min(unit, n - 1)], t1 = a[l][c1];
+  __syncthreads();
+  if (unit < n) a[unit][l] = l < n && l >= unit ? t0 : 0.0;
+  if (unit + units < n) a[c1][l] = l < n && l >= c1 ? t1 : 0.0;
   __syncthreads();
   for (int sweep = 0; sweep < 60; ++sweep) {
     int rot = 0;
     for (int r = 0; r < nn - 1; ++r) {
-      const int pr = wave;
-      if (pr < nn / 2) {
-        int x, y;
-        if (pr == 0) { x = nn - 1; y = r; }
-        else { x = (r + pr) % (nn - 1); y = (r - pr + nn - 1) % (nn - 1); }
-        const int p = min(x, y), q = max(x, y);
-        if (q < n) {
-          const double ap = a[p][lane], aq = a[q][lane];
-          double al = ap * ap, be = aq * aq, ga = ap * aq;
-          for (int o = 32; o > 0; o >>= 1) {
-            al += __shfl_xor(al, o);
-            be += __shfl_xor(be, o);
-            ga += __shfl_xor(ga, o);
-          }
-          if (ga != 0.0 && fabs(ga) > 1e-15 * sqrt(al * be)) {
-            const double zeta = (be - al) / (2.0 * ga);
-            const double t = (zeta >= 0.0 ? 1.0 : -1.0) / (fabs(zeta) + sqrt(1.0 + zeta * zeta));
-            const double c = 1.0 / sqrt(1.0 + t * t), sn = c * t;
-            a[p][lane] = c * ap - sn * aq;
-            a[q][lane] = sn * ap + c * aq;
-            if (lane < n) {
-              const double vp = v[lane][p], vq = v[lane][q];
-              v[lane][p] = c * vp - sn * vq;
-              v[lane][q] = sn * vp + c * vq;
-            }
-            rot = 1;
-          }
-        }
+      int x = nn - 1, y = r;
+      if (unit > 0) {
+        x = r + unit;
+        if (x >= nn - 1) x -= nn - 1;
+        y = r - unit;
+        if (y < 0) y += nn - 1;
+      }
+      const int p = min(x, y), q = max(x, y);
+      const bool pair = unit < nn / 2 && q < n;
+      const int pc = pair ? p : 0, qc = pair ? q : 0;
+      const double ap = a[pc][l], aq = a[qc][l], vp = v[pc][l], vq = v[qc][l];
+      // row 0 of the half sums one value, row 1 the other
+      const double n2 = sum16(swap16_sum(ap * ap, aq * aq));
+      const double ga = sum32(ap * aq);
+      double al, be;
+      swap16(n2, n2, al, be);
+      const double ab = al * be;
+      // in squares unless they leave the range of a double
+      if (pair && ga != 0.0 &&
+          (ab > 1e-200 ? ga * ga > 1e-30 * ab : fabs(ga) > 1e-15 * sqrt(ab))) {
+        // t = sgn(zeta) / (|zeta| + sqrt(1 + zeta^2)), zeta = (be - al) / (2 ga)
+        const double dl = be - al, h2 = fma(dl, dl, 4.0 * ga * ga);
+        const double t = h2 > 1e-280 && h2 < 1e280
+                             ? copysign(2.0, dl) * ga * rcp_nr(fabs(dl) + h2 * rsqrt_nr(h2))
+                             : tiny_tangent(dl, ga);
+        const double c = rsqrt_nr(fma(t, t, 1.0)), sn = c * t;
+        a[p][l] = c * ap - sn * aq;
+        a[q][l] = sn * ap + c * aq;
+        v[p][l] = c * vp - sn * vq;
+        v[q][l] = sn * vp + c * vq;
+        rot = 1;
       }
       __syncthreads();
     }
     if (!__syncthreads_or(rot)) break;
   }
-  for (int c = wave; c < n; c += SVD_NT / 64) {
-    const double x = a[c][lane];
-    double ss = x * x;
-    for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o);
-    if (lane == 0) nrm[c] = sqrt(ss);
+  norms(a);
+  falling_order(nrm, order, n);
+  // U = Q W, a column a unit; V = P Y
+  for (int k0 = 0; k0 < n; k0 += units) {
+    const int k = k0 + unit, c = order[min(k, n - 1)];
+    double u = v[c][l];
+    for (int j = n - 1; j >= 0; --j) {
+      const double h = vh[j][l];
+      u = fma(-tau[j] * sum32(h * u), h, u);
+    }
+    if (k < n && l < n) {
+      U[l * n + k] = u;
+      V[perm[l] * n + k] = nrm[c] > 0.0 ? a[c][l] / nrm[c] : 0.0;
+    }
+    if (k < n && l == 0) s[k] = nrm[c];
   }
-  __syncthreads();
-  if (tid < n) {
-    int rank = 0;
-    for (int j = 0; j < n; ++j) rank += (nrm[j] > nrm[tid]) || (nrm[j] == nrm[tid] && j < tid);
-    order[rank] = tid;
-  }
-  __syncthreads();
-  for (int e = tid; e < m * n; e += SVD_NT) {
-    const int r = e / n, k = e % n, c = order[k];
-    U[e] = nrm[c] > 0.0 ? a[c][r] / nrm[c] : 0.0;
-  }
-  for (int e = tid; e < n * n; e += SVD_NT) {
-    const int r = e / n, k = e % n;
-    V[e] = v[r][order[k]];
-  }
-  if (tid < n) s[tid] = nrm[order[tid]];
 }
 
 // ---------------------------------------------------------------------------
@@ -834,18 +1039,61 @@ void householder_qr(const double* A, int m, int n, double* W, double* Q, double*
   ACETN_HIP_CHECK(hipGetLastError());
 }
 
-void svd_small(const double* A, int m, int n, double* U, double* sv, double* V, hipStream_t s) {
-  ACETN_REQUIRE(m >= 1 && m <= 64 && n >= 1 && n <= kSvdMaxN, "svd_small: unsupported shape");
-  hipLaunchKernelGGL(svd_small_kernel, dim3(1), dim3(SVD_NT), 0, s, A, m, n, U, sv, V,
+namespace {
+template <int NC, int R, int NWV>
+void launch_qr(const QrProblem& a, const QrProblem& b, int count, int m, int n, hipStream_t s) {
+  hipLaunchKernelGGL((qr_reg_kernel<NC, R, NWV>), dim3(count), dim3(64 * NWV), 0, s, a, b, m, n);
+  ACETN_HIP_CHECK(hipGetLastError());
+}
+template <int NC, int R>
+bool launch_qr_rows(const QrProblem& a, const QrProblem& b, int count, int m, int n, hipStream_t s) {
+  if (m <= 64 * R) launch_qr<NC, R, 1>(a, b, count, m, n, s);
+  else if (m <= 128 * R) launch_qr<NC, R, 2>(a, b, count, m, n, s);
+  else if (m <= 256 * R) launch_qr<NC, R, 4>(a, b, count, m, n, s);
+  else if (m <= 512 * R) launch_qr<NC, R, 8>(a, b, count, m, n, s);
+  else return false;
+  return true;
+}
+}  // namespace
+
+void householder_qr_pair(const QrProblem& a, const QrProblem& b, int count, int m, int n,
+                         double* M, double* W, hipStream_t s) {
+  ACETN_REQUIRE(m >= 1 && n >= 1 && n <= kQrMaxN, "householder_qr: unsupported shape");
+  // rows per thread so that the matrix and Q fit the registers
+  bool done = false;
+  if (n <= 4) done = launch_qr_rows<4, 4>(a, b, count, m, n, s);
+  else if (n <= 8) done = launch_qr_rows<8, 4>(a, b, count, m, n, s);
+  else if (n <= 12) done = launch_qr_rows<12, 4>(a, b, count, m, n, s);
+  else if (n <= 16) done = launch_qr_rows<16, 2>(a, b, count, m, n, s);
+  if (done) return;
+  for (int i = 0; i < count; ++i) {
+    const QrProblem& p = i ? b : a;
+    PermDesc d{};
+    d.n = 5; d.total = (int64_t)m * n;
+    d.od[0] = m / (p.rd0 * p.rd1); d.od[1] = p.rd0; d.od[2] = p.rd1; d.od[3] = n / p.cd; d.od[4] = p.cd;
+    for (int x = 0; x < 3; ++x) d.is[x] = p.rs[x];
+    d.is[3] = p.cs[0]; d.is[4] = p.cs[1];
+    permute_copy(p.A, M, d, 1.0, s);
+    householder_qr(M, m, n, W, p.Q, p.R, s);
+  }
+}
+
+namespace {
+int svd_threads(int n) { return 64 * ((n + 3) / 4); }
+}  // namespace
+
+void svd_small(const double* A, int n, double* U, double* sv, double* V, hipStream_t s) {
+  ACETN_REQUIRE(n >= 1 && n <= kSvdMaxN, "svd_small: unsupported shape");
+  hipLaunchKernelGGL(svd_small_kernel, dim3(1), dim3(svd_threads(n)), 0, s, A, n, U, sv, V,
                      (int64_t)0);
   ACETN_HIP_CHECK(hipGetLastError());
 }
 
-void svd_small_batch(const double* A, int m, int n, double* U, double* sv, double* V, int count,
+void svd_small_batch(const double* A, int n, double* U, double* sv, double* V, int count,
                      int64_t stride, hipStream_t s) {
-  ACETN_REQUIRE(m >= 1 && m <= 64 && n >= 1 && n <= kSvdMaxN, "svd_small: unsupported shape");
-  ACETN_REQUIRE(count >= 1 && stride >= (int64_t)m * n, "svd_small_batch: bad batch layout");
-  hipLaunchKernelGGL(svd_small_kernel, dim3(count), dim3(SVD_NT), 0, s, A, m, n, U, sv, V,
+  ACETN_REQUIRE(n >= 1 && n <= kSvdMaxN, "svd_small: unsupported shape");
+  ACETN_REQUIRE(count >= 1 && stride >= (int64_t)n * n, "svd_small_batch: bad batch layout");
+  hipLaunchKernelGGL(svd_small_kernel, dim3(count), dim3(svd_threads(n)), 0, s, A, n, U, sv, V,
                      stride);
   ACETN_HIP_CHECK(hipGetLastError());
 }

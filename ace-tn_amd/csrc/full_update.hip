@@ -49,19 +49,13 @@ void decompose(Ctx& c, const double* A1, const double* A2, int k, const FuDims& 
   if (!c.launch) return;
   int64_t st[4];
   site_strides(D, d, st);
-  PermDesc p{};
-  p.n = 5; p.total = m * nD;
-  p.od[0] = D; p.od[1] = D; p.od[2] = D; p.od[3] = D; p.od[4] = d;
-  // a1: (r, d, u, l, p) of the bond frame; bond axis j is site axis (j + k) % 4
-  p.is[0] = st[(2 + k) & 3]; p.is[1] = st[(3 + k) & 3]; p.is[2] = st[(1 + k) & 3];
-  p.is[3] = st[k]; p.is[4] = 1;
-  permute_copy(A1, M, p, 1.0, c.st);
-  householder_qr(M, (int)m, (int)nD, W, a1q, a1r, c.st);
-  // a2: (d, l, u, r, p)
-  p.is[0] = st[(3 + k) & 3]; p.is[1] = st[k]; p.is[2] = st[(1 + k) & 3];
-  p.is[3] = st[(2 + k) & 3]; p.is[4] = 1;
-  permute_copy(A2, M, p, 1.0, c.st);
-  householder_qr(M, (int)m, (int)nD, W, a2q, a2r, c.st);
+  // a1: (r, d, u, l, p) of the bond frame, a2: (d, l, u, r, p); bond axis j is
+  // site axis (j + k) % 4
+  const QrProblem q1{A1, a1q, a1r, (int)D, (int)D, (int)d,
+                     {st[(2 + k) & 3], st[(3 + k) & 3], st[(1 + k) & 3]}, {st[k], 1}};
+  const QrProblem q2{A2, a2q, a2r, (int)D, (int)D, (int)d,
+                     {st[(3 + k) & 3], st[k], st[(1 + k) & 3]}, {st[(2 + k) & 3], 1}};
+  householder_qr_pair(q1, q2, 2, (int)m, (int)nD, M, W, c.st);
 }
 
 // ---------------------------------------------------------------------------
@@ -158,21 +152,14 @@ void gauge_fix(Ctx& c, const double* nz, const double* a12g_in, const FuDims& f,
   double* nz2 = c.take((size_t)nD3 * nD);
   double* U1 = c.take((size_t)nD2 * d2);
   if (c.launch) {
-    PermDesc p{};
-    p.n = 3; p.total = nD3 * nD;
-    p.od[0] = nD2; p.od[1] = nD; p.od[2] = nD;
-    // nzxr: R of "yxz->zyx" as (nD^3, nD)
-    p.is[0] = 1; p.is[1] = nD * nD2; p.is[2] = nD2;
-    permute_copy(nz, M, p, 1.0, c.st);
-    householder_qr(M, (int)nD3, (int)nD, W, nullptr, nzxr, c.st);
-    // nzyr: R of "yxz->zxy"
-    p.is[0] = 1; p.is[1] = nD2; p.is[2] = nD * nD2;
-    permute_copy(nz, M, p, 1.0, c.st);
-    householder_qr(M, (int)nD3, (int)nD, W, nullptr, nzyr, c.st);
+    // nzxr: R of "yxz->zyx" as (nD^3, nD); nzyr: R of "yxz->zxy"
+    const QrProblem px{nz, nullptr, nzxr, 1, (int)nD, 1, {1, 0, nD * nD2}, {nD2, 0}};
+    const QrProblem py{nz, nullptr, nzyr, 1, (int)nD, 1, {1, 0, nD2}, {nD * nD2, 0}};
+    householder_qr_pair(px, py, 2, (int)nD3, (int)nD, M, W, c.st);
     // pseudo-inverses with absolute cutoff (torch.linalg.pinv(atol=...))
-    svd_small(nzxr, (int)nD, (int)nD, U, sv, V, c.st);
+    svd_small(nzxr, (int)nD, U, sv, V, c.st);
     pinv_finish(U, sv, V, (int)nD, (int)nD, atol, nzxr_inv, c.st);
-    svd_small(nzyr, (int)nD, (int)nD, U, sv, V, c.st);
+    svd_small(nzyr, (int)nD, U, sv, V, c.st);
     pinv_finish(U, sv, V, (int)nD, (int)nD, atol, nzyr_inv, c.st);
   }
   // T[y][z][w] = sum_x nz[y][x][z] nzxr_inv[x][w]
@@ -256,7 +243,7 @@ void plain_start(Ctx& c, const double* a12g, const FuDims& f, double* a1r, doubl
   p.od[0] = nD; p.od[1] = d; p.od[2] = nD; p.od[3] = d;   // "yxpq->ypxq"
   p.is[0] = nD * d * d; p.is[1] = d; p.is[2] = d * d; p.is[3] = 1;
   permute_copy(a12g, M, p, 1.0, c.st);
-  svd_small(M, (int)n, (int)n, U, sv, V, c.st);
+  svd_small(M, (int)n, U, sv, V, c.st);
   hipLaunchKernelGGL(plain_start_kernel, dim3(1), dim3(256), 0, c.st, U, sv, V, (int)nD, (int)D,
                      (int)d, a1r, a2r);
   ACETN_HIP_CHECK(hipGetLastError());
@@ -330,19 +317,15 @@ void finalize_reduced(Ctx& c, const double* a1r_in, const double* a2r_in, const 
     ACETN_HIP_CHECK(hipMemcpyAsync(a2r, a2r_in, sizeof(double) * nD * Dd, hipMemcpyDeviceToDevice, c.st));
   }
   if (c.launch) {
-    PermDesc p{};
-    p.n = 3; p.total = nD * Dd;
-    p.od[0] = nD; p.od[1] = d; p.od[2] = D;   // "yup->ypu"
-    p.is[0] = Dd; p.is[1] = 1; p.is[2] = d;
-    permute_copy(a1r, P, p, 1.0, c.st);
-    householder_qr(P, (int)(nD * d), (int)D, W, q1, r1, c.st);
-    permute_copy(a2r, P, p, 1.0, c.st);
-    householder_qr(P, (int)(nD * d), (int)D, W, q2, r2, c.st);
+    // "yup->ypu"
+    const QrProblem p1{a1r, q1, r1, 1, (int)d, 1, {Dd, 0, 1}, {d, 0}};
+    const QrProblem p2{a2r, q2, r2, 1, (int)d, 1, {Dd, 0, 1}, {d, 0}};
+    householder_qr_pair(p1, p2, 2, (int)(nD * d), (int)D, P, W, c.st);
   }
   // "au,bu->ab"
   mm(c, (int)D, (int)D, (int)D, false, r1, D, true, r2, D, Mr, D);
   if (c.launch) {
-    svd_small(Mr, (int)D, (int)D, U, sv, V, c.st);
+    svd_small(Mr, (int)D, U, sv, V, c.st);
     finalize_scale(U, sv, V, (int)D, (int)D, r1n, r2n, c.st);
   }
   // a1r[y][u][p] = sum_a q1[(y,p)][a] r1n[a][u] ; a2r[x][v][q] = sum_b q2[(x,q)][b] r2n[v][b]
@@ -403,7 +386,7 @@ void simple_update_bond(Ctx& c, const double* A1, const double* A2, int k,
     p.od[0] = nD; p.od[1] = d; p.od[2] = nD; p.od[3] = d;   // "yxrs->yrxs"
     p.is[0] = nD * d * d; p.is[1] = d; p.is[2] = d * d; p.is[3] = 1;
     permute_copy(a12g, M, p, 1.0, c.st);
-    svd_small(M, (int)n, (int)n, U, sv, V, c.st);
+    svd_small(M, (int)n, U, sv, V, c.st);
     su_split(U, sv, V, (int)nD, (int)D, (int)d, a1r, a2r, lam_out, c.st);
     bond_gauge(a1r, a2r, (int)nD, (int)nD, (int)D, (int)d, c.st);
   }
@@ -653,7 +636,7 @@ int acetn_hip_als_solve_batch(const double* n12, const double* a12g, double* a1r
                            (int)f.nD, (int)f.d, M);
         ACETN_HIP_CHECK(hipGetLastError());
         // U and V share one stride so that svd_small_batch can offset both
-        svd_small_batch(M, (int)n, (int)n, U, sv, V, (int)count, n * n, c.st);
+        svd_small_batch(M, (int)n, U, sv, V, (int)count, n * n, c.st);
         hipLaunchKernelGGL(plain_start_batch_kernel, dim3(count), dim3(256), 0, c.st, U, sv, V,
                            (int)f.nD, (int)f.D, (int)f.d, a1r, a2r);
         ACETN_HIP_CHECK(hipGetLastError());

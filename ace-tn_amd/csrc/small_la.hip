@@ -10,6 +10,7 @@
 // The q x q working matrices are kept as packed upper triangles (q(q+1)/2
 // doubles), in LDS when they fit and in a global scratch area otherwise.
 #include "internal.h"
+#include "lanes.h"
 
 #include <cmath>
 
@@ -436,11 +437,6 @@ __global__ __launch_bounds__(CB_NT) void chol_rinv_blk_kernel(const double* __re
 // q = 272 144 against 6050.
 constexpr int kCtMaxQ = 272;          // 17 tile rows: 136 slots, 10 a wave (80 VGPRs)
 constexpr int kCtMaxT = kCtMaxQ / 16;
-
-__device__ __forceinline__ double lane_value(double x, int lane) {
-  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x), lane),
-                          __builtin_amdgcn_readlane(__double2loint(x), lane));
-}
 
 // One wave: Cholesky of the diagonal tile D (LDS, symmetric) with the rank
 // guard, column j of D in lane j and column j of I in lane 16 + j (the upper

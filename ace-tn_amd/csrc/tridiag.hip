@@ -12,56 +12,12 @@
 // conditioned: vectors of separate eigenvalues are orthogonal to eps |G| / gap,
 // and those of one cluster are random in its subspace).
 #include "internal.h"
+#include "lanes.h"
 
 #include <cmath>
 
 namespace acetn {
 namespace {
-
-// ---- sums over lanes by data-parallel moves (no LDS round trip); every lane
-// gets the same bits
-template <int CTRL>
-__device__ __forceinline__ double dpp_mov(double x) {
-  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), CTRL, 0xF, 0xF, false);
-  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), CTRL, 0xF, 0xF, false);
-  return __hiloint2double(hi, lo);
-}
-__device__ __forceinline__ double sum16(double x) {
-  x += dpp_mov<0xB1>(x);   // lane ^ 1
-  x += dpp_mov<0x4E>(x);   // lane ^ 2
-  x += dpp_mov<0x141>(x);  // the other quad of the 8
-  x += dpp_mov<0x140>(x);  // the other half of the row of 16
-  return x;
-}
-// sum over each half-wave of 32
-__device__ __forceinline__ double sum32(double x) {
-  x = sum16(x);
-  const unsigned lo = __double2loint(x), hi = __double2hiint(x);
-  const auto a = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
-  const auto b = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
-  return __hiloint2double(b[0], a[0]) + __hiloint2double(b[1], a[1]);
-}
-__device__ __forceinline__ double sum64(double x) {
-  x = sum32(x);
-  const unsigned lo = __double2loint(x), hi = __double2hiint(x);
-  const auto a = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
-  const auto b = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
-  return __hiloint2double(b[0], a[0]) + __hiloint2double(b[1], a[1]);
-}
-
-// 1/sqrt(x) and 1/x from the hardware approximations with two Newton steps
-// (a few ulps: the reflectors are orthogonal to that much)
-__device__ __forceinline__ double rsqrt_nr(double x) {
-  double y = __builtin_amdgcn_rsq(x);
-  const double h = 0.5 * x;
-  y = y * fma(-h * y, y, 1.5);
-  return y * fma(-h * y, y, 1.5);
-}
-__device__ __forceinline__ double rcp_nr(double x) {
-  double r = __builtin_amdgcn_rcp(x);
-  r = fma(fma(-x, r, 1.0), r, r);
-  return fma(fma(-x, r, 1.0), r, r);
-}
 
 // The reflector H = I - tau u u^T that takes a column with leading entry alpha
 // and |rest|^2 = s2 to beta e_1: u = (alpha - beta, rest).  False: nothing to

@@ -117,3 +117,70 @@ def test_large_gemm_tile_edges(hip, N, ta):
         exact = (A.T if ta else A) @ B
         scale = np.linalg.norm(A, axis=0 if ta else 1)[:, None] * np.linalg.norm(B, axis=0)
         assert np.all(np.abs(C - exact) <= 4.4e-16 * K * scale), (M, N, K)
+
+
+@pytest.mark.parametrize("d", [1, 2, 3, 4])
+@pytest.mark.parametrize("D", [2, 3, 4, 5, 6, 7, 8])
+def test_bond_decompose_shapes(hip, D, d):
+    """The register QR at every column count and wave layout (D^3 x d D, up to
+    512 x 32, where the memory kernel takes over), each bond direction, against
+    LAPACK.  m n half-ulps of the norm for the residual and for the
+    orthonormality; R times the condition of its matrix more."""
+    from oracle import full_update as ofu
+    g = np.random.default_rng(10 * D + d)
+    m, n = D ** 3, D * d
+    for k in range(4):
+        A1, A2 = (g.standard_normal((D, D, D, D, d)) for _ in range(2))
+        a = [np.transpose(A, ofu.bond_permutation(k)) for A in (A1, A2)]
+        ref = ofu.decompose_site_tensors(*a)
+        out = [t.cpu().numpy() for t in hip.bond_decompose(
+            torch.as_tensor(A1, device="cuda"), torch.as_tensor(A2, device="cuda"), k)]
+        for i in (0, 2):
+            assert out[i].shape == ref[i].shape
+            q = out[i].reshape(m, n)
+            assert np.abs(q.T @ q - np.eye(n)).max() <= m * n * 2.0 ** -53
+            R = ref[i + 1]
+            norm, cond = np.linalg.norm(R), np.linalg.cond(np.moveaxis(R, 1, 2).reshape(n, n))
+            tol = m * n * 2.0 ** -53 * cond
+            assert np.abs(out[i + 1] - R).max() <= tol * norm
+            assert np.abs(out[i] - ref[i]).max() <= tol
+
+
+@pytest.mark.parametrize("nD", [1, 2, 3, 4, 5, 6, 7, 8, 12, 16])
+def test_gauge_fix_shapes(hip, nD):
+    """The tall QR pair (nD^3 x nD, 1 to 4096 rows) behind the reduced gauge,
+    through the pseudo-inverses of its factors, whose row signs are free.  The
+    columns are Gaussian, so the condition stays below 100 for nD >= 2."""
+    g = np.random.default_rng(nD)
+    nz = g.standard_normal((nD, nD, nD * nD))
+    a12g = g.standard_normal((nD, nD, 2, 2))
+    _, _, xi, yi = [t.cpu().numpy() for t in hip.gauge_fix(
+        torch.as_tensor(nz, device="cuda"), torch.as_tensor(a12g, device="cuda"), 1e-12)]
+    for h, axis in ((xi, 1), (yi, 0)):
+        A = np.moveaxis(nz, axis, -1).reshape(-1, nD)
+        # pinv(R) pinv(R)^T = (A^T A)^-1
+        exact = np.linalg.inv(A.T @ A)
+        tol = 100 * nD ** 4 * 2.0 ** -53 * np.linalg.cond(A) ** 2
+        assert np.abs(h @ h.T - exact).max() <= tol * np.abs(exact).max()
+
+
+@pytest.mark.parametrize("case", ["full", "graded", "deficient", "equal"])
+@pytest.mark.parametrize("n,scale", [(1, 1.0), (2, 1.0), (3, 1.0), (8, 1.0), (15, 1.0), (24, 1.0),
+                                     (31, 1.0), (32, 1.0), (24, 1e-70), (24, 1e70)])
+def test_small_svd_spectra(hip, n, scale, case):
+    """The one-wave-a-pair Jacobi SVD of the bond update through the plain
+    start, which returns U s^1/2 and V s^1/2 in units of s_0: products of both
+    against the matrix, n^2 rotations' worth of rounding (60 n eps)."""
+    s = {"full": np.linspace(1.0, 0.1, n), "graded": np.exp(-30.0 * np.arange(n) / n),
+         "deficient": np.where(np.arange(n) < (n + 1) // 2, 1.0, 0.0) * np.linspace(1.0, 0.5, n),
+         "equal": np.ones(n)}[case]
+    g = np.random.default_rng(n)
+    U = np.linalg.qr(g.standard_normal((n, n)))[0]
+    V = np.linalg.qr(g.standard_normal((n, n)))[0]
+    M = (U * s) @ V.T
+    a12g = torch.as_tensor(M.reshape(n, n, 1, 1) * scale, device="cuda")
+    a1, a2 = [t.cpu().numpy().reshape(n, n) for t in hip.als_initialize(a12g, n)]
+    tol = 60 * n * 2.2e-16
+    assert np.abs(a1 @ a2.T - M / s[0]).max() <= tol
+    for a, W in ((a1, U), (a2, V)):
+        assert np.abs(a.T @ a - np.diag(s / s[0])).max() <= tol
