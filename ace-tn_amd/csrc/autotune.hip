@@ -4,7 +4,7 @@
 // from hand-set thresholds.  With tuning on, the first product of every new
 // shape (kind, M, N, K, operand flags) instead times each candidate (the
 // four tile shapes, each with split-K counts around its default that fit the
-// caller's scratch) on the caller's stream with HIP events, keeps the
+// caller's scratch, and the small FP64 product in its range) on the caller's stream with HIP events, keeps the
 // fastest, and re-runs it so that the result is the chosen kernel's.  Later
 // products of that shape use the table; a CTMRG iteration repeats the same
 // shapes, so one warmup iteration tunes a whole run.  The table can be saved
@@ -146,7 +146,9 @@ int64_t autotune_load(const char* path) {
                     &ks, &ms, &var) < 8)
       continue;
     const bool tile_ok = (wm == 1 && wn == 5) || (wm == 2 && wn == 5) || (wm == 2 && wn == 2) ||
-                         (wm == 4 && wn == 4);
+                         (wm == 4 && wn == 4) ||
+                         (kind == 0 && wm == 1 && wn == 1 && ks == 1 && var == 0);
+    // 1 x 1 is the small FP64 product (used where the shape is in its range);
     // the wider FP64 variants exist for single-stride products: 2 x 5 tiles
     // in variants 1-3, 1 x 5 tiles in variant 3; two-piece split products
     // have 64-deep k-tiles as variant 1

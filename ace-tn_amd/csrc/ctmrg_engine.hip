@@ -566,6 +566,9 @@ void general_projectors(Ctx& c, const acetn_site* const* st, int k, int system, 
                         int64_t chi, int64_t oversampling, int niter, double cutoff,
                         uint64_t seed, uint64_t sstream, const HalfOut& out, int phase = 0) {
   const bool full = system == kSysFull;
+  // the full-rank branch keeps singular pairs down to 1e-10 of the first, whose
+  // squares follow the rounding of every product (results move by 1e-9 with it)
+  c.in_order = svd == kSvdFullRank;
   const acetn_site* s1 = st[0];
   const acetn_site* s4 = st[3];
   const QuarterDims d1 = quarter_dims(s1, k);

@@ -28,6 +28,7 @@ struct Ctx {
   bool recover = true; // range finder re-derives the columns CholeskyQR drops
   bool trust = false;  // range finder only reports dropped columns (ACETN_HIP_RF_TRUST)
   DropFlags drops;     // where it does
+  bool in_order = false;  // FP64 products keep the plain kernel's order of sums
   int split = 0;       // split level of the products enqueued now (0 = FP64)
 
   double* take(size_t n) {
@@ -81,7 +82,7 @@ struct SplitScope {
 
 inline void gemm(Ctx& c, const GemmDesc& gd, const double* A, const double* B, double* C) {
   GemmDesc g = gd;
-  g.pipe = !c.mixed;
+  g.pipe = !c.mixed && !c.in_order;
   if (!c.run) {
     c.gwork_need = std::max({c.gwork_need, gemm_f64_work_elems(g, 1), gemm_split_work_elems(g, 1)});
     return;

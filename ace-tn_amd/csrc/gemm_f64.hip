@@ -499,6 +499,117 @@ __global__ __launch_bounds__(PP_NT, 2) void gemm_f64_pipe_kernel(GemmDesc g, con
     }
 }
 
+// Small products (M, N and K each a few hundred at most): 64 x 64 tiles leave
+// most CUs empty and every tile a serial chain over K (315 x 37 x 315: 5
+// workgroups, 22.6 us; 66 x 66 x 1024 in 8 k parts: 12.8 us and a 4.4 us sum of
+// the parts).  Here a workgroup owns one 16 x 16 tile and its waves (one for
+// 64 k at most) each a run of k, read straight into registers in the matrix
+// instruction's layout, four k steps a lane at a time; the waves' partial tiles are
+// added in LDS in a fixed order.  Bound by two round trips to L2: 315 x 37 x
+// 315 5.4 us, 66 x 66 x 1024 7.2 us.
+// AK / BC: A's and B's k index has unit stride, so a lane's four steps are two
+// 16-byte loads (their k order is free, the same for A and B).  GEN: any
+// operand maps; the k parts of the addresses are evaluated once into LDS.
+typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));
+constexpr int SP_U = 4;          // k blocks of 16 in flight per wave
+constexpr int SP_MAXK = 3072;
+template <bool AK, bool BC, bool GEN>
+__global__ __launch_bounds__(1024) void gemm_f64_small_kernel(GemmDesc g, GemmBatch bt) {
+  __shared__ double pool[GEN ? 2 * SP_MAXK : 16 * 256];
+  if (g.run_if && *g.run_if == 0) return;
+  const int tid = threadIdx.x, lane = tid & 63, nw = blockDim.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int m0 = blockIdx.y * 16, n0 = blockIdx.x * 16;
+  const int64_t sak = g.ak.s0, sbk = g.bk.s0;
+  const int mr = min(m0 + (lane & 15), g.M - 1), nr = min(n0 + (lane & 15), g.N - 1);
+  const double* __restrict__ pa = bt.A[blockIdx.z] + (GEN ? imap(g.am, mr) : mr * g.am.s0);
+  const double* __restrict__ pb = bt.B[blockIdx.z] + (GEN ? imap(g.bn, nr) : nr * g.bn.s0);
+  int64_t* koff = reinterpret_cast<int64_t*>(pool);
+  if (GEN) {
+    for (int e = tid; e < 2 * g.K; e += blockDim.x)
+      koff[e] = e < g.K ? imap(g.ak, e) : imap(g.bk, e - g.K);
+    __syncthreads();
+  }
+  auto a_at = [&](int k) { return pa[GEN ? koff[k] : k * sak]; };
+  auto b_at = [&](int k) { return pb[GEN ? koff[g.K + k] : k * sbk]; };
+  const int nb = (g.K + 15) / 16, kl = 4 * (lane >> 4);
+  const int b0 = nb * wave / nw, b1 = nb * (wave + 1) / nw;
+  d4 acc = {0.0, 0.0, 0.0, 0.0};
+  for (int b = b0; b < b1; b += SP_U) {
+    double a[SP_U][4], w[SP_U][4];
+#pragma unroll
+    for (int u = 0; u < SP_U; ++u) {
+      if (b + u >= b1) continue;
+      const int k = 16 * (b + u) + kl;
+      if (16 * (b + u) + 16 <= g.K) {
+        if (AK) {
+          const d2u x = *(const d2u*)(pa + k), y = *(const d2u*)(pa + k + 2);
+          a[u][0] = x[0]; a[u][1] = x[1]; a[u][2] = y[0]; a[u][3] = y[1];
+        } else {
+#pragma unroll
+          for (int s = 0; s < 4; ++s) a[u][s] = a_at(k + s);
+        }
+        if (BC) {
+          const d2u x = *(const d2u*)(pb + k), y = *(const d2u*)(pb + k + 2);
+          w[u][0] = x[0]; w[u][1] = x[1]; w[u][2] = y[0]; w[u][3] = y[1];
+        } else {
+#pragma unroll
+          for (int s = 0; s < 4; ++s) w[u][s] = b_at(k + s);
+        }
+      } else {
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          const int kc = min(k + s, g.K - 1);
+          a[u][s] = k + s < g.K ? a_at(kc) : 0.0;
+          w[u][s] = k + s < g.K ? b_at(kc) : 0.0;
+        }
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < SP_U; ++u) {
+      if (b + u >= b1) continue;
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u][s], w[u][s], acc, 0, 0, 0);
+    }
+  }
+  if (GEN) __syncthreads();  // the offsets have been read
+#pragma unroll
+  for (int r = 0; r < 4; ++r) pool[wave * 256 + r * 64 + lane] = acc[r];
+  __syncthreads();
+  for (int e = tid; e < 256; e += blockDim.x) {
+    const int m = m0 + ((e & 63) >> 4) + 4 * (e >> 6), n = n0 + (e & 15);
+    double v = pool[e];
+    for (int w = 1; w < nw; ++w) v += pool[w * 256 + e];
+    if (m >= g.M || n >= g.N) continue;
+    double* C = bt.C[blockIdx.z];
+    const int64_t off = imap(g.cm, m) + imap(g.cn, n);
+    C[off] = (g.beta != 0.0) ? g.alpha * v + g.beta * C[off] : g.alpha * v;
+  }
+}
+
+bool small_shape(const GemmDesc& g, int count) {
+  if (!g.pipe || g.K <= 0) return false;
+  const int64_t tiles = (int64_t)((g.M + 15) / 16) * ((g.N + 15) / 16) * count;
+  // below the pipelined kernel's range; K too long for one workgroup's waves
+  // (102 x 102 x 2500: 15 us against 22, 16 x 16 x 4096: 24 against 16) and
+  // many tiles of next to no k (1000 x 1000 x 20: 12.6 against 11.9) stay
+  // with the split and the larger tiles
+  return (double)g.M * g.N * g.K * count < 5e7 && g.K <= SP_MAXK && tiles <= (g.K >= 32 ? 4096 : 1024);
+}
+void launch_small(const GemmDesc& g, const GemmBatch& b, hipStream_t s) {
+  const dim3 grid((g.N + 15) / 16, (g.M + 15) / 16, b.count);
+  const dim3 block(64 * std::min(16, std::max(1, (g.K + 63) / 64)));
+  const bool lin = g.am.n0 <= 0 && g.ak.n0 <= 0 && g.bk.n0 <= 0 && g.bn.n0 <= 0;
+  const bool ak = g.ak.s0 == 1, bc = g.bk.s0 == 1;
+  auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, 0, s, g, b); };
+  if (!lin) launch(gemm_f64_small_kernel<false, false, true>);
+  else if (ak && bc) launch(gemm_f64_small_kernel<true, true, false>);
+  else if (ak) launch(gemm_f64_small_kernel<true, false, false>);
+  else if (bc) launch(gemm_f64_small_kernel<false, true, false>);
+  else launch(gemm_f64_small_kernel<false, false, false>);
+}
+
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 // Shapes the pipelined kernel takes over: plainly strided as above (rows of even
@@ -732,7 +843,8 @@ void gemm_f64(const GemmDesc& g, const GemmBatch& b, double* work, size_t work_e
   const bool lin = g.am.n0 <= 0 && g.ak.n0 <= 0 && g.bk.n0 <= 0 && g.bn.n0 <= 0;
   auto launch_choice = [&](const TuneChoice& c) {
     hipEvent_t e0 = kernel_timing_begin(s);
-    if (c.wm == 2 && c.wn == 5 && lin && c.var == 1) launch_gemm_wide<2, 4, 16>(g, b, c.ks, work, s);
+    if (c.wn == 1) launch_small(g, b, s);
+    else if (c.wm == 2 && c.wn == 5 && lin && c.var == 1) launch_gemm_wide<2, 4, 16>(g, b, c.ks, work, s);
     else if (c.wm == 2 && c.wn == 5 && lin && c.var == 2) launch_gemm_wide<2, 2, 32>(g, b, c.ks, work, s);
     else if (c.wm == 2 && c.wn == 5 && lin && c.var == 3) launch_gemm_wide<2, 4, 32>(g, b, c.ks, work, s);
     else if (c.wm == 1 && c.wn == 5 && lin && c.var == 3) launch_gemm_wide<1, 4, 32>(g, b, c.ks, work, s);
@@ -753,7 +865,9 @@ void gemm_f64(const GemmDesc& g, const GemmBatch& b, double* work, size_t work_e
   };
   const TuneKey key{0, g.M, g.N, g.K, (lin ? 1 : 0) | (b.count << 1)};
   TuneChoice listed;
-  const bool in_table = autotune_lookup(key, &listed) && fits(listed.ks) && (listed.var == 0 || lin);
+  const bool small = small_shape(g, b.count);
+  const bool in_table = autotune_lookup(key, &listed) && fits(listed.ks) &&
+                        (listed.var == 0 || lin) && (small || listed.wn != 1);
   if (!in_table && pipe_shape(g, b.count) && aligned16(b.A[0]) && aligned16(b.B[0])) {
     const int ks = pipe_ksplit(g);
     if (ks == 1 || (work != nullptr && work_elems >= (size_t)ks * g.M * g.N)) {
@@ -782,6 +896,7 @@ void gemm_f64(const GemmDesc& g, const GemmBatch& b, double* work, size_t work_e
   }
   if (autotune_should_tune(key, g, s)) {
     std::vector<TuneChoice> cands;
+    if (small) cands.push_back(TuneChoice{1, 1, 1});
     const Tile tiles[8] = {{1, 5},    {2, 5},    {2, 2},    {4, 4},
                            {2, 5, 1}, {2, 5, 2}, {2, 5, 3}, {1, 5, 3}};
     for (const Tile& t : tiles) {
@@ -806,6 +921,7 @@ void gemm_f64(const GemmDesc& g, const GemmBatch& b, double* work, size_t work_e
   if (!fits(ks)) ks = 1;
   const Tile t = choose_tile(g);
   TuneChoice ch{t.wm, t.wn, ks};
+  if (small) ch = TuneChoice{1, 1, 1};
   if (in_table) ch = listed;
   launch_choice(ch);
 }

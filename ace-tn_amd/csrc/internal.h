@@ -85,8 +85,9 @@ struct GemmDesc {
   const int* run_if = nullptr;  // device flag: when given and zero the product is skipped
   bool c_f32 = false;           // split-bf16 products only: C holds FP32 (the pointer is a float*)
   bool a_f32 = false;           // split-bf16 products on the plane path only: A holds FP32
-  bool pipe = false;            // FP64 products: the pipelined kernel may be used, which sums in
-                                // another order (set outside mixed precision, see chol_rinv)
+  bool pipe = false;            // FP64 products: the pipelined and the small kernel may be used,
+                                // which sum in another order (set outside mixed precision, see
+                                // chol_rinv, and outside the full-rank projectors)
   int8_t planar = -1;           // split-bf16 products: 1 / 0 forces the plane / general path,
                                 // -1 picks by size (gemm_split_is_planar)
 };

@@ -184,3 +184,20 @@ def test_small_svd_spectra(hip, n, scale, case):
     assert np.abs(a1 @ a2.T - M / s[0]).max() <= tol
     for a, W in ((a1, U), (a2, V)):
         assert np.abs(a.T @ a - np.diag(s / s[0])).max() <= tol
+
+
+@pytest.mark.parametrize("ta,tb", [(False, False), (True, False), (False, True), (True, True)])
+@pytest.mark.parametrize("K", [1, 15, 16, 17, 63, 64, 65, 315, 1023, 1025, 3071, 3072, 3073])
+def test_small_gemm_tile_edges(hip, K, ta, tb):
+    """The one-tile-a-workgroup FP64 product at the remainders of its tiles and
+    k blocks, every operand order, one to sixteen waves and the first K past
+    its range, against numpy: 2 eps K at most in units of the norms."""
+    g = np.random.default_rng(K)
+    for M, N in ((1, 1), (15, 17), (16, 16), (33, 66), (315, 37), (64, 129), (700, 5)):
+        A = g.standard_normal((K, M) if ta else (M, K))
+        B = g.standard_normal((N, K) if tb else (K, N))
+        C = hip.gemm(torch.as_tensor(A, device="cuda"), torch.as_tensor(B, device="cuda"),
+                     ta=ta, tb=tb).cpu().numpy()
+        a, b = (A.T if ta else A), (B.T if tb else B)
+        scale = np.linalg.norm(a, axis=1)[:, None] * np.linalg.norm(b, axis=0)
+        assert np.all(np.abs(C - a @ b) <= 4.4e-16 * (K + 1) * scale), (M, N, K)
