@@ -711,7 +711,7 @@ __device__ __forceinline__ void round_pair(int n, int r, int a, int& p, int& qq)
 __device__ __forceinline__ void jacobi_rotation(double app, double aqq, double apq, double& c,
                                                 double& s) {
   const double d = aqq - app;
-  const double h = sqrt(d * d + 4.0 * apq * apq);
+  const double h = sqrt(fma(d, d, 4.0 * apq * apq));  // the same bits wherever it is inlined
   double t;
   if (h > 0.0 && isfinite(h)) {
     t = (d >= 0.0 ? 2.0 * apq : -2.0 * apq) / (fabs(d) + h);
@@ -984,6 +984,115 @@ __device__ __forceinline__ int bj_global(int li, int I, int J) {
   return li < 8 ? 8 * I + li : 8 * J + li - 8;
 }
 
+// The 8 inner rounds of cross pairs of one block pair (I, J), one wave, with
+// the subproblem in registers: lane 8 a + b holds the 2 x 2 block of the pairs
+// a and b (p = a, q = 8 + (a + round) mod 8), both triangles, so that a round
+// ends with three lane exchanges instead of a walk through LDS by indexes (the
+// rounds are bound by instruction issue, ten waves on one CU; q = 150: BJ_NEW
+// us a solve against 1125).  Lanes below the diagonal mirror the arithmetic of
+// those above it, operand by operand, and so hold the same bits.
+__device__ __forceinline__ double bj_pull(double x, int from4) {
+  return __hiloint2double(__builtin_amdgcn_ds_bpermute(from4, __double2hiint(x)),
+                          __builtin_amdgcn_ds_bpermute(from4, __double2loint(x)));
+}
+__device__ __forceinline__ void bj_cross_rounds(double* S, double* V, double* cs, int* rot_out,
+                                                int q, int N, int r, int pair, int lane, double tol,
+                                                double* out, double* flag_out) {
+  int I, J;
+  round_pair(N, r, pair, I, J);
+  const int a = lane >> 3, b = lane & 7;
+  double A = S[bj_addr(8 * I + a, 8 * I + b)], B = S[bj_addr(8 * I + a, 8 * J + b)];
+  double C = S[bj_addr(8 * I + b, 8 * J + a)], D = S[bj_addr(8 * J + a, 8 * J + b)];
+  const double da = S[bj_addr(8 * I + a, 8 * I + a)], db = S[bj_addr(8 * J + b, 8 * J + b)];
+  // V_a: row vr, columns vk, vk + 1 and those of their partners
+  const int vr = lane >> 2, vk = 2 * (lane & 3);
+  double v0p = vr == vk ? 1.0 : 0.0, v1p = vr == vk + 1 ? 1.0 : 0.0;
+  double v0q = vr == vk + 8 ? 1.0 : 0.0, v1q = vr == vk + 9 ? 1.0 : 0.0;
+  // no cross pair over the threshold: no rotation, V_a stays the identity
+  const bool rotate = __any(B != 0.0 && B * B > tol * tol * fabs(da * db));
+  if (rotate) {
+    // local indices >= nI (block I) or >= nJ (block J) are padding
+    const int nI = min(8, max(0, q - 8 * I)), nJ = min(8, max(0, q - 8 * J));
+    const int lo = min(a, b), hi = max(a, b);
+    const bool upper = a < b;
+    const int fromB = 4 * ((lane & 56) | ((b + 1) & 7)), fromC = 4 * ((lane + 8) & 63);
+    const int fromD = 4 * (8 * ((a + 1) & 7) + ((b + 1) & 7));
+#pragma unroll 1
+    for (int rr = 0; rr < 8; ++rr) {
+      double c = 1.0, s = 0.0;
+      if (a == b) {
+        const bool live = a < nI && ((a + rr) & 7) < nJ;
+        if (live && B != 0.0 && B * B > tol * tol * fabs(A * D)) jacobi_rotation(A, D, B, c, s);
+        cs[2 * a] = c;
+        cs[2 * a + 1] = s;
+      }
+      if (__any(s != 0.0)) {
+        rep_wave_sync();
+        const double ca = cs[2 * lo], sa = cs[2 * lo + 1], cb = cs[2 * hi], sb = cs[2 * hi + 1];
+        const double c0 = cs[2 * vk], s0 = cs[2 * vk + 1], c1 = cs[2 * vk + 2], s1 = cs[2 * vk + 3];
+        if (a == b) {
+          if (s != 0.0) {
+            const double t = s / c;
+            A = A - t * B;
+            D = D + t * B;
+            B = 0.0;
+            C = 0.0;
+          }
+        } else if (sa != 0.0 || sb != 0.0) {
+          // (fma and product as in the round of all pairs)
+          const double x11 = A, x12 = upper ? B : C, x21 = upper ? C : B, x22 = D;
+          const double y11 = fma(x11, cb, -(x12 * sb)), y12 = fma(x11, sb, x12 * cb);
+          const double y21 = fma(x21, cb, -(x22 * sb)), y22 = fma(x21, sb, x22 * cb);
+          A = fma(ca, y11, -(sa * y21));
+          const double z12 = fma(ca, y12, -(sa * y22)), z21 = fma(sa, y11, ca * y21);
+          D = fma(sa, y12, ca * y22);
+          B = upper ? z12 : z21;
+          C = upper ? z21 : z12;
+        }
+        if (s0 != 0.0) {
+          const double x = fma(c0, v0p, -(s0 * v0q));
+          v0q = fma(s0, v0p, c0 * v0q);
+          v0p = x;
+        }
+        if (s1 != 0.0) {
+          const double x = fma(c1, v1p, -(s1 * v1q));
+          v1q = fma(s1, v1p, c1 * v1q);
+          v1p = x;
+        }
+      }
+      // the partners move on by one
+      B = bj_pull(B, fromB);
+      C = bj_pull(C, fromC);
+      D = bj_pull(D, fromD);
+      const double next = dpp_mov<0x39>(v0q);  // the next lane of the four
+      v0q = v1q;
+      v1q = next;
+      rep_wave_sync();
+    }
+    int l = lane;
+    asm volatile("" : "+v"(l));  // the addresses are made again
+    const int ga = bj_global(l >> 3, I, J), gb = bj_global(l & 7, I, J);
+    const int ha = bj_global(8 + (l >> 3), I, J), hb = bj_global(8 + (l & 7), I, J);
+    if (a <= b) {
+      S[bj_addr(ga, gb)] = A;
+      S[bj_addr(ha, hb)] = D;
+    }
+    S[bj_addr(ga, hb)] = B;
+    out[vr * 16 + vk] = v0p;
+    out[vr * 16 + vk + 1] = v1p;
+    out[vr * 16 + vk + 8] = v0q;
+    out[vr * 16 + vk + 9] = v1q;
+  }
+  V[vr * BJ_LD + vk] = v0p;
+  V[vr * BJ_LD + vk + 1] = v1p;
+  V[vr * BJ_LD + vk + 8] = v0q;
+  V[vr * BJ_LD + vk + 9] = v1q;
+  if (lane == 0) {
+    *rot_out = rotate ? 1 : 0;
+    *flag_out = rotate ? 1.0 : 0.0;
+  }
+}
+
 __global__ __launch_bounds__(BJE_NT) void jacobi_blk_kernel(const double* __restrict__ Gin, int q,
                                                            double* __restrict__ w,
                                                            double* __restrict__ vrec, int* info,
@@ -1037,7 +1146,13 @@ __global__ __launch_bounds__(BJE_NT) void jacobi_blk_kernel(const double* __rest
     for (int r = 0; r < N - 1; ++r) {
       // ---- phase 1: wave a rotates the subproblem of block pair a ----
       // (on a dense symmetric copy W, element (x, y) at min * BJ_LD + max)
-      if (wave < NP) {
+      if (wave < NP && r > 0) {
+        int l = lane;
+        asm volatile("" : "+v"(l));  // what hangs on it is made again, not held (registers)
+        bj_cross_rounds(S, Vs[wave], &csw[wave][0][0], &rotw[wave], q, N, r, wave, l, tol,
+                        vrec + ((int64_t)(sweep * (N - 1) + r) * NP + wave) * 256,
+                        vflag + (int64_t)(sweep * (N - 1) + r) * NP + wave);
+      } else if (wave < NP) {
         int I, J;
         round_pair(N, r, wave, I, J);
         double* V = Vs[wave];
@@ -1050,26 +1165,24 @@ __global__ __launch_bounds__(BJE_NT) void jacobi_blk_kernel(const double* __rest
         // local indices >= nI (block I) or >= 8 + nJ (block J) are padding
         const int nI = min(8, max(0, q - 8 * I)), nJ = min(8, max(0, q - 8 * J));
         rep_wave_sync();
-        // Does any pair the inner rounds visit (all pairs in the first block
-        // round of a sweep, the cross pairs otherwise) pass the threshold?  If
-        // none does, no rotation happens (W only changes by rotations), so
-        // the rounds are skipped and V_a stays the identity.
+        // Does any pair pass the threshold?  If none does, no rotation happens
+        // (W only changes by rotations), so the rounds are skipped and V_a
+        // stays the identity.
         bool want = false;
         for (int e = lane; e < 256; e += 64) {
           const int x = e >> 4, y = e & 15;
-          if (x < y && (r == 0 || (x < 8 && y >= 8))) {
+          if (x < y) {
             const double apq = W[x * BJ_LD + y];
             want |= apq != 0.0 &&
                     apq * apq > tol * tol * fabs(W[x * (BJ_LD + 1)] * W[y * (BJ_LD + 1)]);
           }
         }
         const bool rotate = __any(want);
-        const int inner = !rotate ? 0 : (r == 0) ? 15 : 8;
+        const int inner = rotate ? 15 : 0;
         for (int rr = 0; rr < inner; ++rr) {
           if (lane < 8) {
             int p, qq;
-            if (r == 0) round_pair(16, rr, lane, p, qq);
-            else { p = lane; qq = 8 + ((lane + rr) & 7); }
+            round_pair(16, rr, lane, p, qq);
             double c = 1.0, sn = 0.0;
             const bool live = (p < 8 ? p < nI : p - 8 < nJ) && (qq < 8 ? qq < nI : qq - 8 < nJ);
             if (live) {
