@@ -600,40 +600,105 @@ struct AlsShared {
   double* S;     // nR x d
   double* a1;    // nD x D x d
   double* a2;
-  double* T;     // nD x nD x D x d (one outer index of the R build)
+  double* T;     // nD x nD x D x d for each of grp outer indices of the R build
   double* n12g;  // nD^2 d^2
   double* a12n;  // nD^2 d^2
   double* red;   // ALS_NT/64
 };
 
-// N(a, b, A, B): side 0 -> n12[a][b][A][B], side 1 -> n12[b][a][B][A]
-__device__ __forceinline__ int64_t nidx(int side, int nD, int a, int b, int A, int B) {
-  return side == 0 ? (((int64_t)a * nD + b) * nD + A) * nD + B
-                   : (((int64_t)b * nD + a) * nD + B) * nD + A;
+typedef double als_d4 __attribute__((ext_vector_type(4)));
+
+// na = N x for x[(y,x)][pq] in LDS (nD^2 x d^2): 16 x 16 tiles on the matrix
+// cores, a row tile a wave at a time; take(e, value) gets element e of na.
+template <class F>
+__device__ __forceinline__ void als_apply_norm(const double* __restrict__ n12,
+                                               const double* __restrict__ x, int nD, int d2,
+                                               F&& take) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, m = lane & 15, kq = lane >> 4;
+  const int n2 = nD * nD, mt = (n2 + 15) / 16, nt = (d2 + 15) / 16;
+  for (int t = wave; t < mt * nt; t += ALS_NT / 64) {
+    const int row = t % mt * 16, cl = t / mt * 16 + m, cc = min(cl, d2 - 1);
+    const double* pa = n12 + min(row + m, n2 - 1);
+    als_d4 acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 8
+    for (int k0 = 0; k0 < n2; k0 += 4) {
+      const int k = min(k0 + kq, n2 - 1);
+      const double av = pa[(int64_t)k * n2], bv = x[k * d2 + cc];
+      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(k0 + kq < n2 ? av : 0.0, bv, acc, 0, 0, 0);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int i = row + kq + 4 * r;
+      if (i < n2 && cl < d2) take(i * d2 + cl, acc[r]);
+    }
+  }
 }
 
-// Build R and S for the tensor of side ``side`` from ``other`` (the fixed one).
+// Build R and S for the tensor of side ``side`` from ``other`` (the fixed one),
+// ``grp`` outer indices a at a time (as many as T holds).  Both contractions run
+// on the matrix cores, operands straight from memory and LDS: on 256 threads'
+// vector units every product cost a load of its own (nD = 12, the whole call of a
+// D=6 bond: 1530 -> 675 us).
 __device__ void als_build(const AlsShared& sh, const double* __restrict__ n12, int side, int nD,
-                          int D, int d, const double* other) {
-  const int tid = threadIdx.x;
-  const int nR = nD * D, Dd = D * d;
-  for (int a = 0; a < nD; ++a) {
-    // T[A][B][u][Q] = sum_b N(a,b,A,B) other[b][u][Q]
-    for (int e = tid; e < nD * nD * Dd; e += ALS_NT) {
-      const int A = e / (nD * Dd), r = e % (nD * Dd), B = r / Dd, uQ = r % Dd;
-      double acc = 0.0;
-      for (int b = 0; b < nD; ++b) acc += n12[nidx(side, nD, a, b, A, B)] * other[b * Dd + uQ];
-      sh.T[e] = acc;
+                          int D, int d, int grp, const double* other) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, m = lane & 15, kq = lane >> 4;
+  const int nR = nD * D, Dd = D * d, n2 = nD * nD;
+  const int mt = (n2 + 15) / 16, nt = (Dd + 15) / 16;
+  for (int a0 = 0; a0 < nD; a0 += grp) {
+    const int ga = min(grp, nD - a0);
+    // T[a][A][B][uQ] = sum_b N(a,b,A,B) other[b][uQ]; N is contiguous in (A, B)
+    // on side 0, in (B, A) on side 1
+    for (int t0 = wave * 2; t0 < ga * mt * nt; t0 += ALS_NT / 32) {
+      als_d4 acc[2];
+      const double *pa[2], *pb[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int t = min(t0 + h, ga * mt * nt - 1), g = t / (mt * nt), row = t % mt * 16;
+        acc[h] = als_d4{0.0, 0.0, 0.0, 0.0};
+        pa[h] = n12 + (int64_t)(side == 0 ? (a0 + g) * nD : a0 + g) * n2 + min(row + m, n2 - 1);
+        pb[h] = other + min(t / mt % nt * 16 + m, Dd - 1);
+      }
+      const int64_t sb = side == 0 ? n2 : (int64_t)nD * n2;  // from b to b + 1
+#pragma unroll 3
+      for (int k0 = 0; k0 < nD; k0 += 4) {
+        const int k = min(k0 + kq, nD - 1);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const double av = pa[h][k * sb], bv = pb[h][k * Dd];
+          acc[h] = __builtin_amdgcn_mfma_f64_16x16x4f64(k0 + kq < nD ? av : 0.0, bv, acc[h], 0, 0, 0);
+        }
+      }
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int t = t0 + h, g = t / (mt * nt), row = t % mt * 16, cl = t / mt % nt * 16 + m;
+        if (t >= ga * mt * nt || cl >= Dd) continue;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int i = row + kq + 4 * r;
+          const int ab = side == 0 ? i : i % nD * nD + i / nD;
+          if (i < n2) sh.T[((int64_t)g * n2 + ab) * Dd + cl] = acc[h][r];
+        }
+      }
     }
     __syncthreads();
-    // R[(A,U),(a,u)] = sum_{B,Q} T[A][B][u][Q] other[B][U][Q]
-    for (int e = tid; e < nD * D * D; e += ALS_NT) {
-      const int A = e / (D * D), U = (e / D) % D, u = e % D;
-      double acc = 0.0;
-      for (int B = 0; B < nD; ++B)
-        for (int Q = 0; Q < d; ++Q)
-          acc += sh.T[((A * nD + B) * D + u) * d + Q] * other[(B * D + U) * d + Q];
-      sh.R[(int64_t)(A * D + U) * nR + a * D + u] = acc;
+    // R[(A,U),(a,u)] = sum_{B,Q} T[a][A][B][u][Q] other[B][U][Q], rows (A, u), columns U
+    const int rt = (nR + 15) / 16, ut = (D + 15) / 16, K = nD * d;
+    for (int t = wave; t < ga * rt * ut; t += ALS_NT / 64) {
+      const int g = t / (rt * ut), row = t % rt * 16, cl = t / rt % ut * 16 + m;
+      const int i = min(row + m, nR - 1), U = min(cl, D - 1);
+      const double* pt = sh.T + (int64_t)g * n2 * Dd + i / D * nD * Dd + i % D * d;
+      als_d4 acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 2
+      for (int k0 = 0; k0 < K; k0 += 4) {
+        const int k = min(k0 + kq, K - 1), B = k / d, Q = k - B * d;
+        const double av = pt[B * Dd + Q], bv = other[(B * D + U) * d + Q];
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(k0 + kq < K ? av : 0.0, bv, acc, 0, 0, 0);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int x = row + kq + 4 * r, A = x / D, u = x % D;
+        if (x < nR && cl < D) sh.R[(int64_t)(A * D + cl) * nR + (a0 + g) * D + u] = acc[r];
+      }
     }
     __syncthreads();
   }
@@ -670,9 +735,6 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Solve (sym(R) + eps max|R| I) X = S in place (X -> S), wave 0 doing the
-// factorisation.  Returns (block-uniform) 1 if the Cholesky factorisation
-// failed and partial-pivoting elimination was used, 2 if that found R singular.
 // ALS system through the pseudo-inverse (als_solver.py:228-230:
 // pinv(R, hermitian=True, rcond=eps) @ S): R <- (R + R^T)/2 (no shift),
 // R = V diag(lam) V^T by cyclic two-sided Jacobi with round-robin parallel
@@ -776,81 +838,143 @@ __device__ void als_pinv_solve(const AlsShared& sh, int nR, int d, double eps,
   __syncthreads();
 }
 
-__device__ int als_solve_system(const AlsShared& sh, int nR, int d, double eps,
-                                double* __restrict__ Rsave, int* flag) {
-  const int tid = threadIdx.x, lane = tid & 63;
+// The elimination behind als_solve_system with the lower triangle in registers:
+// thread (ti, tj) of 16 x 16 holds rows ti + 16 r and columns tj + 16 c, r >= c
+// < RC.  A step publishes its column and its row of S (one barrier, two buffers
+// in turn) and every thread subtracts the products of the column with itself
+// over the pivot from its part, right-hand sides included; columns stay
+// unscaled (L D).  On return R's lower triangle holds L D, dinv 1 / D and S the
+// forward-substituted right-hand sides.  False if a pivot was not positive: S
+// and R's upper triangle are then untouched.
+template <int RC>
+__device__ bool als_eliminate(double* R, double* S, int nR, int d, double shift,
+                              double* __restrict__ pub, double* dinv) {
+  constexpr int PB = 16 * RC + 8;  // a published column and the row of S
+  const int tid = threadIdx.x, ti = tid >> 4, tj = tid & 15;
+  double a[RC][RC], s[RC];
+#pragma unroll
+  for (int r = 0; r < RC; ++r) {
+    const int i = ti + 16 * r;
+#pragma unroll
+    for (int c = 0; c <= r; ++c) {
+      const int k = tj + 16 * c;
+      const double v = (i < nR && k < nR && k <= i) ? R[k * nR + i] : 0.0;
+      a[r][c] = i == k ? v + shift : v;
+    }
+    s[r] = (i < nR && tj < d) ? S[i * d + tj] : 0.0;
+  }
+#pragma unroll
+  for (int cj = 0; cj < RC; ++cj) {
+#pragma unroll 1
+    for (int jj = 0; jj < 16; ++jj) {
+      const int j = 16 * cj + jj;
+      if (j >= nR) break;
+      double* col = pub + (j & 1) * PB;
+      if (tj == jj) {
+#pragma unroll
+        for (int r = cj; r < RC; ++r) {
+          const int i = ti + 16 * r;
+          col[i] = a[r][cj];
+          if (i >= j && i < nR) R[i * nR + j] = a[r][cj];
+        }
+      }
+      if (ti == jj && tj < d) col[16 * RC + tj] = s[cj];
+      __syncthreads();
+      const double piv = col[j];
+      if (!(piv > 0.0)) return false;
+      const double inv = 1.0 / piv;
+      if (tid == 0) dinv[j] = inv;
+      double ck[RC];
+#pragma unroll
+      for (int c = cj; c < RC; ++c) ck[c] = tj + 16 * c > j ? col[tj + 16 * c] * inv : 0.0;
+      const double sk = tj < d ? col[16 * RC + tj] * inv : 0.0;
+#pragma unroll
+      for (int r = cj; r < RC; ++r) {
+        const double x = ti + 16 * r > j ? col[ti + 16 * r] : 0.0;
+#pragma unroll
+        for (int c = cj; c <= r; ++c) a[r][c] = fma(-x, ck[c], a[r][c]);
+        s[r] = fma(-x, sk, s[r]);
+      }
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < RC; ++r) {
+    const int i = ti + 16 * r;
+    if (i < nR && tj < d) S[i * d + tj] = s[r];
+  }
+  __syncthreads();
+  return true;
+}
+
+// Solve (sym(R) + eps max|R| I) X = S in place (X -> S).  Returns (block-
+// uniform) 0, 1 if a pivot was not positive and partial-pivoting elimination was
+// used, 2 if that found R singular.  The factorisation was one wave's walk
+// through LDS and most of a sweep; on all 256 threads it is bound by the step's
+// round trip (nR = 72, the whole call of a D=6 bond: 2440 -> 1530 us).
+constexpr int kAlsMaxTiles = 9;  // nR <= 144 (LDS holds less)
+__device__ int als_solve_system(const AlsShared& sh, int nR, int d, double eps, int* flag) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  __shared__ double pub[2 * (16 * kAlsMaxTiles + 8)], dinv[16 * kAlsMaxTiles];
   double* R = sh.R;
   double* S = sh.S;
-  // symmetrise and regularise
+  // the symmetric part goes to the upper triangle
+  double mx = 0.0;
   for (int e = tid; e < nR * nR; e += ALS_NT) {
     const int i = e / nR, j = e % nR;
-    if (i < j) {
+    if (i <= j) {
       const double v = 0.5 * (R[i * nR + j] + R[j * nR + i]);
       R[i * nR + j] = v;
-      R[j * nR + i] = v;
+      mx = fmax(mx, fabs(v));
     }
   }
-  __syncthreads();
-  double mx = 0.0;
-  for (int e = tid; e < nR * nR; e += ALS_NT) mx = fmax(mx, fabs(R[e]));
   mx = block_max(mx, sh.red);
-  for (int i = tid; i < nR; i += ALS_NT) R[i * nR + i] += eps * mx;
-  __syncthreads();
-  for (int e = tid; e < nR * nR; e += ALS_NT) Rsave[e] = R[e];
-  for (int e = tid; e < nR * d; e += ALS_NT) Rsave[nR * nR + e] = S[e];
+  const double shift = eps * mx;
+  // the lower triangle takes the factor, the diagonal with it
+  double diag = tid < nR ? R[tid * nR + tid] + shift : 0.0;
   if (tid == 0) *flag = 0;
   __syncthreads();
-  if (tid < 64) {
-    // Cholesky R = L L^T (lower, in place)
-    int fail = 0;
-    for (int j = 0; j < nR && !fail; ++j) {
-      const double piv = R[j * nR + j];
-      if (!(piv > 0.0)) { fail = 1; break; }
-      const double ljj = sqrt(piv);
-      wave_sync();
-      if (lane == 0) R[j * nR + j] = ljj;
-      for (int i = j + 1 + lane; i < nR; i += 64) R[i * nR + j] /= ljj;
-      wave_sync();
-      for (int i = j + 1 + lane; i < nR; i += 64) {
-        const double lij = R[i * nR + j];
-        for (int k = j + 1; k <= i; ++k) R[i * nR + k] -= lij * R[k * nR + j];
+  bool ok;
+  if (nR <= 48) ok = als_eliminate<3>(R, S, nR, d, shift, pub, dinv);
+  else if (nR <= 80) ok = als_eliminate<5>(R, S, nR, d, shift, pub, dinv);
+  else ok = als_eliminate<kAlsMaxTiles>(R, S, nR, d, shift, pub, dinv);
+  if (ok) {
+    // D L^T x = S, a right-hand side a wave: lane l holds rows l, l + 64, l + 128
+    for (int c = wave; c < d; c += ALS_NT / 64) {
+      double x[3], w[3];
+#pragma unroll
+      for (int t = 0; t < 3; ++t) {
+        const int i = lane + 64 * t;
+        x[t] = i < nR ? S[i * d + c] : 0.0;
+        w[t] = i < nR ? dinv[i] : 0.0;
       }
-      wave_sync();
-    }
-    if (!fail) {
-      // forward: L y = S ; backward: L^T x = y   (all right-hand sides)
-      for (int k = 0; k < nR; ++k) {
-        const double lkk = R[k * nR + k];
-        wave_sync();
-        if (lane < d) S[k * d + lane] /= lkk;
-        wave_sync();
-        for (int i = k + 1 + lane; i < nR; i += 64) {
-          const double lik = R[i * nR + k];
-          for (int c = 0; c < d; ++c) S[i * d + c] -= lik * S[k * d + c];
+#pragma unroll
+      for (int t = 2; t >= 0; --t) {
+#pragma unroll 4
+        for (int k = min(nR, 64 * t + 64) - 1; k >= 64 * t; --k) {
+          const double xk = lane_value(x[t] * w[t], k - 64 * t);
+#pragma unroll
+          for (int h = 0; h <= t; ++h) {
+            const int i = lane + 64 * h;
+            const double l = R[k * nR + min(i, k)];
+            x[h] = fma(-(i < k ? l : 0.0), xk, x[h]);
+          }
         }
-        wave_sync();
       }
-      for (int k = nR - 1; k >= 0; --k) {
-        const double lkk = R[k * nR + k];
-        wave_sync();
-        if (lane < d) S[k * d + lane] /= lkk;
-        wave_sync();
-        for (int i = lane; i < k; i += 64) {
-          const double lki = R[k * nR + i];
-          for (int c = 0; c < d; ++c) S[i * d + c] -= lki * S[k * d + c];
-        }
-        wave_sync();
-      }
-    } else if (lane == 0) {
-      *flag = 1;
+#pragma unroll
+      for (int t = 0; t < 3; ++t)
+        if (lane + 64 * t < nR) S[(lane + 64 * t) * d + c] = x[t] * w[t];
     }
+    __syncthreads();
+    return 0;
   }
+  // LU with partial pivoting on the regularised system
   __syncthreads();
-  int status = *flag;
-  if (status == 0) return 0;
-  // LU with partial pivoting on the saved (regularised) system
-  for (int e = tid; e < nR * nR; e += ALS_NT) R[e] = Rsave[e];
-  for (int e = tid; e < nR * d; e += ALS_NT) S[e] = Rsave[nR * nR + e];
+  for (int e = tid; e < nR * nR; e += ALS_NT) {
+    const int i = e / nR, j = e % nR;
+    if (i < j) R[j * nR + i] = R[i * nR + j];
+  }
+  if (tid < nR) R[tid * nR + tid] = diag;
+  if (tid == 0) *flag = 1;
   __syncthreads();
   if (tid < 64) {
     int singular = 0;
@@ -923,14 +1047,9 @@ __device__ double als_cost(const AlsShared& sh, const double* __restrict__ n12, 
   }
   __syncthreads();
   double part = 0.0;
-  for (int e = tid; e < nE; e += ALS_NT) {
-    const int Y = e / (nD * d2), X = (e / d2) % nD, pq = e % d2;
-    double na = 0.0;
-    for (int y = 0; y < nD; ++y)
-      for (int x = 0; x < nD; ++x)
-        na += n12[(((int64_t)y * nD + x) * nD + Y) * nD + X] * sh.a12n[(y * nD + x) * d2 + pq];
+  als_apply_norm(n12, sh.a12n, nD, d2, [&](int e, double na) {
     part += na * sh.a12n[e] - 2.0 * sh.n12g[e] * sh.a12n[e];
-  }
+  });
   return block_sum(part, sh.red);
 }
 
@@ -942,7 +1061,8 @@ __global__ __launch_bounds__(ALS_NT) void als_kernel(const double* __restrict__ 
                                                      int method, double* __restrict__ gwork,
                                                      double* __restrict__ out_cost,
                                                      int* __restrict__ out_info,
-                                                     int64_t n12_stride, int64_t gwork_stride) {
+                                                     int64_t n12_stride, int64_t gwork_stride,
+                                                     int grp) {
   // workgroup b solves problem b of a batch: n12 n12_stride doubles apart,
   // a12g nE apart, a1r/a2r nR*d apart, scratch gwork_stride apart, one cost
   // and two info words each
@@ -969,38 +1089,27 @@ __global__ __launch_bounds__(ALS_NT) void als_kernel(const double* __restrict__ 
   sh.a1 = sh.S + (size_t)nR * d;
   sh.a2 = sh.a1 + (size_t)nR * d;
   sh.T = sh.a2 + (size_t)nR * d;
-  sh.n12g = sh.T + (size_t)nD * nD * D * d;
+  sh.n12g = sh.T + (size_t)grp * nD * nD * D * d;
   sh.a12n = sh.n12g + nE;
   sh.red = sh.a12n + nE;
   for (int e = tid; e < nR * d; e += ALS_NT) { sh.a1[e] = a1r[e]; sh.a2[e] = a2r[e]; }
   // n12g[Y][X][p][q] = sum_{y,x} n12[y][x][Y][X] a12g[y][x][p][q]
-  for (int e = tid; e < nE; e += ALS_NT) {
-    const int Y = e / (nD * d2), X = (e / d2) % nD, pq = e % d2;
-    double acc = 0.0;
-    for (int y = 0; y < nD; ++y)
-      for (int x = 0; x < nD; ++x)
-        acc += n12[(((int64_t)y * nD + x) * nD + Y) * nD + X] * a12g[(y * nD + x) * d2 + pq];
-    sh.n12g[e] = acc;
-  }
+  als_apply_norm(n12, a12g, nD, d2, [&](int e, double v) { sh.n12g[e] = v; });
   __syncthreads();
   const double c0 = als_cost(sh, n12, nD, D, d);
   if (tid == 0) { s_d1 = fabs(c0); s_d2 = c0; s_stop = 0; }
   __syncthreads();
   int sweeps = 0, info = 0;
   for (int i = 0; i < niter; ++i) {
-    als_build(sh, n12, 0, nD, D, d, sh.a2);
-    int st = 0;
-    if (method == 1) als_pinv_solve(sh, nR, d, eps, gwork);
-    else st = als_solve_system(sh, nR, d, eps, gwork, &flag);
-    info |= st;
-    for (int e = tid; e < nR * d; e += ALS_NT) sh.a1[e] = sh.S[e];
-    __syncthreads();
-    als_build(sh, n12, 1, nD, D, d, sh.a1);
-    if (method == 1) als_pinv_solve(sh, nR, d, eps, gwork);
-    else st = als_solve_system(sh, nR, d, eps, gwork, &flag);
-    info |= st;
-    for (int e = tid; e < nR * d; e += ALS_NT) sh.a2[e] = sh.S[e];
-    __syncthreads();
+#pragma unroll 1
+    for (int side = 0; side < 2; ++side) {
+      double* own = side == 0 ? sh.a1 : sh.a2;
+      als_build(sh, n12, side, nD, D, d, grp, side == 0 ? sh.a2 : sh.a1);
+      if (method == 1) als_pinv_solve(sh, nR, d, eps, gwork);
+      else info |= als_solve_system(sh, nR, d, eps, &flag);
+      for (int e = tid; e < nR * d; e += ALS_NT) own[e] = sh.S[e];
+      __syncthreads();
+    }
     sweeps = i + 1;
     const double c = als_cost(sh, n12, nD, D, d);
     if (tid == 0) {
@@ -1172,7 +1281,10 @@ void als_solve_device(const double* n12, const double* a12g, double* a1r, double
                       double* out_cost, int* out_info, hipStream_t s, int method, int count) {
   ACETN_REQUIRE(count >= 1, "als: empty batch");
   als_check_shape(nD, D, d, method);
-  const size_t lds = als_lds_bytes(nD, D, d);
+  // one problem has the CU to itself: T takes what LDS is left
+  const size_t one = als_lds_bytes(nD, D, d), t1 = sizeof(double) * (size_t)nD * nD * D * d;
+  const int grp = count > 1 ? 1 : (int)std::min<size_t>(nD, 1 + (150 * 1024 - one) / t1);
+  const size_t lds = one + (grp - 1) * t1;
   static bool attr = false;
   if (!attr) {
     ACETN_HIP_CHECK(hipFuncSetAttribute((const void*)als_kernel,
@@ -1182,7 +1294,7 @@ void als_solve_device(const double* n12, const double* a12g, double* a1r, double
   const int64_t n12_stride = (int64_t)nD * nD * nD * nD;
   hipLaunchKernelGGL(als_kernel, dim3(count), dim3(ALS_NT), lds, s, n12, a12g, a1r, a2r, nD, D, d,
                      niter, tol, eps, method, gwork, out_cost, out_info, n12_stride,
-                     (int64_t)als_work_elems(nD, D, d));
+                     (int64_t)als_work_elems(nD, D, d), grp);
   ACETN_HIP_CHECK(hipGetLastError());
 }
 

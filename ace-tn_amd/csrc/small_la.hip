@@ -988,8 +988,8 @@ __device__ __forceinline__ int bj_global(int li, int I, int J) {
 // the subproblem in registers: lane 8 a + b holds the 2 x 2 block of the pairs
 // a and b (p = a, q = 8 + (a + round) mod 8), both triangles, so that a round
 // ends with three lane exchanges instead of a walk through LDS by indexes (the
-// rounds are bound by instruction issue, ten waves on one CU; q = 150: BJ_NEW
-// us a solve against 1125).  Lanes below the diagonal mirror the arithmetic of
+// rounds are bound by instruction issue, ten waves on one CU; q = 150: 2310
+// us a solve against 2820).  Lanes below the diagonal mirror the arithmetic of
 // those above it, operand by operand, and so hold the same bits.
 __device__ __forceinline__ double bj_pull(double x, int from4) {
   return __hiloint2double(__builtin_amdgcn_ds_bpermute(from4, __double2hiint(x)),

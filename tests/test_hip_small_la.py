@@ -201,3 +201,52 @@ def test_small_gemm_tile_edges(hip, K, ta, tb):
         a, b = (A.T if ta else A), (B.T if tb else B)
         scale = np.linalg.norm(a, axis=1)[:, None] * np.linalg.norm(b, axis=0)
         assert np.all(np.abs(C - a @ b) <= 4.4e-16 * (K + 1) * scale), (M, N, K)
+
+
+@pytest.mark.parametrize("sign", [1.0, -1.0])
+@pytest.mark.parametrize("nD,D,d", [(1, 1, 1), (2, 1, 2), (3, 2, 1), (4, 2, 2), (5, 3, 3), (8, 4, 2),
+                                    (9, 5, 1), (12, 4, 2), (7, 7, 1), (12, 6, 2), (10, 8, 1),
+                                    (9, 9, 2), (16, 7, 2), (22, 5, 1), (15, 8, 1)])
+def test_als_sweep_shapes(hip, nD, D, d, sign):
+    """One ALS sweep at the edges of its tiles and of the register factor's
+    three sizes (nD D up to 120), alone and in a batch, against numpy's solve.
+    The norm is Gaussian with four samples a row, so the systems' condition
+    stays near 10; a negative one takes the pivoted elimination.  2 nR^2
+    half-ulps times the condition of each system, both in turn."""
+    g = np.random.default_rng(100 * nD + 10 * D + d)
+    n2, nR = nD * nD, nD * D
+    M = g.standard_normal((n2, 4 * n2))
+    N = (M @ M.T / (4 * n2) * sign).reshape(nD, nD, nD, nD)
+    a12g = g.standard_normal((nD, nD, d, d))
+    a1, a2 = g.standard_normal((nD, D, d)), g.standard_normal((nD, D, d))
+    n12g = np.tensordot(N, a12g, ((0, 1), (0, 1)))                       # [Y, X, p, q]
+    tol = 0.0
+    for side in (0, 1):
+        n, x, G = (N, a2, n12g) if side == 0 else (
+            N.transpose(1, 0, 3, 2), a1, n12g.transpose(1, 0, 3, 2))
+        t = np.tensordot(n, x, ((1,), (0,)))                             # [a, A, B, u, Q]
+        R = np.tensordot(t, x, ((2, 4), (0, 2)))                         # [a, A, u, U]
+        R = R.transpose(1, 3, 0, 2).reshape(nR, nR)
+        S = np.tensordot(G, x, ((1, 3), (0, 2))).transpose(0, 2, 1).reshape(nR, d)
+        R = 0.5 * (R + R.T)
+        R = R + 1e-12 * np.abs(R).max() * np.eye(nR)
+        X = np.linalg.solve(R, S).reshape(nD, D, d)
+        tol += 2 * nR ** 2 * 2.0 ** -53 * np.linalg.cond(R)
+        if side == 0:
+            a1n, a1 = X, X
+        else:
+            a2n = X
+    dv = lambda t: torch.as_tensor(t, device="cuda")
+    start = g.standard_normal((nD, D, d))  # the first tensor's start does not enter
+    h1, h2, _, _, flags = hip.als_solve(dv(N), dv(a12g), dv(start), dv(a2), 1, 1e-15, "cholesky",
+                                        1e-12)
+    assert flags == (0 if sign > 0 else 1)
+    assert np.abs(h1.cpu().numpy() - a1n).max() <= tol * np.abs(a1n).max()
+    assert np.abs(h2.cpu().numpy() - a2n).max() <= tol * np.abs(a2n).max()
+    b1, b2, _, _, bf = hip.als_solve_batch(dv(N)[None].repeat(2, 1, 1, 1, 1),
+                                           dv(a12g)[None].repeat(2, 1, 1, 1, 1), D, 1, 1e-15,
+                                           "cholesky", 1e-12,
+                                           (dv(start)[None].repeat(2, 1, 1, 1),
+                                            dv(a2)[None].repeat(2, 1, 1, 1)))
+    for i in (0, 1):
+        assert torch.equal(b1[i], h1) and torch.equal(b2[i], h2) and int(bf[i]) == flags
