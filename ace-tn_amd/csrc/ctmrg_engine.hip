@@ -919,15 +919,6 @@ void site_rdm(Ctx& c, const acetn_site* s, double* rho) {
   const int64_t N1 = c4 * D2, Ne = e3 * D2;
   double* t1b = c.take((size_t)N1 * Ne);
   corner_edge(c, t1a, N1, s->E[2], e3, a0, D2, t1b);
-  // t1c[c][l][e][d][U][R][P] = sum_{L,D} t1b[c][l][L][e][d][D] abar[L][U][R][D][P]
-  const int64_t Mc = c4 * D * e3 * D, Nc = D2 * d;
-  double* t1c = c.take((size_t)Mc * Nc);
-  gemm(c, gdesc((int)Mc, (int)Nc, (int)D2,
-                grouped4((int)D, D, (int)e3, D2, (int)D, D * Ne, D2 * Ne),  // m = (c,l,e,d)
-                grouped((int)D, 1, Ne),                                   // k = (L,D)
-                grouped((int)D, d, D * D2 * d),                           // A: D -> d, L -> D^3 d
-                grouped3((int)d, 1, (int)D, D * d, D2 * d),               // n = (U,R,P)
-                plain(Nc), plain(1)), t1b, s->A, t1c);
   // t2[a][c][u][U] = c1 . e1
   const int64_t a1 = s->C_dim[0][0], b1 = s->C_dim[0][1];
   ACETN_REQUIRE(s->E_dim[0][0] == b1, "site rdm: c1/e1 mismatch");
@@ -952,17 +943,15 @@ void site_rdm(Ctx& c, const acetn_site* s, double* rho) {
   const int64_t Mb = b3 * D2, Na = a1 * D2;
   double* t3c = c.take((size_t)Mb * Na);
   corner_edge(c, t3b, Mb, t2, a1, e2, D2, t3c);
-  // t4[r][u][l][d][P] = sum_{e,R,c,U} t3c[e][r][R][c][u][U] t1c[c][l][e][d][U][R][P]
+  // t4[r][u][l][d][P] = sum_{e,R,c,U} t3c[e][r][R][c][u][U]
+  //                     sum_{L,D} t1b[c][l][L][e][d][D] abar[L][U][R][D][P]
   //   (t3c's leading index b plays e, its a plays c)
   ACETN_REQUIRE(b3 == e3 && a1 == c4, "site rdm: ring dimension mismatch");
-  const int64_t ne = b3, nc = a1, Kt = ne * D * nc * D;
+  const int64_t ne = b3, nc = a1;
   double* t4 = c.take((size_t)D2 * D2 * d);
-  gemm(c, gdesc((int)D2, (int)(D2 * d), (int)Kt,
-                grouped((int)D, D, D * nc * D2),                               // m = (r,u)
-                grouped4((int)D, 1, (int)nc, D2, (int)D, nc * D2, D2 * nc * D2),  // k = (e,R,c,U)
-                grouped4((int)D, D * d, (int)nc, D * e3 * D * D2 * d, (int)D, d, D * D2 * d),
-                grouped3((int)d, 1, (int)D, D2 * d, e3 * D * D2 * d),           // n = (l,d,P)
-                plain(D2 * d), plain(1)), t3c, t1c, t4);
+  double* part = c.take(ring_close_work_elems((int)D, (int)d, (int)ne, (int)nc));
+  if (c.launch)
+    ring_close(t1b, t3c, s->A, (int)D, (int)d, (int)ne, (int)nc, part, t4, c.st);
   // rho[P][p] = sum_{r,u,l,d} t4[(r,u,l,d)][P] a[l][u][r][d][p]
   gemm(c, gdesc((int)d, (int)d, (int)(D2 * D2), plain(1), plain(d),
                 grouped4((int)D, d, (int)D, D * D2 * d, (int)D, D2 * d, D * d),

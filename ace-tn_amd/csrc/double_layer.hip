@@ -290,4 +290,149 @@ void double_layer_f32(const DLDesc& g, const double* X, const double* A, double*
   double_layer_t<float>(g, X, A, Y, s);
 }
 
+// ---------------------------------------------------------------------------
+// The closing contraction of a one-site network,
+//
+//   Y[r,u; l,b,p] = sum_{e,R,c,U} T3[e; r,R; c; u,U] sum_{L,B} T1[c; l,L; e; b,B]
+//                                 * conj(A)[L,U,R,B,p]
+//
+// (T1 c4.e4.e3, T3 the other three sides).  Block (c, e) of the boundary gives
+// two D^2 x D^2 x D^2 products per p, Z = A_p^T T1 and Y_p += T3 Z, chained in
+// registers: an element r of the 16 x 16 result tile tm of Z is the operand of
+// k step 4 tm + r.  Wave (p, tn) of a workgroup keeps column tile tn of Y_p over
+// all its blocks; the workgroups' sums are added in a fixed order.  As two
+// products over memory, with the chi^2 D^4 d intermediate between them, D=5,
+// chi=100 took 470 us; so 55 us, bound by the loads of the two tensors
+// (100 MB, 48 - 200 bytes at a stretch).
+// ---------------------------------------------------------------------------
+namespace {
+constexpr int kRingWGs = 512;
+constexpr int kRingP = 2;  // physical indices a launch: 8 waves at most, 256 registers
+
+template <int D>
+__global__ __launch_bounds__(64 * kRingP * ((D * D + 15) / 16)) void ring_close_kernel(
+    const double* __restrict__ T1, const double* __restrict__ T3, const double* __restrict__ A,
+    int ne, int nc, int d, int p0, double* __restrict__ part) {
+  constexpr int D2 = D * D, NT = (D2 + 15) / 16, KS = (D2 + 3) / 4;
+  extern __shared__ __align__(16) double Ac[];  // [p][k = (L, B)][row = (R, U)], zero padded
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, m = lane & 15, kq = lane >> 4;
+  const int np = (int)blockDim.x / (64 * NT);  // indices p0 .. p0 + np - 1 of d
+  for (int x = tid; x < np * KS * 4 * NT * 16; x += blockDim.x) {
+    const int row = x % (NT * 16), k = x / (NT * 16) % (KS * 4), p = p0 + x / (NT * 16 * KS * 4);
+    double v = 0.0;
+    if (row < D2 && k < D2) {
+      const int L = k / D, B = k % D, R = row / D, U = row % D;
+      v = A[((((int64_t)L * D + U) * D + R) * D + B) * d + p];
+    }
+    Ac[x] = v;
+  }
+  __syncthreads();
+  const int p = wave / NT, tn = wave % NT;
+  const double* Ap = Ac + (size_t)p * KS * 4 * NT * 16;
+  const int64_t s1 = (int64_t)ne * D2, s3 = (int64_t)nc * D2;
+  // this lane's column (l, b) of T1 and rows (r, u) of T3
+  const int cl = min(tn * 16 + m, D2 - 1);
+  const int64_t c1 = (int64_t)(cl / D) * D * s1 + cl % D * D;
+  d4 acc[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) acc[t] = d4{0.0, 0.0, 0.0, 0.0};
+  for (int blk = blockIdx.x; blk < ne * nc; blk += gridDim.x) {
+    const int c = blk / ne, e = blk % ne;
+    const double* x1 = T1 + c * (int64_t)D2 * s1 + (int64_t)e * D2 + c1;
+    double xb[KS];
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      const int k = 4 * ks + kq, kc = min(k, D2 - 1);
+      const double v = x1[kc / D * s1 + kc % D];
+      xb[ks] = k < D2 ? v : 0.0;
+    }
+    d4 z[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      z[t] = d4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks)
+        z[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(Ap[(4 * ks + kq) * NT * 16 + t * 16 + m],
+                                                    xb[ks], z[t], 0, 0, 0);
+    }
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      if constexpr (NT > 3) __builtin_amdgcn_sched_barrier(0);  // one row tile's loads at a time
+      const int rw = min(t * 16 + m, D2 - 1);
+      const double* x3 = T3 + ((int64_t)e * D + rw / D) * D * s3 + (int64_t)c * D2 + rw % D * D;
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        const int k = 4 * ks + kq, kc = min(k, D2 - 1);
+        const double v = x3[kc / D * s3 + kc % D];
+        acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(k < D2 ? v : 0.0, z[ks >> 2][ks & 3], acc[t],
+                                                      0, 0, 0);
+      }
+    }
+  }
+  double* out = part + (int64_t)blockIdx.x * D2 * D2 * d + p0 + p;
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int row = t * 16 + kq + 4 * r, col = tn * 16 + m;
+      if (row < D2 && col < D2) out[((int64_t)row * D2 + col) * d] = acc[t][r];
+    }
+}
+
+// Y = the sum of the workgroups' parts: 16 elements a workgroup, 16 threads
+// each summing every 16th part, then those in order
+__global__ __launch_bounds__(256) void ring_sum_kernel(const double* __restrict__ part, int n,
+                                                       int parts, double* __restrict__ Y) {
+  __shared__ double red[16][16];
+  const int o = threadIdx.x & 15, g = threadIdx.x >> 4, e = blockIdx.x * 16 + o;
+  double s = 0.0;
+  if (e < n) {
+#pragma unroll 8
+    for (int w = g; w < parts; w += 16) s += part[(int64_t)w * n + e];
+  }
+  red[g][o] = s;
+  __syncthreads();
+  if (g > 0 || e >= n) return;
+  for (int w = 1; w < 16; ++w) s += red[w][o];
+  Y[e] = s;
+}
+
+template <int D>
+void launch_ring(const double* T1, const double* T3, const double* A, int ne, int nc, int d,
+                 double* part, int wgs, hipStream_t s) {
+  constexpr int D2 = D * D, NT = (D2 + 15) / 16, KS = (D2 + 3) / 4;
+  for (int p0 = 0; p0 < d; p0 += kRingP) {
+    const int np = std::min(kRingP, d - p0);
+    const size_t lds = sizeof(double) * (size_t)np * KS * 4 * NT * 16;  // 64 KB at D = 8
+    hipLaunchKernelGGL(ring_close_kernel<D>, dim3(wgs), dim3(64 * np * NT), lds, s, T1, T3, A, ne,
+                       nc, d, p0, part);
+  }
+}
+}  // namespace
+
+size_t ring_close_work_elems(int D, int d, int ne, int nc) {
+  return (size_t)std::min<int64_t>(kRingWGs, (int64_t)ne * nc) * D * D * D * D * d;
+}
+
+void ring_close(const double* T1, const double* T3, const double* A, int D, int d, int ne, int nc,
+                double* work, double* Y, hipStream_t s) {
+  ACETN_REQUIRE(D >= 1 && D <= 8 && d >= 1 && ne >= 1 && nc >= 1 &&
+                    (int64_t)ne * nc < (int64_t(1) << 31),
+                "ring_close: unsupported shape");
+  const int wgs = (int)std::min<int64_t>(kRingWGs, (int64_t)ne * nc), n = D * D * D * D * d;
+  switch (D) {
+    case 1: launch_ring<1>(T1, T3, A, ne, nc, d, work, wgs, s); break;
+    case 2: launch_ring<2>(T1, T3, A, ne, nc, d, work, wgs, s); break;
+    case 3: launch_ring<3>(T1, T3, A, ne, nc, d, work, wgs, s); break;
+    case 4: launch_ring<4>(T1, T3, A, ne, nc, d, work, wgs, s); break;
+    case 5: launch_ring<5>(T1, T3, A, ne, nc, d, work, wgs, s); break;
+    case 6: launch_ring<6>(T1, T3, A, ne, nc, d, work, wgs, s); break;
+    case 7: launch_ring<7>(T1, T3, A, ne, nc, d, work, wgs, s); break;
+    default: launch_ring<8>(T1, T3, A, ne, nc, d, work, wgs, s); break;
+  }
+  ACETN_HIP_CHECK(hipGetLastError());
+  hipLaunchKernelGGL(ring_sum_kernel, dim3((n + 15) / 16), dim3(256), 0, s, work, n, wgs, Y);
+  ACETN_HIP_CHECK(hipGetLastError());
+}
+
 }  // namespace acetn

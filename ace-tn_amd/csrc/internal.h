@@ -217,6 +217,12 @@ struct DLDesc {
 };
 void double_layer_f64(const DLDesc& g, const double* X, const double* A, double* Y,
                       hipStream_t s);
+// Y[(r,u)][(l,b)][p] of a one-site network closed over its ring (D <= 8):
+// T1[c][l][L][e][b][B], T3[e][r][R][c][u][U], the site tensor A; ``work`` holds
+// ring_close_work_elems doubles.
+size_t ring_close_work_elems(int D, int d, int ne, int nc);
+void ring_close(const double* T1, const double* T3, const double* A, int D, int d, int ne, int nc,
+                double* work, double* Y, hipStream_t s);
 // The same contraction with FP32 operands, products and accumulation on the
 // matrix cores (v_mfma_f32_16x16x4f32): the mixed-precision path.  X and Y
 // are FP64 unless g.x_f32 / g.y_f32 say FP32.

@@ -65,3 +65,25 @@ def test_measure_api_golden_energy(hip, case):
     ip.load_arrays(st)
     e = ip.measure()['Energy'].item()
     assert e == pytest.approx(e_ref, rel=1e-10)
+
+
+@pytest.mark.parametrize("d", [1, 2, 3, 5])
+@pytest.mark.parametrize("D", [1, 2, 3, 4, 5, 6, 7, 8])
+def test_site_rdm_shapes(hip, D, d):
+    """The closing contraction of the ring at every tile count, with one to
+    three launches over the physical index and boundaries of unequal extents
+    (fewer and more blocks than workgroups), against the oracle: one ulp per
+    term of each sum, in units of the sums of magnitudes."""
+    rng = np.random.default_rng(10 * D + d)
+    for n, m in ((3, 4), (23, 29) if D < 5 else (5, 7)):
+        x = {"a0": 5, "b0": 3, "c4": n, "e3": m, "b1": 6, "c1": 4, "a3": 7, "c2": 5}
+        C = [(x["c4"], x["b1"]), (x["c1"], x["c2"]), (x["a3"], x["e3"]), (x["a0"], x["b0"])]
+        E = [(x["b1"], x["c1"]), (x["c2"], x["a3"]), (x["e3"], x["a0"]), (x["b0"], x["c4"])]
+        site = {"A": rng.standard_normal((D, D, D, D, d)),
+                "C": [rng.standard_normal(s) for s in C],
+                "E": [rng.standard_normal(s + (D, D)) for s in E]}
+        mag = {"A": np.abs(site["A"]), "C": [np.abs(t) for t in site["C"]],
+               "E": [np.abs(t) for t in site["E"]]}
+        terms = sum(x.values()) + D * D + n * m * D * D + D ** 4
+        got = hip.site_rdm(dsite(site)).cpu().numpy()
+        assert np.all(np.abs(got - om.site_rdm(site)) <= 2.0 ** -52 * terms * om.site_rdm(mag))
