@@ -10,12 +10,12 @@
 // (acetn/renormalization/directional_mover.py:363-364).
 //
 // For a fixed boundary pair the work is two (D^2 x D^2 x D^2) products per
-// physical index p:  T = X . Abar_p  and  Y += A_p^T . T.  NB blocks are
-// stacked so that the row count is a multiple of the 16-row MFMA tile
-// (NB = 4 at D = 6 gives exactly 144 rows), and both products run on
-// v_mfma_f64_16x16x4_f64 from LDS.  Y stays in registers across p; the
-// 7-index chi^2 D^4 d intermediate never reaches HBM, X and Y are read and
-// written once.
+// physical index p:  T = X . Abar_p  and  Y += A_p^T . T, both on the matrix
+// cores, in two kernels: one stacks NB blocks so that the row count is a multiple
+// of the 16-row MFMA tile (NB = 4 at D = 6 gives exactly 144 rows) and works from
+// LDS, the other gives each wave a block and chains the products in registers.
+// Y stays in registers across p; the 7-index chi^2 D^4 d intermediate never
+// reaches HBM, X and Y are read and written once.
 #include "internal.h"
 
 namespace acetn {
@@ -35,6 +35,8 @@ template <> struct DLMath<double> {
     return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
   }
   static __device__ __forceinline__ int row(int lane, int r) { return (lane >> 4) + 4 * r; }
+  // result tile -> the operands of the next product's four k steps
+  static __device__ __forceinline__ void to_operand(acc_t&) {}
 };
 template <> struct DLMath<float> {
   typedef f4 acc_t;
@@ -42,6 +44,22 @@ template <> struct DLMath<float> {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
   }
   static __device__ __forceinline__ int row(int lane, int r) { return 4 * (lane >> 4) + r; }
+  // the 4 x 4 transpose of registers and rows of 16 lanes
+  static __device__ __forceinline__ void to_operand(acc_t& z) {
+    const auto swap = [](float a, float b, bool half, float& lo, float& hi) {
+      const unsigned x = __float_as_uint(a), y = __float_as_uint(b);
+      const auto w = half ? __builtin_amdgcn_permlane32_swap(x, y, false, false)
+                          : __builtin_amdgcn_permlane16_swap(x, y, false, false);
+      lo = __uint_as_float(w[0]);
+      hi = __uint_as_float(w[1]);
+    };
+    float a, b, c, e, t0, t1, t2, t3;
+    swap(z[0], z[2], true, a, c);
+    swap(z[1], z[3], true, b, e);
+    swap(a, b, false, t0, t1);
+    swap(c, e, false, t2, t3);
+    z = acc_t{t0, t1, t2, t3};
+  }
 };
 
 namespace {
@@ -54,7 +72,7 @@ constexpr int NW = NT / 64;
 template <int D>
 struct DLShape {
   static constexpr int D2 = D * D;
-  static constexpr int NB = (D == 6) ? 4 : ((64 / D2) > 0 ? (64 / D2) : 1);
+  static constexpr int NB = (D == 6) ? 4 : (D == 5) ? 2 : 1;
   static constexpr int ROWS = NB * D2;            // stacked rows
   static constexpr int MP = (ROWS + 15) / 16 * 16; // padded rows (step c M, step d N)
   static constexpr int KP = (D2 + 3) / 4 * 4;      // padded contraction length
@@ -65,11 +83,12 @@ struct DLShape {
   static constexpr int XPT = (MP * KP + NT - 1) / NT; // X elements per thread
 };
 
-template <int D, typename T>
+template <int D>
 __global__ __launch_bounds__(NT) void dl_mfma_kernel(DLDesc g, const double* __restrict__ X,
                                                      const double* __restrict__ A,
                                                      double* __restrict__ Y) {
   using S = DLShape<D>;
+  using T = double;
   using M = DLMath<T>;
   typedef typename M::acc_t acc_t;
   extern __shared__ __align__(16) char smem[];
@@ -88,7 +107,7 @@ __global__ __launch_bounds__(NT) void dl_mfma_kernel(DLDesc g, const double* __r
       const int l1 = kk / D, l2 = kk % D, l3 = nn / D, l4 = nn % D;
       v = A[l1 * g.a_leg[0] + l2 * g.a_leg[1] + l3 * g.a_leg[2] + l4 * g.a_leg[3] + p * g.a_p];
     }
-    Ac[e] = (T)v;
+    Ac[e] = v;
   }
 
   const int nblk = g.n1 * g.n2;
@@ -123,12 +142,7 @@ __global__ __launch_bounds__(NT) void dl_mfma_kernel(DLDesc g, const double* __r
 #pragma unroll
       for (int bb = 0; bb < S::NB; ++bb)
         if (x_blk[t] == bb) bo = base[bb];
-      if (bo < 0)
-        xr[t] = (T)0;
-      else if (g.x_f32)
-        xr[t] = (T)reinterpret_cast<const float*>(X)[bo + x_loff[t]];
-      else
-        xr[t] = (T)X[bo + x_loff[t]];
+      xr[t] = bo < 0 ? 0.0 : X[bo + x_loff[t]];
     }
   };
   if ((int)blockIdx.x < ngroups) load_x(blockIdx.x);
@@ -139,7 +153,7 @@ __global__ __launch_bounds__(NT) void dl_mfma_kernel(DLDesc g, const double* __r
 #pragma unroll
     for (int t = 0; t < S::XPT; ++t) {
       const int e = tid + t * NT;
-      if (e < S::MP * S::KP) Xs[(e / S::KP) * S::XLD + e % S::KP] = (T)xr[t];
+      if (e < S::MP * S::KP) Xs[(e / S::KP) * S::XLD + e % S::KP] = xr[t];
     }
     if (grp + (int)gridDim.x < ngroups) load_x(grp + gridDim.x);
     acc_t yacc[S::TPW];
@@ -211,10 +225,7 @@ __global__ __launch_bounds__(NT) void dl_mfma_kernel(DLDesc g, const double* __r
                   if (m < S::D2) {
                     const int k3 = m / D, k4 = m % D;
                     const int64_t yo = yb + k3 * g.y_k3 + b3 * g.y_b3 + k4 * g.y_k4 + b4 * g.y_b4;
-                    if (g.y_f32)
-                      reinterpret_cast<float*>(Y)[yo] = (float)yacc[t][r];
-                    else
-                      Y[yo] = (double)yacc[t][r];
+                    Y[yo] = yacc[t][r];
                   }
                 }
               }
@@ -226,41 +237,181 @@ __global__ __launch_bounds__(NT) void dl_mfma_kernel(DLDesc g, const double* __r
   }
 }
 
+// The same two products, a boundary block a wave: X is read straight into the
+// operands of the first (rows (k1,k2), k (b1,b2)), whose result tiles are the
+// second's operands, so a wave meets no barrier and only A is in LDS.  One column
+// tile of (b3,b4) at a time, X kept for all of them.  More padding than the
+// stacked rows above at D = 5 and 6, no intermediate in LDS; bound by the
+// scattered loads and stores (32 - 48 byte pieces) and, in FP64, by the products.
+// The order of sums is that of the stacked kernel, bit for bit.
 template <int D, typename T>
-void launch_dl(const DLDesc& g, const double* X, const double* A, double* Y, hipStream_t s) {
+__global__ __launch_bounds__(256) void dl_wave_kernel(DLDesc g, const double* __restrict__ X,
+                                                      const double* __restrict__ A,
+                                                      double* __restrict__ Y) {
+  using M = DLMath<T>;
+  typedef typename M::acc_t acc_t;
+  constexpr int D2 = D * D, NT = (D2 + 15) / 16, KS = (D2 + 3) / 4, KP = 4 * KS, NP = 16 * NT;
+  extern __shared__ __align__(16) char smem[];
+  int64_t* yrow = reinterpret_cast<int64_t*>(smem);  // (k3, k4)
+  int64_t* ycol = yrow + NP;                         // (b3, b4)
+  T* Ac = reinterpret_cast<T*>(ycol + NP);           // [p][KP][NP], zero padded
+  const int d = g.d;
+  const int tid = threadIdx.x, lane = tid & 63, m = lane & 15, kq = lane >> 4;
+  for (int e = tid; e < d * KP * NP; e += 256) {
+    const int p = e / (KP * NP), r = e % (KP * NP), kk = r / NP, nn = r % NP;
+    double v = 0.0;
+    if (kk < D2 && nn < D2)
+      v = A[kk / D * g.a_leg[0] + kk % D * g.a_leg[1] + nn / D * g.a_leg[2] + nn % D * g.a_leg[3] +
+            p * g.a_p];
+    Ac[e] = (T)v;
+  }
+  if (tid < NP) {
+    const int i = min(tid, D2 - 1);
+    yrow[tid] = i / D * g.y_k3 + i % D * g.y_k4;
+    ycol[tid] = i / D * g.y_b3 + i % D * g.y_b4;
+  }
+  __syncthreads();
+  int xrow[NT], xcol[KS];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    const int i = min(16 * t + m, D2 - 1);
+    xrow[t] = (int)(i / D * g.x_k1 + i % D * g.x_k2);
+  }
+#pragma unroll
+  for (int s = 0; s < KS; ++s) {
+    const int i = min(4 * s + kq, D2 - 1);
+    xcol[s] = (int)(i / D * g.x_b1 + i % D * g.x_b2);
+  }
+  const int nblk = g.n1 * g.n2, nwave = gridDim.x * 4;
+  for (int blk = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(tid >> 6); blk < nblk;
+       blk += nwave) {
+    const int o1 = blk / g.n2, o2 = blk % g.n2;
+    const int64_t xo = o1 * g.x_o1 + o2 * g.x_o2, yo = o1 * g.y_o1 + o2 * g.y_o2;
+    T xa[NT][KS];
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int s = 0; s < KS; ++s) {
+        const int64_t at = xo + xrow[t] + xcol[s];
+        const T v = g.x_f32 ? (T)reinterpret_cast<const float*>(X)[at] : (T)X[at];
+        // padding rows and columns hold zeros where a product reaches them
+        const bool ok = (KP == D2 || 4 * s + kq < D2) && (KP == D2 || 16 * t + m < D2);
+        xa[t][s] = ok ? v : T(0);
+      }
+#pragma unroll 1
+    for (int tn = 0; tn < NT; ++tn) {
+      acc_t y[NT];
+#pragma unroll
+      for (int t = 0; t < NT; ++t) y[t] = acc_t{0, 0, 0, 0};
+      // closed: sum_p A_p^T (X Abar_p);  open: every (p, pb) pair written out
+#pragma unroll 1
+      for (int pb = 0; pb < d; ++pb) {
+        const T* Ab = Ac + (size_t)pb * KP * NP + kq * NP + tn * 16 + m;
+        acc_t z[NT];
+#pragma unroll
+        for (int t = 0; t < NT; ++t) z[t] = acc_t{0, 0, 0, 0};
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+          const T b = Ab[4 * s * NP];
+#pragma unroll
+          for (int t = 0; t < NT; ++t) z[t] = M::mfma(xa[t][s], b, z[t]);
+        }
+#pragma unroll
+        for (int t = 0; t < NT; ++t) M::to_operand(z[t]);
+        const int p_hi = g.open_p ? d : pb + 1;
+#pragma unroll 1
+        for (int p = g.open_p ? 0 : pb; p < p_hi; ++p) {
+          const T* Ap = Ac + (size_t)p * KP * NP + kq * NP + m;
+          if (g.open_p) {
+#pragma unroll
+            for (int t = 0; t < NT; ++t) y[t] = acc_t{0, 0, 0, 0};
+          }
+#pragma unroll
+          for (int s = 0; s < KS; ++s)
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+              y[t] = M::mfma(Ap[4 * s * NP + 16 * t], z[s >> 2][s & 3], y[t]);
+          if (!g.open_p && p < d - 1) continue;
+          const int64_t yc = yo + ycol[16 * tn + m] +
+                             (g.open_p ? p * g.y_p + pb * g.y_pb : (int64_t)0);
+#pragma unroll
+          for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              const int row = 16 * t + M::row(lane, r);
+              if (16 * tn + m >= D2 || row >= D2) continue;
+              const int64_t at = yc + yrow[row];
+              if (g.y_f32) reinterpret_cast<float*>(Y)[at] = (float)y[t][r];
+              else Y[at] = (double)y[t][r];
+            }
+        }
+      }
+    }
+  }
+}
+
+// one round of resident workgroups, each looping over its share of the blocks:
+// the A tensor is staged once per workgroup
+template <int D>
+void launch_dl_stacked(const DLDesc& g, const double* X, const double* A, double* Y, hipStream_t s) {
   using S = DLShape<D>;
   static_assert(S::TC == (S::NP / 16) * (S::MP / 16), "tile counts of the two products differ");
-  const size_t lds = sizeof(T) * ((size_t)g.d * S::KP * S::NP + (size_t)S::MP * S::XLD +
-                                  (size_t)S::MP * S::NP);
+  const size_t lds = sizeof(double) * ((size_t)g.d * S::KP * S::NP + (size_t)S::MP * S::XLD +
+                                       (size_t)S::MP * S::NP);
   ACETN_REQUIRE(lds <= 160 * 1024, "double_layer: LDS budget exceeded");
-  ACETN_REQUIRE((int64_t)(D - 1) * (g.x_k1 + g.x_b1 + g.x_k2 + g.x_b2) < (int64_t(1) << 31),
-                "double_layer: block strides exceed 32-bit offsets");
   static bool attr = false;
   if (!attr) {
-    ACETN_HIP_CHECK(hipFuncSetAttribute((const void*)dl_mfma_kernel<D, T>,
+    ACETN_HIP_CHECK(hipFuncSetAttribute((const void*)dl_mfma_kernel<D>,
                                         hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
     attr = true;
   }
-  const int64_t nblk = (int64_t)g.n1 * g.n2;
-  const int64_t ngroups = (nblk + S::NB - 1) / S::NB;
-  // one round of resident workgroups (LDS-limited, 256 CUs), each looping
-  // over its share of the groups with the next group's X prefetched: the A
-  // tensor is staged once per workgroup instead of once per group or two
+  const int64_t ngroups = ((int64_t)g.n1 * g.n2 + S::NB - 1) / S::NB;
   const int per_cu = (int)std::max<size_t>(1, std::min<size_t>(8, (160 * 1024) / lds));
   const int grid = (int)std::min<int64_t>(ngroups, 256 * per_cu);
-  const double d6 = (double)S::D2 * S::D2 * S::D2;
-  const double flops = (double)nblk * (2.0 * g.d * d6 + 2.0 * (g.open_p ? g.d * g.d : g.d) * d6);
+  hipLaunchKernelGGL(dl_mfma_kernel<D>, dim3(grid), dim3(NT), lds, s, g, X, A, Y);
+}
+
+template <int D, typename T>
+void launch_dl_wave(const DLDesc& g, const double* X, const double* A, double* Y, hipStream_t s) {
+  constexpr int NP = (D * D + 15) / 16 * 16, KP = (D * D + 3) / 4 * 4;
+  constexpr int kPerCu = D >= 5 && sizeof(T) == 8 ? 3 : 4;  // D=6: 256, 247, 293 us at 2, 3, 4
+  const size_t lds = 16 * NP + sizeof(T) * (size_t)g.d * KP * NP;
+  static bool attr = false;
+  if (!attr) {
+    ACETN_HIP_CHECK(hipFuncSetAttribute((const void*)dl_wave_kernel<D, T>,
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+    attr = true;
+  }
+  const int per_cu = (int)std::max<size_t>(1, std::min<size_t>(kPerCu, (160 * 1024) / lds));
+  const int grid = (int)std::min<int64_t>(((int64_t)g.n1 * g.n2 + 3) / 4, 256 * per_cu);
+  hipLaunchKernelGGL((dl_wave_kernel<D, T>), dim3(grid), dim3(256), lds, s, g, X, A, Y);
+}
+
+// Which kernel: the wave one wherever it was the faster (us, stacked / wave;
+// FP32 D=6 198 / 164, D=8 2890 / 2730; FP64 D=2 6.5 / 3.6, D=3 6.0 / 4.5, D=4
+// 10.1 / 8, D=5 82 / 72, D=6 258 / 247), the stacked one for FP64 at D = 7 and 8
+// (385 / 398, 452 / 487) and, from D = 5, with the physical legs open (D=5 144 /
+// 166: four times the stores).
+template <int D, typename T>
+void launch_dl(const DLDesc& g, const double* X, const double* A, double* Y, hipStream_t s) {
+  ACETN_REQUIRE((int64_t)(D - 1) * (g.x_k1 + g.x_b1 + g.x_k2 + g.x_b2) < (int64_t(1) << 31),
+                "double_layer: block strides exceed 32-bit offsets");
+  const double d2 = (double)D * D, d6 = d2 * d2 * d2, nblk = (double)g.n1 * g.n2;
+  const double flops = nblk * (2.0 * g.d * d6 + 2.0 * (g.open_p ? g.d * g.d : g.d) * d6);
   hipEvent_t e0 = kernel_timing_begin(s);
-  hipLaunchKernelGGL((dl_mfma_kernel<D, T>), dim3(grid), dim3(NT), lds, s, g, X, A, Y);
+  if constexpr (sizeof(T) == 8 && D >= 5) {
+    if (D > 6 || g.open_p) launch_dl_stacked<D>(g, X, A, Y, s);
+    else launch_dl_wave<D, T>(g, X, A, Y, s);
+  } else {
+    launch_dl_wave<D, T>(g, X, A, Y, s);
+  }
   ACETN_HIP_CHECK(hipGetLastError());
   // algorithmic bytes: the X blocks read once, the Y blocks written once
   const double yblk = g.open_p ? (double)g.d * g.d : 1.0;
   const double xb = g.x_f32 ? 4.0 : 8.0, yb = g.y_f32 ? 4.0 : 8.0;
-  kernel_timing_end(e0, s, kKDoubleLayer, flops, (double)nblk * S::D2 * S::D2 * (xb + yb * yblk));
+  kernel_timing_end(e0, s, kKDoubleLayer, flops, nblk * d2 * d2 * (xb + yb * yblk));
 }
-}  // namespace
 
-namespace {
 template <typename T>
 void double_layer_t(const DLDesc& g, const double* X, const double* A, double* Y, hipStream_t s) {
   ACETN_REQUIRE(g.d >= 1 && g.d <= 4, "double_layer: d must be in [1, 4]");

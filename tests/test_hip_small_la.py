@@ -250,3 +250,39 @@ def test_als_sweep_shapes(hip, nD, D, d, sign):
                                             dv(a2)[None].repeat(2, 1, 1, 1)))
     for i in (0, 1):
         assert torch.equal(b1[i], h1) and torch.equal(b2[i], h2) and int(bf[i]) == flags
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("d", [1, 2, 3])
+@pytest.mark.parametrize("D", [1, 2, 3, 4, 5, 6, 7, 8])
+def test_double_layer_shapes(hip, D, d, precision):
+    """The double-layer absorption at every tile count and padding, fewer and
+    more boundary blocks than waves, against the oracle's enlarged corner:
+    one ulp (of FP32 in mixed precision, with the split corner's rounding) per
+    term of the longest sum, in units of the sums of magnitudes."""
+    from oracle import ctmrg as oc
+
+    def raw(s):  # oracle.make_quarter_tensor before it is scaled
+        a = oc.bond_permute(s["A"], 1)
+        q = oc.ein("acuU,ealL->cuUelL", oc.ein("ab,bcuU->acuU", s["C"][1], s["E"][1]), s["E"][0])
+        q = oc.ein("lurdp,cuelRDp->crRedD", a, oc.ein("cuUelL,LURDp->cuelRDp", q, a))
+        return q.reshape(q.shape[0] * D * D, -1)
+
+    rng = np.random.default_rng(10 * D + d)
+    for chi in (3, 33) if D <= 4 else (3, 7):
+        site = {"A": rng.standard_normal((D, D, D, D, d)),
+                "C": [rng.standard_normal((chi, chi)) for _ in range(4)],
+                "E": [rng.standard_normal((chi, chi, D, D)) for _ in range(4)]}
+        mag = {k: np.abs(v) if k == "A" else [np.abs(t) for t in v] for k, v in site.items()}
+        dv = lambda t: torch.as_tensor(t, device="cuda")
+        try:
+            got = hip.quarter_tensor((dv(site["A"]), [dv(t) for t in site["C"]],
+                                      [dv(t) for t in site["E"]]), 1, precision=precision)
+        except RuntimeError as e:
+            assert "LDS budget" in str(e) and (D, d) == (8, 3) and precision == "fp64"
+            continue
+        got, ref, mg = got.cpu().numpy(), raw(site), raw(mag)
+        sc = np.abs(ref).max() / np.abs(got).max()  # the engine's may be scaled
+        ulp = 2.0 ** -52 if precision == "fp64" else 2.0 ** -23
+        terms = 2 * chi + D ** 4 * d
+        assert np.all(np.abs(got * sc - ref) <= 2 * ulp * terms * mg)
