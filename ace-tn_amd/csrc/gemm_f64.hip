@@ -588,28 +588,6 @@ __global__ __launch_bounds__(1024) void gemm_f64_small_kernel(GemmDesc g, GemmBa
   }
 }
 
-bool small_shape(const GemmDesc& g, int count) {
-  if (!g.pipe || g.K <= 0) return false;
-  const int64_t tiles = (int64_t)((g.M + 15) / 16) * ((g.N + 15) / 16) * count;
-  // below the pipelined kernel's range; K too long for one workgroup's waves
-  // (102 x 102 x 2500: 15 us against 22, 16 x 16 x 4096: 24 against 16) and
-  // many tiles of next to no k (1000 x 1000 x 20: 12.6 against 11.9) stay
-  // with the split and the larger tiles
-  return (double)g.M * g.N * g.K * count < 5e7 && g.K <= SP_MAXK && tiles <= (g.K >= 32 ? 4096 : 1024);
-}
-void launch_small(const GemmDesc& g, const GemmBatch& b, hipStream_t s) {
-  const dim3 grid((g.N + 15) / 16, (g.M + 15) / 16, b.count);
-  const dim3 block(64 * std::min(16, std::max(1, (g.K + 63) / 64)));
-  const bool lin = g.am.n0 <= 0 && g.ak.n0 <= 0 && g.bk.n0 <= 0 && g.bn.n0 <= 0;
-  const bool ak = g.ak.s0 == 1, bc = g.bk.s0 == 1;
-  auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, 0, s, g, b); };
-  if (!lin) launch(gemm_f64_small_kernel<false, false, true>);
-  else if (ak && bc) launch(gemm_f64_small_kernel<true, true, false>);
-  else if (ak) launch(gemm_f64_small_kernel<true, false, false>);
-  else if (bc) launch(gemm_f64_small_kernel<false, true, false>);
-  else launch(gemm_f64_small_kernel<false, false, false>);
-}
-
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 // Shapes the pipelined kernel takes over: plainly strided as above (rows of even
@@ -648,6 +626,33 @@ int pipe_ksplit(const GemmDesc& g) {
     }
   }
   return best;
+}
+
+// Shapes the small kernel takes: within its range of K (102 x 102 x 2500: 15 us
+// against 22, 16 x 16 x 4096: 24 against 16), not many tiles of next to no k
+// (1000 x 1000 x 20: 12.6 us against 11.9), and up to 1.4e8 multiply-adds with the
+// padding of its tiles, where reading the operands once a tile begins to cost
+// more than the pipelined kernel's second launch (1024 x 66 x 1024: 15 - 17 us
+// against 17.6 in two launches, 500^3: 16 against 24, 1600 x 72 x 1600: even, 8000 x
+// 24 x 600: 26 against 19); one that the pipelined kernel takes in one launch
+// stays there (1024 x 1024 x 64: 15.6 us against 16.2).
+bool small_shape(const GemmDesc& g, int count) {
+  if (!g.pipe || g.K <= 0 || g.K > SP_MAXK) return false;
+  const int64_t tiles = (int64_t)((g.M + 15) / 16) * ((g.N + 15) / 16) * count;
+  if (256.0 * tiles * g.K >= 1.4e8 || tiles > (g.K >= 32 ? 4096 : 1024)) return false;
+  return !pipe_shape(g, count) || pipe_ksplit(g) > 1;
+}
+void launch_small(const GemmDesc& g, const GemmBatch& b, hipStream_t s) {
+  const dim3 grid((g.N + 15) / 16, (g.M + 15) / 16, b.count);
+  const dim3 block(64 * std::min(16, std::max(1, (g.K + 63) / 64)));
+  const bool lin = g.am.n0 <= 0 && g.ak.n0 <= 0 && g.bk.n0 <= 0 && g.bn.n0 <= 0;
+  const bool ak = g.ak.s0 == 1, bc = g.bk.s0 == 1;
+  auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, 0, s, g, b); };
+  if (!lin) launch(gemm_f64_small_kernel<false, false, true>);
+  else if (ak && bc) launch(gemm_f64_small_kernel<true, true, false>);
+  else if (ak) launch(gemm_f64_small_kernel<true, false, false>);
+  else if (bc) launch(gemm_f64_small_kernel<false, true, false>);
+  else launch(gemm_f64_small_kernel<false, false, false>);
 }
 
 template <int WN>
@@ -803,8 +808,7 @@ void launch_gemm_wide(const GemmDesc& g, const GemmBatch& b, int ks, double* wor
 }  // namespace
 
 // Large enough that 64-row tiles and a few k parts fill the chip: below 5e7
-// products (324 x 38 x 324 has 4e6) a call is launches and latency either way,
-// and 1024 x 66 x 1024 (7e7) takes 17 us against 20.
+// products (324 x 38 x 324 has 4e6) a call is launches and latency either way.
 bool gemm_f64_large(int64_t M, int64_t N, int64_t K) {
   return M >= 96 && N >= 17 && K >= 32 && (double)M * N * K >= 5e7;
 }
@@ -868,7 +872,7 @@ void gemm_f64(const GemmDesc& g, const GemmBatch& b, double* work, size_t work_e
   const bool small = small_shape(g, b.count);
   const bool in_table = autotune_lookup(key, &listed) && fits(listed.ks) &&
                         (listed.var == 0 || lin) && (small || listed.wn != 1);
-  if (!in_table && pipe_shape(g, b.count) && aligned16(b.A[0]) && aligned16(b.B[0])) {
+  if (!in_table && !small && pipe_shape(g, b.count) && aligned16(b.A[0]) && aligned16(b.B[0])) {
     const int ks = pipe_ksplit(g);
     if (ks == 1 || (work != nullptr && work_elems >= (size_t)ks * g.M * g.N)) {
       hipEvent_t e0 = kernel_timing_begin(s);
