@@ -170,11 +170,17 @@ const double* orthonormalize(Ctx& c, double* Y, int64_t m, int64_t q, bool steer
     gr.run_if = run_if;
     gemm(c, gr, src, Rinv, dst);
   };
-  // pass 0: shifted (Y -> Yt)
-  pass(Y, Yt, 11.0 * ((double)m * q + (double)q * (q + 1)) * u, 0.0, nullptr, nullptr, false);
-  if (single) return Yt;
-  // pass 1: plain with rank guard (Yt -> Y); dropped columns come out zero
-  pass(Yt, Y, 0.0, 1e-14, dead, nullptr, false);
+  const double shift = 11.0 * ((double)m * q + (double)q * (q + 1)) * u;
+  if (!c.mixed && ortho_small_fits(m, q)) {
+    // passes 0 and 1 in one launch
+    if (c.launch) ortho_small(Y, Yt, G, Rinv, mi, qi, shift, 1e-14, dead, c.st);
+  } else {
+    // pass 0: shifted (Y -> Yt)
+    pass(Y, Yt, shift, 0.0, nullptr, nullptr, false);
+    if (single) return Yt;
+    // pass 1: plain with rank guard (Yt -> Y); dropped columns come out zero
+    pass(Yt, Y, 0.0, 1e-14, dead, nullptr, false);
+  }
   if (c.trust) {
     if (c.launch) c.drops.add(any);
     return Y;

@@ -256,6 +256,11 @@ void chol_rinv(const double* G, double* Rinv, int q, double shift_rel, double ra
 // row-major) by N(0,1) Philox vectors.
 void refill_dead_columns(double* Y, int64_t m, int q, const int* dead, uint64_t seed,
                          hipStream_t s);
+// The first two CholeskyQR passes of a small basis in one launch: Y (m x q) ->
+// Yt (shifted) -> Y (rank guard; dead as chol_rinv's dead_out).
+bool ortho_small_fits(int64_t m, int64_t q);
+void ortho_small(double* Y, double* Yt, double* G, double* Rinv, int m, int q, double shift_rel,
+                 double rank_tol, int* dead, hipStream_t s);
 // Zero the columns of Y (m x q) not flagged in ``dead`` (device, q + 1 ints,
 // dead[q] = any); a no-op when none is flagged.
 void keep_dead_columns(double* Y, int64_t m, int q, const int* dead, hipStream_t s);

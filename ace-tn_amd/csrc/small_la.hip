@@ -470,9 +470,9 @@ __device__ __forceinline__ void ct_factor_diag(const double* D, double* Zs, int 
 }
 
 template <int NW, int NS>
-__global__ __launch_bounds__(64 * NW) void chol_rinv_tile_kernel(
-    const double* __restrict__ G, double* __restrict__ Rinv, int q, double shift_rel,
-    double rank_tol, int* dead_out, const int* run_if, double near_identity) {
+__device__ __forceinline__ void chol_rinv_tiles(const double* G, double* Rinv, int q,
+                                                double shift_rel, double rank_tol, int* dead_out,
+                                                const int* run_if, double near_identity) {
   constexpr int NT = 64 * NW, NO = NW - 1;  // waves with slots
   __shared__ double pan[kCtMaxT][CB_TS];    // the panel: R_kI (I > k), Z_kJ (J < k)
   __shared__ double dg[kCtMaxT][CB_TS];     // diagonal tiles
@@ -631,6 +631,85 @@ __global__ __launch_bounds__(64 * NW) void chol_rinv_tile_kernel(
     }
     anyd = __syncthreads_or(anyd);
     if (tid == 0) dead_out[q] = anyd;
+  }
+}
+
+template <int NW, int NS>
+__global__ __launch_bounds__(64 * NW) void chol_rinv_tile_kernel(
+    const double* __restrict__ G, double* __restrict__ Rinv, int q, double shift_rel,
+    double rank_tol, int* dead_out, const int* run_if, double near_identity) {
+  chol_rinv_tiles<NW, NS>(G, Rinv, q, shift_rel, rank_tol, dead_out, run_if, near_identity);
+}
+
+// The first two CholeskyQR passes of a small basis (m x q) in one launch of one
+// workgroup: Gram matrix, factor and product of the shifted pass (Y -> Yt), then
+// of the plain one with the rank guard (Yt -> Y).  G and Rinv hold those of the
+// last pass, as after the six launches this replaces.  At these sizes a launch
+// costs the host more than its kernel runs (Gram 5, factor 11 - 15, product 5 us).
+constexpr int kOsWaves = 8;
+__global__ __launch_bounds__(64 * kOsWaves) void ortho_small_kernel(double* Y, double* Yt, double* G,
+                                                                    double* Rinv, int m, int q,
+                                                                    double shift_rel,
+                                                                    double rank_tol, int* dead) {
+  const int lane = threadIdx.x & 63, x = lane & 15, kq = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int Q = (q + 15) / 16, rows = (m + 15) / 16;
+#pragma unroll 1
+  for (int pass = 0; pass < 2; ++pass) {
+    const double* src = pass == 0 ? Y : Yt;
+    double* dst = pass == 0 ? Yt : Y;
+    // upper tiles of G = src^T src
+#pragma unroll 1
+    for (int t = wave; t < Q * (Q + 1) / 2; t += kOsWaves) {
+      int J = 0;
+      while ((J + 1) * (J + 2) / 2 <= t) ++J;
+      const int I = t - J * (J + 1) / 2;
+      const double* pa = src + min(16 * I + x, q - 1);
+      const double* pb = src + min(16 * J + x, q - 1);
+      cb_d4 acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 16
+      for (int k0 = 0; k0 < m; k0 += 4) {
+        const int k = min(k0 + kq, m - 1);
+        const double a = pa[(int64_t)k * q], b = pb[(int64_t)k * q];
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(k0 + kq < m ? a : 0.0, b, acc, 0, 0, 0);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int i = 16 * I + kq + 4 * r, j = 16 * J + x;
+        if (i < q && j < q) G[(int64_t)i * q + j] = acc[r];
+      }
+    }
+    __syncthreads();
+    chol_rinv_tiles<kOsWaves, 4>(G, Rinv, q, pass == 0 ? shift_rel : 0.0,
+                                 pass == 0 ? 0.0 : rank_tol, pass == 0 ? nullptr : dead, nullptr,
+                                 -1.0);
+    __syncthreads();
+    // dst = src Rinv, Rinv upper triangular (zeros below, so k runs to q for all
+    // four column tiles at once)
+    for (int I = wave; I < rows; I += kOsWaves) {
+      const double* pa = src + (int64_t)min(16 * I + x, m - 1) * q;
+      cb_d4 acc[4];
+#pragma unroll
+      for (int J = 0; J < 4; ++J) acc[J] = cb_d4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll 4
+      for (int k0 = 0; k0 < q; k0 += 4) {
+        const int k = min(k0 + kq, q - 1);
+        const double v = pa[k], a = k0 + kq < q ? v : 0.0;
+#pragma unroll
+        for (int J = 0; J < 4; ++J)
+          if (J < Q)
+            acc[J] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+                a, Rinv[(int64_t)k * q + min(16 * J + x, q - 1)], acc[J], 0, 0, 0);
+      }
+#pragma unroll
+      for (int J = 0; J < 4; ++J)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int i = 16 * I + kq + 4 * r, j = 16 * J + x;
+          if (i < m && j < q) dst[(int64_t)i * q + j] = acc[J][r];
+        }
+    }
+    __syncthreads();
   }
 }
 
@@ -1556,6 +1635,21 @@ void chol_rinv(const double* G, double* Rinv, int q, double shift_rel, double ra
     hipLaunchKernelGGL(chol_rinv_kernel<false>, dim3(1), dim3(LA_NT), 0, s, G, Rinv, q, shift_rel,
                        rank_tol, gscratch, use_lds, dead_out, run_if);
   ACETN_HIP_CHECK(hipGetLastError());
+}
+
+// The line: 1e5 multiply-adds a product.  80 x 22 (4e4) takes 38 us against 40 in six
+// launches and spares the host five of them; 315 x 37 (4e5) takes 103 us against 52.
+bool ortho_small_fits(int64_t m, int64_t q) {
+  return q <= 64 && (double)m * q * q <= 1e5;
+}
+void ortho_small(double* Y, double* Yt, double* G, double* Rinv, int m, int q, double shift_rel,
+                 double rank_tol, int* dead, hipStream_t s) {
+  ACETN_REQUIRE(m >= 1 && q >= 1 && ortho_small_fits(m, q), "ortho_small: unsupported shape");
+  hipEvent_t e0 = kernel_timing_begin(s);
+  hipLaunchKernelGGL(ortho_small_kernel, dim3(1), dim3(64 * kOsWaves), 0, s, Y, Yt, G, Rinv, m, q,
+                     shift_rel, rank_tol, dead);
+  ACETN_HIP_CHECK(hipGetLastError());
+  if (e0) kernel_timing_end(e0, s, kKCholesky, (double)q * q * q + 6.0 * m * q * q, 0.0);
 }
 
 void keep_dead_columns(double* Y, int64_t m, int q, const int* dead, hipStream_t s) {

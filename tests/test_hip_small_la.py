@@ -286,3 +286,25 @@ def test_double_layer_shapes(hip, D, d, precision):
         ulp = 2.0 ** -52 if precision == "fp64" else 2.0 ** -23
         terms = 2 * chi + D ** 4 * d
         assert np.all(np.abs(got * sc - ref) <= 2 * ulp * terms * mg)
+
+
+@pytest.mark.parametrize("rank", ["full", "half"])
+@pytest.mark.parametrize("m,q", [(1, 1), (16, 1), (17, 16), (33, 17), (80, 22), (97, 32), (84, 33),
+                                 (48, 45), (64, 39), (65, 40), (24, 64)])
+def test_orthonormalize_small_bases(hip, m, q, rank):
+    """The one-launch CholeskyQR at the remainders of its tiles and on both
+    sides of its line (1e5 multiply-adds), with full and deficient columns,
+    against LAPACK's spans (columns of condition 1e3: 1e-12)."""
+    g = np.random.default_rng(m + q)
+    q = min(m, q)
+    r = q if rank == "full" else (q + 1) // 2
+    Y = g.standard_normal((m, r)) * np.logspace(0, -3, r)
+    Y = np.concatenate([Y, Y[:, :q - r] + Y[:, r - 1:r]], axis=1)
+    Q = hip.orthonormalize(torch.as_tensor(Y, device="cuda")).cpu().numpy()
+    assert np.abs(Q.T @ Q - np.eye(q)).max() <= 1e-13
+    ref = np.linalg.qr(Y[:, :r])[0]
+    for n in sorted({1, (r + 1) // 2, r}):
+        P = ref[:, :n] - Q[:, :r] @ (Q[:, :r].T @ ref[:, :n])
+        if rank == "half":
+            P = ref[:, :n] - Q @ (Q.T @ ref[:, :n])
+        assert np.abs(P).max() <= 1e-12
