@@ -912,9 +912,10 @@ __device__ bool als_eliminate(double* R, double* S, int nR, int d, double shift,
 // through LDS and most of a sweep; on all 256 threads it is bound by the step's
 // round trip (nR = 72, the whole call of a D=6 bond: 2440 -> 1530 us).
 constexpr int kAlsMaxTiles = 9;  // nR <= 144 (LDS holds less)
+template <int RC>
 __device__ int als_solve_system(const AlsShared& sh, int nR, int d, double eps, int* flag) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  __shared__ double pub[2 * (16 * kAlsMaxTiles + 8)], dinv[16 * kAlsMaxTiles];
+  __shared__ double pub[2 * (16 * RC + 8)], dinv[16 * RC];
   double* R = sh.R;
   double* S = sh.S;
   // the symmetric part goes to the upper triangle
@@ -933,11 +934,7 @@ __device__ int als_solve_system(const AlsShared& sh, int nR, int d, double eps, 
   double diag = tid < nR ? R[tid * nR + tid] + shift : 0.0;
   if (tid == 0) *flag = 0;
   __syncthreads();
-  bool ok;
-  if (nR <= 48) ok = als_eliminate<3>(R, S, nR, d, shift, pub, dinv);
-  else if (nR <= 80) ok = als_eliminate<5>(R, S, nR, d, shift, pub, dinv);
-  else ok = als_eliminate<kAlsMaxTiles>(R, S, nR, d, shift, pub, dinv);
-  if (ok) {
+  if (als_eliminate<RC>(R, S, nR, d, shift, pub, dinv)) {
     // D L^T x = S, a right-hand side a wave: lane l holds rows l, l + 64, l + 128
     for (int c = wave; c < d; c += ALS_NT / 64) {
       double x[3], w[3];
@@ -1053,12 +1050,17 @@ __device__ double als_cost(const AlsShared& sh, const double* __restrict__ n12, 
   return block_sum(part, sh.red);
 }
 
+// RC: the elimination's tiles (nR <= 16 RC), 0 for the pseudo-inverse: one kernel
+// each, for what the largest holds in registers would halve a batch of small
+// problems' workgroups a CU (4000 of D=3: 1.26 ms, 3.2 ms with one kernel for all,
+// 2.1 ms with one wave factorising; 1000 of D=6: 2.5, 4.1, 8.0)
+template <int RC>
 __global__ __launch_bounds__(ALS_NT) void als_kernel(const double* __restrict__ n12,
                                                      const double* __restrict__ a12g,
                                                      double* __restrict__ a1r,
                                                      double* __restrict__ a2r, int nD, int D,
                                                      int d, int niter, double tol, double eps,
-                                                     int method, double* __restrict__ gwork,
+                                                     double* __restrict__ gwork,
                                                      double* __restrict__ out_cost,
                                                      int* __restrict__ out_info,
                                                      int64_t n12_stride, int64_t gwork_stride,
@@ -1105,8 +1107,8 @@ __global__ __launch_bounds__(ALS_NT) void als_kernel(const double* __restrict__ 
     for (int side = 0; side < 2; ++side) {
       double* own = side == 0 ? sh.a1 : sh.a2;
       als_build(sh, n12, side, nD, D, d, grp, side == 0 ? sh.a2 : sh.a1);
-      if (method == 1) als_pinv_solve(sh, nR, d, eps, gwork);
-      else info |= als_solve_system(sh, nR, d, eps, &flag);
+      if constexpr (RC == 0) als_pinv_solve(sh, nR, d, eps, gwork);
+      else info |= als_solve_system<RC>(sh, nR, d, eps, &flag);
       for (int e = tid; e < nR * d; e += ALS_NT) own[e] = sh.S[e];
       __syncthreads();
     }
@@ -1285,17 +1287,23 @@ void als_solve_device(const double* n12, const double* a12g, double* a1r, double
   const size_t one = als_lds_bytes(nD, D, d), t1 = sizeof(double) * (size_t)nD * nD * D * d;
   const int grp = count > 1 ? 1 : (int)std::min<size_t>(nD, 1 + (150 * 1024 - one) / t1);
   const size_t lds = one + (grp - 1) * t1;
-  static bool attr = false;
-  if (!attr) {
-    ACETN_HIP_CHECK(hipFuncSetAttribute((const void*)als_kernel,
-                                        hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024));
-    attr = true;
-  }
   const int64_t n12_stride = (int64_t)nD * nD * nD * nD;
-  hipLaunchKernelGGL(als_kernel, dim3(count), dim3(ALS_NT), lds, s, n12, a12g, a1r, a2r, nD, D, d,
-                     niter, tol, eps, method, gwork, out_cost, out_info, n12_stride,
-                     (int64_t)als_work_elems(nD, D, d), grp);
-  ACETN_HIP_CHECK(hipGetLastError());
+  auto launch = [&](auto kernel) {
+    // (set on each call: one kernel a size class, and cheap)
+    ACETN_HIP_CHECK(hipFuncSetAttribute((const void*)kernel,
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024));
+    hipLaunchKernelGGL(kernel, dim3(count), dim3(ALS_NT), lds, s, n12, a12g, a1r, a2r, nD, D, d,
+                       niter, tol, eps, gwork, out_cost, out_info, n12_stride,
+                       (int64_t)als_work_elems(nD, D, d), grp);
+    ACETN_HIP_CHECK(hipGetLastError());
+  };
+  const int tiles = (nD * D + 15) / 16;
+  if (method == 1) launch(als_kernel<0>);
+  else if (tiles <= 1) launch(als_kernel<1>);
+  else if (tiles <= 2) launch(als_kernel<2>);
+  else if (tiles <= 3) launch(als_kernel<3>);
+  else if (tiles <= 5) launch(als_kernel<5>);
+  else launch(als_kernel<kAlsMaxTiles>);
 }
 
 }  // namespace acetn
