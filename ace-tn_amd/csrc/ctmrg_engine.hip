@@ -255,7 +255,7 @@ const double* orthonormalize(Ctx& c, double* Y, int64_t m, int64_t q, bool steer
 // the Gram matrix instead and solved by another to full precision.
 // The eigensolver's kernels, one pair, D=6, chi=144 (q = 146): a Jacobi pass as
 // preconditioner and one to full precision behind it (``signs``, mixed) take
-// 2.45 ms with their replays, this 0.55 ms (tridiagonal form 209 us, vectors
+// 2.0 ms with their replays, this 0.55 ms (tridiagonal form 209 us, vectors
 // 105, a dozen q x q products and the scan); D=4, chi=64: 0.70 against 0.25 ms.
 // ``signs``: the caller hands the vectors out without a sign gauge of its own,
 // so they keep the signs of the Jacobi rotations.  Mixed precision keeps the

@@ -292,7 +292,7 @@ __global__ __launch_bounds__(64 * NWV) void qr_reg_kernel(QrProblem p0, QrProble
 // holds row i), round-robin pair ordering; a pair is rotated while
 // |a_p . a_q| > 1e-15 * ||a_p|| ||a_q||.  Bound by instruction issue: one
 // barrier a round, the three inner products summed by lane exchanges without
-// LDS, the rotation by refined hardware reciprocals (24 x 24, graded: 114
+// LDS, the rotation by refined hardware reciprocals (24 x 24, graded: 111
 // us; 153 us with a wave a pair, 270 us without the factorisation as well,
 // 430 us with shuffles and full divisions).
 // ---------------------------------------------------------------------------
@@ -425,7 +425,9 @@ __global__ __launch_bounds__(SVD_NT) void svd_small_kernel(const double* __restr
         a[q][l] = sn * ap + c * aq;
         v[p][l] = c * vp - sn * vq;
         v[q][l] = sn * vp + c * vq;
-        rot = 1;
+        // cosines and angles below 1e-9 all through a sweep leave products of two
+        // of them, below 1e-17: the sweep that would find nothing is not run
+        rot |= ga * ga > 1e-18 * ab || fabs(t) > 1e-9;
       }
       __syncthreads();
     }

@@ -404,10 +404,10 @@ using namespace acetn;
 
 namespace {
 
-// Scratch of acetn_hip_als_solve_noalloc: the ALS system matrix and
-// right-hand sides of the largest problem it accepts (nD * D <= 128 rows,
-// d <= 4), then the final cost and the sweep / flag words.  One copy per
-// device, held until the process ends; the kernel writes every element it
+// Scratch of acetn_hip_als_solve_noalloc: room for the system of the largest
+// problem it accepts (nD * D <= 128 rows, d <= 4; the elimination now keeps it in
+// registers and LDS), then the final cost and the sweep / flag words.  One copy
+// per device, held until the process ends; the kernel writes every element it
 // reads, so nothing has to start at zero.
 constexpr int kNoAllocMaxNR = 128;
 constexpr size_t kNoAllocWork = (size_t)kNoAllocMaxNR * kNoAllocMaxNR + (size_t)kNoAllocMaxNR * 4;
