@@ -308,3 +308,21 @@ def test_orthonormalize_small_bases(hip, m, q, rank):
         if rank == "half":
             P = ref[:, :n] - Q @ (Q.T @ ref[:, :n])
         assert np.abs(P).max() <= 1e-12
+
+
+@pytest.mark.parametrize("chi,cd", [(1, 1), (2, 7), (16, 16), (17, 15), (64, 65), (64, 255),
+                                    (127, 129), (128, 128), (128, 129), (181, 90), (256, 64)])
+def test_renormalized_norms(hip, chi, cd):
+    """The Frobenius normalisation at the edges of its blocks of 256 and on both
+    sides of its one-launch range (64 of them), through the renormalised
+    corners (chi x cd) and edge: unit norms to the rounding of a tree of sums
+    and of one scaling, 20 ulps."""
+    g = np.random.default_rng(chi + cd)
+    dv = lambda *s: torch.as_tensor(g.standard_normal(s), device="cuda")
+    D = 2
+    site = (dv(D, D, D, D, 2), [dv(chi, chi) for _ in range(4)],
+            [dv(chi, chi, D, D) for _ in range(4)])
+    P = [dv(chi * D * D, cd) for _ in range(4)]
+    out = hip.renormalize_boundary(site, 0, *P)
+    for t in out:
+        assert abs(float(torch.linalg.vector_norm(t.cpu())) - 1.0) <= 20 * 2.0 ** -52
