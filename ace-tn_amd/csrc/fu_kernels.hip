@@ -7,6 +7,7 @@
 #include "lanes.h"
 
 #include <algorithm>
+#include <type_traits>
 #include <cmath>
 
 namespace acetn {
@@ -1290,22 +1291,26 @@ void als_solve_device(const double* n12, const double* a12g, double* a1r, double
   const int grp = count > 1 ? 1 : (int)std::min<size_t>(nD, 1 + (150 * 1024 - one) / t1);
   const size_t lds = one + (grp - 1) * t1;
   const int64_t n12_stride = (int64_t)nD * nD * nD * nD;
-  auto launch = [&](auto kernel) {
-    // (set on each call: one kernel a size class, and cheap)
-    ACETN_HIP_CHECK(hipFuncSetAttribute((const void*)kernel,
-                                        hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024));
-    hipLaunchKernelGGL(kernel, dim3(count), dim3(ALS_NT), lds, s, n12, a12g, a1r, a2r, nD, D, d,
+  auto launch = [&](auto rc) {
+    constexpr int RC = decltype(rc)::value;
+    static bool attr = false;
+    if (!attr) {
+      ACETN_HIP_CHECK(hipFuncSetAttribute((const void*)als_kernel<RC>,
+                                          hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024));
+      attr = true;
+    }
+    hipLaunchKernelGGL(als_kernel<RC>, dim3(count), dim3(ALS_NT), lds, s, n12, a12g, a1r, a2r, nD, D, d,
                        niter, tol, eps, gwork, out_cost, out_info, n12_stride,
                        (int64_t)als_work_elems(nD, D, d), grp);
     ACETN_HIP_CHECK(hipGetLastError());
   };
   const int tiles = (nD * D + 15) / 16;
-  if (method == 1) launch(als_kernel<0>);
-  else if (tiles <= 1) launch(als_kernel<1>);
-  else if (tiles <= 2) launch(als_kernel<2>);
-  else if (tiles <= 3) launch(als_kernel<3>);
-  else if (tiles <= 5) launch(als_kernel<5>);
-  else launch(als_kernel<kAlsMaxTiles>);
+  if (method == 1) launch(std::integral_constant<int, 0>{});
+  else if (tiles <= 1) launch(std::integral_constant<int, 1>{});
+  else if (tiles <= 2) launch(std::integral_constant<int, 2>{});
+  else if (tiles <= 3) launch(std::integral_constant<int, 3>{});
+  else if (tiles <= 5) launch(std::integral_constant<int, 5>{});
+  else launch(std::integral_constant<int, kAlsMaxTiles>{});
 }
 
 }  // namespace acetn
