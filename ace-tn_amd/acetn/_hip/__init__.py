@@ -671,8 +671,9 @@ class ProjectorJob:
 
     def _begin(self, trust, mark=False):
         niter, cutoff, seed, stream_id, nspec = self.begin_args
+        self.begun = self.prec | trust  # the matching end takes the same bits
         args = (self.arr, self.k, self.chi, self.p, niter, cutoff, seed, stream_id, self.system,
-                self.svd, self.prec | trust)
+                self.svd, self.begun)
         with torch.cuda.stream(self.stream):
             # zero-filled on the pair's stream, ahead of the kernels that write it
             self.spec = torch.zeros(nspec, dtype=torch.float64, device=self.dev)
@@ -718,8 +719,9 @@ class ProjectorJob:
             P1 = torch.empty(self.rows, n, dtype=torch.float64, device=self.dev)
             P2 = torch.empty(self.rows, n, dtype=torch.float64, device=self.dev)
             check(lib().acetn_hip_projectors_end(
-                self.arr, self.k, self.chi, self.p, self.niter, self.system, self.svd, self.prec,
-                n, ptr(P1), ptr(P2), ptr(self.ws), self.ws.numel(), c_vp(self.stream.cuda_stream)))
+                self.arr, self.k, self.chi, self.p, self.niter, self.system, self.svd,
+                self.begun, n, ptr(P1), ptr(P2), ptr(self.ws), self.ws.numel(),
+                c_vp(self.stream.cuda_stream)))
         return P1, P2
 
 

@@ -181,7 +181,8 @@ const double* orthonormalize(Ctx& c, double* Y, int64_t m, int64_t q, bool steer
     // pass 1: plain with rank guard (Yt -> Y); dropped columns come out zero
     pass(Yt, Y, 0.0, 1e-14, dead, nullptr, false);
   }
-  if (c.trust) {
+  // (the sizing pass goes on: one scratch size and layout with and without it)
+  if (c.trust && c.run) {
     if (c.launch) c.drops.add(any);
     return Y;
   }

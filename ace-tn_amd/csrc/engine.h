@@ -34,7 +34,9 @@ struct Ctx {
   double* take(size_t n) {
     const size_t bytes = ((n * sizeof(double) + 255) / 256) * 256;
     if (!run) { off += bytes; return nullptr; }
-    ACETN_REQUIRE(off + bytes <= cap, "workspace too small");
+    ACETN_REQUIRE(off + bytes <= cap, "workspace too small: " + std::to_string(bytes) +
+                                          " bytes at " + std::to_string(off) + " of " +
+                                          std::to_string(cap));
     double* p = reinterpret_cast<double*>(base + off);
     off += bytes;
     return p;

@@ -107,3 +107,50 @@ def test_boundary_refuses_host_and_non_float64_tensors():
     with pytest.raises(ValueError, match="GPU"):
         _hip.ptr(A)
     assert _hip.ptr(None).value is None
+
+
+def _site(D, C_dim, E_dim):
+    """An acetn_site whose tensors are never read (a call that fails before
+    its first launch)."""
+    from acetn import _hip
+    s = _hip.AcetnSite()
+    s.A, s.D, s.d = 4096, D, 2
+    for k in range(4):
+        s.C[k] = s.E[k] = 4096
+        s.C_dim[k][0], s.C_dim[k][1] = C_dim[k]
+        s.E_dim[k][0], s.E_dim[k][1] = E_dim[k]
+    return s
+
+
+@pytest.mark.parametrize("precision", [0, 1, 0x100, 0x101])
+@pytest.mark.parametrize("D,dims,chi,p", [
+    (3, (51, 3, 9, 1, 1, 6), 23, 9), (1, (1, 4, 41, 12, 2, 15), 36, 1),
+    (2, (1, 25, 24, 1, 52, 5), 21, 9), (4, (4, 19, 4, 1, 3, 2), 39, 7),
+    (2, (20, 20, 20, 20, 20, 20), 20, 2), (6, (144, 144, 144, 144, 144, 144), 144, 2)])
+def test_pair_scratch_does_not_depend_on_trust(D, dims, chi, p, precision):
+    """Both phases of a projector pair carve one workspace, the products'
+    scratch first: begin and end plan the same scratch with and without
+    RF_TRUST.  A workspace of 512 bytes fails at that first buffer, before
+    anything is launched, and the message names its size."""
+    from acetn import _hip
+    lib = _hip.lib()
+    ca, cb, n1, n2, x, n4 = dims
+    s1 = _site(D, [(ca, cb)] * 4, [(cb, n1), (cb, n1), (cb, n1), (n2, ca)])
+    s4 = _site(D, [(x, x)] * 4, [(x, x), (x, x), (n4, x), (x, n2)])
+    arr = (ctypes.POINTER(_hip.AcetnSite) * 4)(*[ctypes.pointer(s) for s in (s1, s1, s1, s4)])
+    buf = ctypes.create_string_buffer(1024)
+    ws = ctypes.cast(buf, ctypes.c_void_p)
+
+    def planned(rc):
+        msg = lib.acetn_hip_last_error().decode()
+        m = re.match(r"workspace too small: (\d+) bytes at 0 of", msg)
+        assert rc != 0 and m, msg
+        return int(m.group(1))
+
+    sizes = set()
+    for bits in (precision, precision | _hip.RF_TRUST):
+        sizes.add(planned(lib.acetn_hip_projectors_begin(
+            arr, 0, chi, p, 2, 0.0, 1, 1, 0, 0, bits, ws, None, ws, 512, None)))
+        sizes.add(planned(lib.acetn_hip_projectors_end(
+            arr, 0, chi, p, 2, 0, 0, bits, 1, ws, ws, ws, 512, None)))
+    assert len(sizes) == 1 and sizes.pop() > 512
