@@ -1308,7 +1308,7 @@ int acetn_hip_projectors_begin_mark(const acetn_site* const sites[4], int k, int
                                     void* mark_event) {
   return guarded([&] {
     check_projector_args(sites, system, svd_type);
-    check_precision(precision);
+    check_precision(precision, true);
     ACETN_REQUIRE(pinned_cD_new, "projectors_begin: null cD target");
     ACETN_REQUIRE(niter >= 0 && niter <= 16, "projectors: niter out of range");
     HalfOut o{nullptr, nullptr, nullptr, pinned_cD_new, 0, spectrum};
@@ -1331,7 +1331,7 @@ int acetn_hip_projectors_end(const acetn_site* const sites[4], int k, int64_t ch
                              size_t ws_bytes, void* stream) {
   return guarded([&] {
     check_projector_args(sites, system, svd_type);
-    check_precision(precision);
+    check_precision(precision, true);
     ACETN_REQUIRE(P1 && P2, "projectors_end: null output");
     HalfOut o{P1, P2, nullptr, nullptr, (int)cD_new, nullptr};
     execute(ws, ws_bytes, stream, [&](Ctx& c) {
@@ -1356,8 +1356,6 @@ int acetn_hip_projectors_begin_graph(const acetn_site* const sites[4], int k, in
     check_precision(precision);
     ACETN_REQUIRE(dev_stream_base && dev_cD_new, "projectors_begin_graph: null device pointer");
     ACETN_REQUIRE(niter >= 0 && niter <= 16, "projectors: niter out of range");
-    ACETN_REQUIRE((precision & ACETN_HIP_RF_TRUST) == 0,
-                  "projectors_begin_graph: nothing reads the count, so RF_TRUST cannot be served");
     HalfOut o{nullptr, nullptr, nullptr, nullptr, 0, spectrum};
     o.stream_base = dev_stream_base;
     o.dev_cD = dev_cD_new;

@@ -133,7 +133,10 @@ inline GemmDesc gdesc(int M, int N, int K, IdxMap am, IdxMap ak, IdxMap bk, IdxM
   return g;
 }
 
-inline void check_precision(int p) {
+// ``trust``: the entry point can report dropped columns (ACETN_HIP_RF_TRUST)
+inline void check_precision(int p, bool trust = false) {
+  ACETN_REQUIRE(trust || (p & ACETN_HIP_RF_TRUST) == 0,
+                "unknown precision mode: RF_TRUST is for projectors_begin and its end only");
   const int base = p & ~(ACETN_HIP_RF_FAST | ACETN_HIP_RF_TRUST);
   ACETN_REQUIRE(base == ACETN_HIP_FP64 || base == ACETN_HIP_MIXED, "unknown precision mode");
 }

@@ -154,3 +154,44 @@ def test_pair_scratch_does_not_depend_on_trust(D, dims, chi, p, precision):
         sizes.add(planned(lib.acetn_hip_projectors_end(
             arr, 0, chi, p, 2, 0, 0, bits, 1, ws, ws, ws, 512, None)))
     assert len(sizes) == 1 and sizes.pop() > 512
+
+
+def test_trust_bit_is_refused_where_no_one_can_start_over():
+    """RF_TRUST is a bit of projectors_begin[_mark] and projectors_end; every
+    other entry point that takes a precision refuses it, before anything else
+    could fail (null outputs and workspaces here)."""
+    from acetn import _hip
+    lib = _hip.lib()
+    s = _site(2, [(4, 4)] * 4, [(4, 4)] * 4)
+    one = ctypes.byref(s)
+    arr = (ctypes.POINTER(_hip.AcetnSite) * 4)(*[ctypes.pointer(s)] * 4)
+    calls = {
+        "quarter_tensor": lambda b: lib.acetn_hip_quarter_tensor(one, 0, b, None, None, 0, None),
+        "half_projectors": lambda b: lib.acetn_hip_half_projectors(
+            one, one, 0, 4, 2, 2, 0.0, 1, 1, b, None, None, None, None, None, 0, None),
+        "half_projectors_begin": lambda b: lib.acetn_hip_half_projectors_begin(
+            one, one, 0, 4, 2, 2, 0.0, 1, 1, b, None, None, None, 0, None),
+        "half_projectors_end": lambda b: lib.acetn_hip_half_projectors_end(
+            one, one, 0, 4, 2, 2, b, 1, None, None, None, 0, None),
+        "projectors_begin_graph": lambda b: lib.acetn_hip_projectors_begin_graph(
+            arr, 0, 4, 2, 2, 0.0, 1, 1, None, 0, 0, b, None, None, None, 0, None),
+        "projectors_end_padded": lambda b: lib.acetn_hip_projectors_end_padded(
+            arr, 0, 4, 2, 2, 0, 0, b, 1, None, None, None, 0, None),
+        "renormalize_boundary": lambda b: lib.acetn_hip_renormalize_boundary(
+            one, 0, None, None, 4, None, None, 4, b, None, None, None, None, 0, None),
+        "renormalize_boundary_part": lambda b: lib.acetn_hip_renormalize_boundary_part(
+            one, 0, 1, 0, None, None, 4, None, None, 4, 4, b, None, None, None, None, 0, None),
+    }
+    for name, call in calls.items():
+        for base in (0, 1, 0x100):
+            assert call(base) != 0
+            assert "precision" not in lib.acetn_hip_last_error().decode(), name
+            assert call(base | _hip.RF_TRUST) != 0
+            assert "precision" in lib.acetn_hip_last_error().decode(), name
+    # the pair's own two calls take it (and fail on what else is missing)
+    for call in (lambda: lib.acetn_hip_projectors_begin(
+                     arr, 0, 4, 2, 2, 0.0, 1, 1, 0, 0, _hip.RF_TRUST, None, None, None, 0, None),
+                 lambda: lib.acetn_hip_projectors_end(
+                     arr, 0, 4, 2, 2, 0, 0, _hip.RF_TRUST, 1, None, None, None, 0, None)):
+        assert call() != 0
+        assert "null" in lib.acetn_hip_last_error().decode()
