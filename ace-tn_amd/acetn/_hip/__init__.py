@@ -628,7 +628,10 @@ class ProjectorJob:
         computed values on the host by the time ``ready`` completes.
         ``trust`` begins the pair without the launches that deal with dropped
         columns (RF_TRUST); should there be any, ``finish`` begins it again
-        with them and waits, so the result is the same either way."""
+        with them and waits (``started_over``), so the result is the same
+        either way.  ``trust`` None: nothing is known of the pair; it is
+        trusted once the boundary has grown to chi, since the spectra of a
+        young one (the default start's D^2 wide) are mostly graded."""
         made = [make_site(*st) for st in sites]
         self.sv = [m[0] for m in made]
         self.keep = [m[1] for m in made]
@@ -667,6 +670,10 @@ class ProjectorJob:
         self.cd_host = torch.zeros(2, dtype=torch.int32, pin_memory=True)
         self.mark = None
         self.begin_args = (niter, cutoff, seed, stream_id, nspec)
+        self.started_over = False
+        if trust is None:
+            trust = all(d >= chi for x in self.sv for e in x.E_dim for d in e)
+        self.trusted = bool(trust)
         self._begin(RF_TRUST if trust else 0, mark)
 
     def _begin(self, trust, mark=False):
@@ -712,6 +719,7 @@ class ProjectorJob:
             return P1, P2
         n = int(self.cd_host[0])
         if n < 0:
+            self.started_over = True
             self._begin(0)
             self.ready.synchronize()
             n = int(self.cd_host[0])

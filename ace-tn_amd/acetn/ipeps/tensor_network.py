@@ -5,6 +5,7 @@ every instance, tensor_network.py:12), each network owns its sites, so
 independent iPEPS instances (e.g. a parameter sweep) can be co-resident."""
 import torch
 
+from ..renormalization.projectors import DropHistory
 from .bond import Bond
 from .site_tensor import SiteTensor
 
@@ -18,6 +19,7 @@ class TensorNetwork:
         self.dtype = dtype
         self.device = device
         self._tensor_network = {}
+        self.drop_history = DropHistory()
         self.setup_tensor_network(tensor_network)
 
     def __getitem__(self, site):
@@ -62,6 +64,7 @@ class TensorNetwork:
             self.load_arrays(read_reference_checkpoint(filename, self.nx, self.ny))
             return
         state = torch.load(filename, weights_only=True)
+        self.drop_history = DropHistory()
         for key, t in state["tensors"].items():
             site = tuple(int(v) for v in key.split(","))
             st = self[site]
@@ -72,6 +75,7 @@ class TensorNetwork:
 
     def load_arrays(self, arrays):
         """Load {site: {'A','C','E'}} of numpy/torch arrays."""
+        self.drop_history = DropHistory()
         for site, t in arrays.items():
             st = self[site]
             st['A'] = torch.as_tensor(t['A'])
@@ -87,6 +91,7 @@ class TensorNetwork:
             self.copy_from(tensor_network)
 
     def initialize_site_tensors(self, site_state_map):
+        self.drop_history = DropHistory()
         self.bond_list = self.build_bond_list()
         self.site_list = self.build_site_list()
         for site in self.site_list:

@@ -9,7 +9,7 @@ from .. import _hip
 
 # s_{q-1} / s_0 at or above which a pair's spectrum counts as not graded
 UNGRADED = 1e-3
-# and from which the range finder is trusted not to drop a column: its Gram
+# and from which the range finder is expected not to drop a column: its Gram
 # matrices see the square of the ratio, the shift of their first pass (1e-9)
 # lifts it, and the rank guard (1e-14) then lies at 2e-6
 TRUSTED = 1e-5
@@ -30,6 +30,42 @@ class SketchCounter:
         return s
 
 
+class DropHistory:
+    """Which pairs of a network to begin without the recovery of dropped
+    columns (RF_TRUST).  Only time hangs on it: a pair that drops one after all
+    is started over, which costs its range finder and SVD a second time.  Kept
+    by the network, as renormalize() makes a calculator per call."""
+
+    def __init__(self):
+        # pair (sites, k, system) -> whether its next computation is trusted
+        self.trusted = {}
+        # pairs that started over and have not been UNGRADED since
+        self.dropped = set()
+        # pairs not to be trusted
+        self.graded = set()
+
+    def trusts(self, key):
+        """True or False, or None where nothing is known: neither of the pair
+        nor of another pair of the network that is not to be trusted."""
+        return self.trusted.get(key, False if self.graded else None)
+
+    def record(self, key, span, trusted, started_over):
+        """A computation that was ``trusted`` and did not start over dropped
+        nothing, so the next one is trusted too; after any other its ``span``
+        s_{q-1} / s_0 decides."""
+        if started_over:
+            self.dropped.add(key)
+        elif span >= UNGRADED:
+            self.dropped.discard(key)
+        if not started_over and (trusted or
+                                 span >= (UNGRADED if key in self.dropped else TRUSTED)):
+            self.trusted[key] = True
+            self.graded.discard(key)
+        else:
+            self.trusted[key] = False
+            self.graded.add(key)
+
+
 class ProjectorCalculator:
     def __init__(self, config, sketch=None):
         self.projectors = config.projectors
@@ -47,8 +83,8 @@ class ProjectorCalculator:
         # pair (sites, k, system) -> its last spectrum was not graded, so the
         # next computation may take the range finder's fast path (RF_FAST)
         self.ungraded = {}
-        # the same pair -> s_{q-1} / s_0 of its last spectrum
-        self.span = {}
+        # for networks that keep none
+        self.drop_history = DropHistory()
         self.set_calculate()
 
     def set_calculate(self):
@@ -99,6 +135,7 @@ class ProjectorCalculator:
         if self.svd_type not in ("rsvd", "full-rank"):
             raise ValueError(f"Invalid svd_type: {self.svd_type}")
         chi = ipeps.dims['chi']
+        history = getattr(ipeps, "drop_history", self.drop_history)
         started = []
         for i, (sites, k) in enumerate(jobs):
             slot = (base + i) % _hip.N_SLOTS if slots is None else slots[i]
@@ -119,8 +156,7 @@ class ProjectorCalculator:
                                     svd=self.svd_type, ws_key=ws_key, graph=graph,
                                     mark=mark,
                                     rf_fast=graph is None and self.ungraded.get(key, False),
-                                    trust=graph is None and
-                                    self.span.get(key, 1.0) >= TRUSTED)
+                                    trust=history.trusts(key) if graph is None else False)
             job.key = key
             started.append(job)
         return started
@@ -146,8 +182,11 @@ class ProjectorCalculator:
                 # the range finder's CholeskyQR keeps every column when the
                 # q values span less than 1e-3 (margin 100 on its rank guard)
                 s0, s1 = float(job.spec_host[0]), float(job.spec_host[-1])
-                self.span[job.key] = s1 / s0 if s0 > 0 else 0.0
                 self.ungraded[job.key] = bool(s0 > 0 and s1 >= UNGRADED * s0)
+                history = getattr(ipeps, "drop_history", self.drop_history)
+                history.record(job.key, s1 / s0 if s0 > 0 else 0.0,
+                               getattr(job, "trusted", False),
+                               getattr(job, "started_over", False))
             # the kept count: a device scalar for a captured pair (written on
             # every replay)
             cd = P1.shape[1] if job.graph is None else job.graph[1][job.graph[2]]

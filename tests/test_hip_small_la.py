@@ -326,3 +326,30 @@ def test_renormalized_norms(hip, chi, cd):
     out = hip.renormalize_boundary(site, 0, *P)
     for t in out:
         assert abs(float(torch.linalg.vector_norm(t.cpu())) - 1.0) <= 20 * 2.0 ** -52
+
+
+@pytest.mark.parametrize("D,chi,projectors,bound", [(2, 4, "half-system", 4), (3, 16, "half-system", 0),
+                                                    (2, 10, "full-system", 0)])
+def test_default_start_is_not_computed_twice(hip, monkeypatch, D, chi, projectors, bound):
+    """From the default start (a boundary of D^2, graded spectra) no pair is
+    begun without the recovery of dropped columns and started over, over
+    several calls of renormalize(); where the boundary is at chi from the
+    first move on, the four pairs begun before anything is known are."""
+    from acetn.ipeps import Ipeps
+    made = []
+    job = hip.ProjectorJob
+
+    class Job(job):
+        def __init__(self, *a, **kw):
+            super().__init__(*a, **kw)
+            made.append(self)
+    monkeypatch.setattr(hip, "ProjectorJob", Job)
+    torch.manual_seed(11)
+    net = Ipeps({"TN": {"nx": 2, "ny": 2, "dims": {"phys": 2, "bond": D, "chi": chi}},
+                 "ctmrg": {"steps": 1, "projectors": projectors, "sketch_seed": 3,
+                           "disable_progressbar": True}})
+    for _ in range(3):
+        net.renormalize()
+    assert len(made) == 3 * 16
+    over = [i for i, j in enumerate(made) if j.started_over]
+    assert len(over) <= bound and all(i < 4 for i in over)

@@ -133,3 +133,65 @@ def test_range_finder_fast_path_follows_the_previous_spectrum(monkeypatch):
     assert run(5e-4) is True      # 2e-3 counts as not graded (>= 1e-3)
     assert run(0.5) is False      # 5e-4 is graded
     assert run(0.5) is True
+
+
+def test_trust_follows_what_is_known_of_the_pair(monkeypatch):
+    """start_many begins a pair without the recovery of dropped columns (trust)
+    as long as it drops none, after that where a spectrum spans less than 1e3,
+    and where the spectrum of one that never dropped any spans less than 1e5;
+    nothing known gives None (the job decides by the boundary's size), but not
+    once another pair of the network is untrusted.  The history is the
+    network's: it outlives the calculator, and another network has its own."""
+    from acetn import _hip
+    from acetn.renormalization import projectors as pj
+    monkeypatch.setattr(torch.cuda, "Event", _Event)
+
+    class FakeJob:
+        def __init__(self, *a, **kw):
+            self.trust, self.graph, self.ready, self.stream = kw["trust"], None, None, None
+            self.spec, self.spec_host = torch.zeros(4), None
+            self.trusted = False
+
+        def finish(self):
+            return torch.zeros(8, 3), torch.zeros(8, 3)
+
+    monkeypatch.setattr(_hip, "ProjectorJob", FakeJob)
+
+    class Cfg:
+        projectors, svd_type, svd_cutoff = "half-system", "rsvd", 1e-12
+        rsvd_niter, rsvd_oversampling = 2, 2
+
+    class Net:
+        def __init__(self):
+            self.dims = {'bond': 2, 'chi': 4}
+            self.drop_history = pj.DropHistory()
+
+        def __getitem__(self, s):
+            return {'A': None, 'C': None, 'E': None}
+    net = Net()
+    sites = [(0, 0), (1, 0), (1, 1), (0, 1)]
+
+    def run(tail, trusted=None, started_over=False, k=0, net=net):
+        """One computation; ``trusted``: what the job made of None."""
+        calc = pj.ProjectorCalculator(Cfg())  # one a call of renormalize()
+        job = calc.start_many(net, [(sites, k)])[0]
+        job.spec_host = torch.tensor([1.0, 0.5, tail], dtype=torch.float64)
+        job.trusted = bool(job.trust if trusted is None else trusted)
+        job.started_over = started_over
+        list(calc.finish_each(net, [job]))
+        return job.trust
+
+    assert run(1e-8, trusted=True) is None         # nothing known
+    assert run(1e-8) is True                       # it dropped nothing, whatever its spectrum
+    assert run(1e-4, k=1) is None                  # nothing known of pair 1, no other untrusted
+    assert run(0.5, started_over=True) is True
+    assert run(0.5, k=2) is False                  # a pair of the network is untrusted
+    assert run(5e-4) is False                      # it started over
+    assert run(2e-3) is False                      # and was still graded then
+    assert run(1e-8) is True                       # 2e-3 is not: forgiven
+    assert run(1e-8, k=1) is True                  # 1e-4, untrusted, spans less than 1e5
+    assert run(5e-6, k=2) is True                  # 0.5 as well
+    other = Net()
+    assert run(5e-6, trusted=False, net=other) is None
+    assert run(2e-5, net=other) is False           # 5e-6 spans more than 1e5
+    assert run(1e-8, net=other) is True
