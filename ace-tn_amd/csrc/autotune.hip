@@ -4,7 +4,8 @@
 // from hand-set thresholds.  With tuning on, the first product of every new
 // shape (kind, M, N, K, operand flags) instead times each candidate (the
 // four tile shapes, each with split-K counts around its default that fit the
-// caller's scratch, and the small FP64 product in its range) on the caller's stream with HIP events, keeps the
+// caller's scratch, and the pipelined and the small FP64 product where they take
+// it) on the caller's stream with HIP events, keeps the
 // fastest, and re-runs it so that the result is the chosen kernel's.  Later
 // products of that shape use the table; a CTMRG iteration repeats the same
 // shapes, so one warmup iteration tunes a whole run.  The table can be saved
@@ -14,6 +15,7 @@
 #include "internal.h"
 
 #include <cstdio>
+#include <cstring>
 #include <map>
 #include <mutex>
 #include <tuple>
@@ -120,7 +122,7 @@ void autotune_save(const char* path) {
   std::lock_guard<std::mutex> g(t.mu);
   FILE* f = std::fopen(path, "w");
   ACETN_REQUIRE(f != nullptr, std::string("autotune: cannot write ") + path);
-  std::fprintf(f, "# acetn gemm tile table: kind M N K flags wm wn ks ms variant\n");
+  std::fprintf(f, "# acetn gemm tile table 2: kind M N K flags wm wn ks ms variant\n");
   for (const auto& kv : t.table) {
     const auto& k = kv.first;
     const TuneChoice& c = kv.second;
@@ -138,8 +140,12 @@ int64_t autotune_load(const char* path) {
   std::lock_guard<std::mutex> g(t.mu);
   char line[256];
   int64_t n = 0;
+  bool old = false;
   while (std::fgets(line, sizeof line, f)) {
-    if (line[0] == '#') continue;
+    if (line[0] == '#') {
+      old |= std::strncmp(line, "# acetn gemm tile table:", 24) == 0;
+      continue;
+    }
     int kind, M, N, K, flags, wm, wn, ks, var = 0;
     double ms = 0.0;
     if (std::sscanf(line, "%d %d %d %d %d %d %d %d %lf %d", &kind, &M, &N, &K, &flags, &wm, &wn,
@@ -147,8 +153,9 @@ int64_t autotune_load(const char* path) {
       continue;
     const bool tile_ok = (wm == 1 && wn == 5) || (wm == 2 && wn == 5) || (wm == 2 && wn == 2) ||
                          (wm == 4 && wn == 4) ||
-                         (kind == 0 && wm == 1 && wn == 1 && ks == 1 && var == 0);
-    // 1 x 1 is the small FP64 product (used where the shape is in its range);
+                         (kind == 0 && wn == 1 && var == 0 && ((wm == 1 && ks == 1) || wm == 4));
+    // 1 x 1 is the small FP64 product, 4 x 1 the pipelined one (used where they
+    // take the product);
     // the wider FP64 variants exist for single-stride products: 2 x 5 tiles
     // in variants 1-3, 1 x 5 tiles in variant 3; two-piece split products
     // have 64-deep k-tiles as variant 1
@@ -156,6 +163,10 @@ int64_t autotune_load(const char* path) {
                                      ((wm == 2 && var <= 3) || (wm == 1 && var == 3))) ||
                         (kind == 2 && var == 1);
     if (!tile_ok || !var_ok || ks < 1 || ks > 64) continue;
+    // a table of the time when the pipelined kernel was no candidate and the key
+    // did not tell who may take it: for the products that may not
+    if (old && kind == 0)
+      flags |= gemm_f64_size_limits(M, N, K, flags >> 1) & ~(wn == 1 ? kTuneNoSmall : 0);
     TuneChoice c{wm, wn, ks, ms};
     c.var = var;
     t.table[std::make_tuple(kind, M, N, K, flags)] = c;

@@ -636,11 +636,14 @@ int pipe_ksplit(const GemmDesc& g) {
 // against 17.6 in two launches, 500^3: 16 against 24, 1600 x 72 x 1600: even, 8000 x
 // 24 x 600: 26 against 19); one that the pipelined kernel takes in one launch
 // stays there (1024 x 1024 x 64: 15.6 us against 16.2).
+bool small_size(int64_t M, int64_t N, int64_t K, int count) {
+  if (K <= 0 || K > SP_MAXK) return false;
+  const int64_t tiles = (M + 15) / 16 * ((N + 15) / 16) * count;
+  return 256.0 * tiles * K < 1.4e8 && tiles <= (K >= 32 ? 4096 : 1024);
+}
 bool small_shape(const GemmDesc& g, int count) {
-  if (!g.pipe || g.K <= 0 || g.K > SP_MAXK) return false;
-  const int64_t tiles = (int64_t)((g.M + 15) / 16) * ((g.N + 15) / 16) * count;
-  if (256.0 * tiles * g.K >= 1.4e8 || tiles > (g.K >= 32 ? 4096 : 1024)) return false;
-  return !pipe_shape(g, count) || pipe_ksplit(g) > 1;
+  return g.pipe && small_size(g.M, g.N, g.K, count) &&
+         (!pipe_shape(g, count) || pipe_ksplit(g) > 1);
 }
 void launch_small(const GemmDesc& g, const GemmBatch& b, hipStream_t s) {
   const dim3 grid((g.N + 15) / 16, (g.M + 15) / 16, b.count);
@@ -656,14 +659,28 @@ void launch_small(const GemmDesc& g, const GemmBatch& b, hipStream_t s) {
 }
 
 template <int WN>
-void launch_pipe(const GemmDesc& g, const double* A, const double* B, double* C, int ks,
-                 double* work, hipStream_t s) {
+void launch_pipe_wn(const GemmDesc& g, const GemmBatch& b, int ks, double* work, hipStream_t s) {
   const dim3 grid((g.N + 16 * WN - 1) / (16 * WN), (g.M + PP_BM - 1) / PP_BM, ks);
   ACETN_REQUIRE(grid.y <= 65535 && grid.z <= 65535, "gemm_f64: grid too large");
   if (g.am.s0 == 1 && g.ak.s0 != 1)
-    hipLaunchKernelGGL((gemm_f64_pipe_kernel<WN, true>), grid, dim3(PP_NT), 0, s, g, A, B, C, ks, work);
+    hipLaunchKernelGGL((gemm_f64_pipe_kernel<WN, true>), grid, dim3(PP_NT), 0, s, g, b.A[0], b.B[0],
+                       b.C[0], ks, work);
   else
-    hipLaunchKernelGGL((gemm_f64_pipe_kernel<WN, false>), grid, dim3(PP_NT), 0, s, g, A, B, C, ks, work);
+    hipLaunchKernelGGL((gemm_f64_pipe_kernel<WN, false>), grid, dim3(PP_NT), 0, s, g, b.A[0], b.B[0],
+                       b.C[0], ks, work);
+}
+void launch_pipe(const GemmDesc& g, const GemmBatch& b, int ks, double* work, hipStream_t s) {
+  switch (pipe_wn(g)) {
+    case 2: launch_pipe_wn<2>(g, b, ks, work, s); break;
+    case 3: launch_pipe_wn<3>(g, b, ks, work, s); break;
+    case 4: launch_pipe_wn<4>(g, b, ks, work, s); break;
+    case 5: launch_pipe_wn<5>(g, b, ks, work, s); break;
+    case 6: launch_pipe_wn<6>(g, b, ks, work, s); break;
+    case 7: launch_pipe_wn<7>(g, b, ks, work, s); break;
+    case 8: launch_pipe_wn<8>(g, b, ks, work, s); break;
+    case 9: launch_pipe_wn<9>(g, b, ks, work, s); break;
+    default: launch_pipe_wn<10>(g, b, ks, work, s); break;
+  }
 }
 
 // Small-output, long-K products (M, N <= 8, e.g. the d^2 x d^2 reduced
@@ -813,6 +830,11 @@ bool gemm_f64_large(int64_t M, int64_t N, int64_t K) {
   return M >= 96 && N >= 17 && K >= 32 && (double)M * N * K >= 5e7;
 }
 
+int gemm_f64_size_limits(int64_t M, int64_t N, int64_t K, int count) {
+  return (count == 1 && gemm_f64_large(M, N, K) ? kTuneNoPipe : 0) |
+         (small_size(M, N, K, count) ? kTuneNoSmall : 0);
+}
+
 size_t gemm_f64_work_elems(const GemmDesc& g, int count) {
   if (dot_small_fits(g)) return (size_t)dot_small_wgs(g) * count * kDotMax * kDotMax;
   int ks = choose_ksplit(g, count);
@@ -847,7 +869,8 @@ void gemm_f64(const GemmDesc& g, const GemmBatch& b, double* work, size_t work_e
   const bool lin = g.am.n0 <= 0 && g.ak.n0 <= 0 && g.bk.n0 <= 0 && g.bn.n0 <= 0;
   auto launch_choice = [&](const TuneChoice& c) {
     hipEvent_t e0 = kernel_timing_begin(s);
-    if (c.wn == 1) launch_small(g, b, s);
+    if (c.wn == 1 && c.wm == 1) launch_small(g, b, s);
+    else if (c.wn == 1) launch_pipe(g, b, c.ks, work, s);
     else if (c.wm == 2 && c.wn == 5 && lin && c.var == 1) launch_gemm_wide<2, 4, 16>(g, b, c.ks, work, s);
     else if (c.wm == 2 && c.wn == 5 && lin && c.var == 2) launch_gemm_wide<2, 2, 32>(g, b, c.ks, work, s);
     else if (c.wm == 2 && c.wn == 5 && lin && c.var == 3) launch_gemm_wide<2, 4, 32>(g, b, c.ks, work, s);
@@ -867,40 +890,25 @@ void gemm_f64(const GemmDesc& g, const GemmBatch& b, double* work, size_t work_e
       ACETN_HIP_CHECK(hipGetLastError());
     }
   };
-  const TuneKey key{0, g.M, g.N, g.K, (lin ? 1 : 0) | (b.count << 1)};
-  TuneChoice listed;
+  // A table entry holds for the products with its candidates: the sizes say
+  // which of the pipelined and the small kernel there may be, the key which of
+  // them this product may not take (order of sums, operand layout, alignment).
   const bool small = small_shape(g, b.count);
-  const bool in_table = autotune_lookup(key, &listed) && fits(listed.ks) &&
-                        (listed.var == 0 || lin) && (small || listed.wn != 1);
-  if (!in_table && !small && pipe_shape(g, b.count) && aligned16(b.A[0]) && aligned16(b.B[0])) {
-    const int ks = pipe_ksplit(g);
-    if (ks == 1 || (work != nullptr && work_elems >= (size_t)ks * g.M * g.N)) {
-      hipEvent_t e0 = kernel_timing_begin(s);
-      switch (pipe_wn(g)) {
-        case 2: launch_pipe<2>(g, b.A[0], b.B[0], b.C[0], ks, work, s); break;
-        case 3: launch_pipe<3>(g, b.A[0], b.B[0], b.C[0], ks, work, s); break;
-        case 4: launch_pipe<4>(g, b.A[0], b.B[0], b.C[0], ks, work, s); break;
-        case 5: launch_pipe<5>(g, b.A[0], b.B[0], b.C[0], ks, work, s); break;
-        case 6: launch_pipe<6>(g, b.A[0], b.B[0], b.C[0], ks, work, s); break;
-        case 7: launch_pipe<7>(g, b.A[0], b.B[0], b.C[0], ks, work, s); break;
-        case 8: launch_pipe<8>(g, b.A[0], b.B[0], b.C[0], ks, work, s); break;
-        case 9: launch_pipe<9>(g, b.A[0], b.B[0], b.C[0], ks, work, s); break;
-        default: launch_pipe<10>(g, b.A[0], b.B[0], b.C[0], ks, work, s); break;
-      }
-      ACETN_HIP_CHECK(hipGetLastError());
-      kernel_timing_end(e0, s, kKGemmF64, 2.0 * g.M * g.N * (double)g.K,
-                        8.0 * ((double)g.M * g.K + (double)g.K * g.N + (double)g.M * g.N));
-      if (ks > 1) {
-        const int blocks = (int)std::min<int64_t>(((int64_t)g.M * g.N + 255) / 256, 2048);
-        hipLaunchKernelGGL(splitk_reduce_kernel, dim3(blocks, 1), dim3(256), 0, s, g, b, ks, work);
-        ACETN_HIP_CHECK(hipGetLastError());
-      }
-      return;
-    }
-  }
-  if (autotune_should_tune(key, g, s)) {
+  const bool pipe = pipe_shape(g, b.count) && aligned16(b.A[0]) && aligned16(b.B[0]);
+  const int limits = gemm_f64_size_limits(g.M, g.N, g.K, b.count) &
+                     ~((pipe ? kTuneNoPipe : 0) | (small ? kTuneNoSmall : 0));
+  const TuneKey key{0, g.M, g.N, g.K, (lin ? 1 : 0) | (b.count << 1) | limits};
+  TuneChoice ch;
+  const bool listed = autotune_lookup(key, &ch) && fits(ch.ks) && (ch.var == 0 || lin) &&
+                      (ch.wn != 1 || (ch.wm == 1 ? small : pipe));
+  if (!listed && autotune_should_tune(key, g, s)) {
     std::vector<TuneChoice> cands;
     if (small) cands.push_back(TuneChoice{1, 1, 1});
+    if (pipe) {
+      const int h = pipe_ksplit(g);
+      for (int k = 1; k <= h; k += std::max(1, h - 1))
+        if (fits(k)) cands.push_back(TuneChoice{4, 1, k});
+    }
     const Tile tiles[8] = {{1, 5},    {2, 5},    {2, 2},    {4, 4},
                            {2, 5, 1}, {2, 5, 2}, {2, 5, 3}, {1, 5, 3}};
     for (const Tile& t : tiles) {
@@ -921,12 +929,14 @@ void gemm_f64(const GemmDesc& g, const GemmBatch& b, double* work, size_t work_e
     autotune_run(key, cands, s, launch_choice);
     return;
   }
-  int ks = choose_ksplit(g, b.count);
-  if (!fits(ks)) ks = 1;
-  const Tile t = choose_tile(g);
-  TuneChoice ch{t.wm, t.wn, ks};
-  if (small) ch = TuneChoice{1, 1, 1};
-  if (in_table) ch = listed;
+  if (!listed) {
+    const Tile t = choose_tile(g);
+    const int ks = choose_ksplit(g, b.count);
+    ch = TuneChoice{t.wm, t.wn, fits(ks) ? ks : 1};
+    const int parts = pipe && !small ? pipe_ksplit(g) : 0;
+    if (small) ch = TuneChoice{1, 1, 1};
+    else if (parts > 0 && fits(parts)) ch = TuneChoice{4, 1, parts};
+  }
   launch_choice(ch);
 }
 

@@ -149,13 +149,19 @@ void gemm_split_planar(const GemmDesc& g, const SplitPlanes& A, const double* B,
 struct TuneKey {
   int kind, M, N, K, flags;
 };
+// flags of an FP64 product whose sizes the pipelined / the small kernel takes,
+// but whose order of sums, layout or alignment it does not
+constexpr int kTuneNoPipe = 1 << 16, kTuneNoSmall = 1 << 17;
+// both, as far as the sizes go (what the kernels older tables know do)
+int gemm_f64_size_limits(int64_t M, int64_t N, int64_t K, int count);
 struct TuneChoice {
   int wm, wn, ks;
   double ms = 0.0;
   // FP64 kernel variant: 0 four waves (2 x 2) with k-tiles of 16, 1 eight
   // waves (4 x 2) with k-tiles of 16, 2 four waves with k-tiles of 32,
   // 3 eight waves with k-tiles of 32 (the split-bf16 kernels have one);
-  // the workgroup tile is (16 wm waves_m) x (32 wn)
+  // the workgroup tile is (16 wm waves_m) x (32 wn).  wn = 1: the FP64 kernels
+  // of other layouts, wm = 1 the small, wm = 4 the pipelined one
   int var = 0;
 };
 void autotune_set_mode(int mode);  // 0 thresholds, 1 tune new shapes, 2 table only

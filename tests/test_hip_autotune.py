@@ -139,3 +139,64 @@ def test_deep_k_tile_split_variant(hip, tmp_path, wm):
             assert np.array_equal(out[0], out[1])
         else:
             np.testing.assert_allclose(out[1], out[0], rtol=0, atol=tol)
+
+
+# a large product that the pipelined kernel takes, and one in the small kernel's range
+NEW_KERNELS = [(1040, 146, 1100), (320, 48, 400)]
+
+
+@pytest.mark.parametrize("M,N,K", NEW_KERNELS)
+def test_older_tables_leave_the_newer_kernels_in_place(hip, tmp_path, M, N, K):
+    """A table saved before the pipelined kernel was a candidate (its header
+    has no version) says nothing about the products that kernel and the small
+    one take: same bits as with the thresholds; the same line in a current
+    table is followed (64 x 64 tiles sum in another order)."""
+    rng = np.random.default_rng(K)
+    A, B = dev(rng.standard_normal((M, K))), dev(rng.standard_normal((K, N)))
+    off = hip.gemm(A, B)
+    for version, same in ((":", True), (" 2:", False)):
+        path = os.path.join(tmp_path, "t.txt")
+        with open(path, "w") as f:
+            f.write(f"# acetn gemm tile table{version} kind M N K flags wm wn ks ms variant\n"
+                    f"0 {M} {N} {K} 3 2 2 1 0.0 0\n")
+        hip.autotune_clear()
+        assert hip.autotune_load(path) == 1
+        hip.autotune("table")
+        assert torch.equal(hip.gemm(A, B), off) is same
+
+
+def test_tuned_choice_is_for_products_with_the_same_candidates(hip, tmp_path):
+    """A product tuned where the pipelined kernel may not take it (an operand
+    off its alignment) leaves the choice for the aligned one of the same
+    shape alone; tuned itself, that one's entry survives save and load, the
+    pipelined kernel's own choice among them."""
+    rng = np.random.default_rng(8)
+    M, N, K = 1040, 146, 1100
+    A, B = dev(rng.standard_normal((M, K))), dev(rng.standard_normal((K, N)))
+    off = hip.gemm(A, B)
+    odd = torch.empty(M * K + 1, dtype=torch.float64, device="cuda")[1:].view(M, K)
+    odd.copy_(A)
+    hip.autotune("tune")
+    hip.gemm(odd, B)
+    assert hip.autotune_entries() == 1
+    hip.autotune("table")
+    assert torch.equal(hip.gemm(A, B), off)
+    hip.autotune("tune")
+    tuned = hip.gemm(A, B)
+    assert hip.autotune_entries() == 2
+    np.testing.assert_allclose(tuned.cpu().numpy(), off.cpu().numpy(), rtol=0,
+                               atol=1e-12 * float(off.abs().max()))
+    path = os.path.join(tmp_path, "t.txt")
+    hip.autotune_save(path)
+    hip.autotune_clear()
+    assert hip.autotune_load(path) == 2
+    hip.autotune("table")
+    assert torch.equal(hip.gemm(A, B), tuned)
+    with open(path, "w") as f:
+        f.write(f"0 {M} {N} {K} 3 4 1 2 0.0 0\n")   # the pipelined kernel in two k parts
+    hip.autotune_clear()
+    assert hip.autotune_load(path) == 1
+    two = hip.gemm(A, B)
+    exact = A.cpu().numpy() @ B.cpu().numpy()
+    np.testing.assert_allclose(two.cpu().numpy(), exact, rtol=0, atol=1e-12 * np.abs(exact).max())
+    assert torch.equal(hip.gemm(odd, B), hip.gemm(odd, B))   # not followed there: another key
