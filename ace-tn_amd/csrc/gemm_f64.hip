@@ -400,13 +400,23 @@ __global__ __launch_bounds__(PP_NT, 2) void gemm_f64_pipe_kernel(GemmDesc g, con
       *reinterpret_cast<pd2*>(&sB[st & 1][bx[i - 2] * LDB + 2 * by[i - 2]]) = r.b[i - 2];
       return;
     }
-    const int k = kbeg + st * PP_BK + (AM ? ax[i] : 2 * ay[i]);
     const int at = AM ? ax[i] * LDA + 2 * ay[i] : ax[i] * PP_BK + 2 * (ay[i] ^ (ax[i] & 7));
-    pd2 v = r.a[i];
-    // past the last k (B's rows are repeated there)
-    if (k >= kend) v.x = 0.0;
-    if (AM ? k >= kend : k + 1 >= kend) v.y = 0.0;
-    *reinterpret_cast<pd2*>(&sA[st & 1][at]) = v;
+    *reinterpret_cast<pd2*>(&sA[st & 1][at]) = r.a[i];
+  };
+  // zeros past the last k, in both operands (what was loaded there may be
+  // infinite): a branch that only a ragged last k-tile takes
+  auto zero_past_end = [&](int st, Regs& r) {
+    const int k0 = kbeg + st * PP_BK;
+    if (k0 + PP_BK <= kend) return;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int k = k0 + (AM ? ax[i] : 2 * ay[i]);
+      if (k >= kend) r.a[i].x = 0.0;
+      if (AM ? k >= kend : k + 1 >= kend) r.a[i].y = 0.0;
+    }
+#pragma unroll
+    for (int i = 0; i < NB; ++i)
+      if (k0 + bx[i] >= kend) r.b[i] = pd2{0.0, 0.0};
   };
   d4 acc[WN];
 #pragma unroll
@@ -437,6 +447,7 @@ __global__ __launch_bounds__(PP_NT, 2) void gemm_f64_pipe_kernel(GemmDesc g, con
 #pragma unroll
       for (int i = 0; i < NP; ++i) load(1, r1, i);
     }
+    zero_past_end(0, r0);
 #pragma unroll
     for (int i = 0; i < NP; ++i) store(0, r0, i);
     if (nst > 2) {
@@ -455,6 +466,7 @@ __global__ __launch_bounds__(PP_NT, 2) void gemm_f64_pipe_kernel(GemmDesc g, con
   auto tile = [&](int st, Regs& next) {
     const int buf = st & 1;
     if (st + 1 < nst) {
+      zero_past_end(st + 1, next);
 #pragma unroll
       for (int i = 0; i < NP; ++i) store(st + 1, next, i);
     }

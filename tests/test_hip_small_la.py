@@ -353,3 +353,25 @@ def test_default_start_is_not_computed_twice(hip, monkeypatch, D, chi, projector
     assert len(made) == 3 * 16
     over = [i for i, j in enumerate(made) if j.started_over]
     assert len(over) <= bound and all(i < 4 for i in over)
+
+
+@pytest.mark.parametrize("ta", [False, True])
+@pytest.mark.parametrize("M,N,K", [(1040, 146, 1100), (5184, 146, 1234), (96, 50, 32838),
+                                   (320, 48, 410)])
+def test_gemm_keeps_infinities_where_they_belong(hip, M, N, K, ta):
+    """An infinity in the last row of B (the one next to the padding of the last
+    k-tile) makes its column infinite with the signs of A's last column, not
+    undefined, and reaches no other; likewise one in A."""
+    g = np.random.default_rng(K)
+    A, B = g.standard_normal((M, K)), g.standard_normal((K, N))
+    dv = lambda t: torch.as_tensor(np.ascontiguousarray(t), device="cuda")
+    run = lambda a, b: hip.gemm(dv(a.T if ta else a), dv(b), ta=ta).cpu().numpy()
+    Bi, Ai = B.copy(), A.copy()
+    Bi[K - 1, N - 1] = np.inf
+    C = run(A, Bi)
+    assert np.array_equal(C[:, N - 1], np.sign(A[:, K - 1]) * np.inf)
+    assert np.isfinite(C[:, :N - 1]).all()
+    Ai[M - 1, K - 1] = -np.inf
+    C = run(Ai, B)
+    assert np.array_equal(C[M - 1], np.sign(B[K - 1]) * -np.inf)
+    assert np.isfinite(C[:M - 1]).all()
