@@ -1,7 +1,7 @@
-// Approximate eigenvectors of a symmetric FP64 matrix (q <= kTridiagMaxQ) through its
+// Approximate eigenvectors of a symmetric FP64 matrix (32 < q <= kTridiagMaxQ) through its
 // tridiagonal form: what the projector SVD is preconditioned with.
 //   * Householder tridiagonalisation, one workgroup: the whole matrix in
-//     registers up to q = 160, read from L2 in panels above;
+//     registers up to q = 192, read from L2 in panels above;
 //   * one wave per eigenpair, all over the chip: its eigenvalue by 64-way
 //     multisection on the Sturm count, its vector by two steps of inverse
 //     iteration from a random start, and the Householder reflectors applied to
@@ -314,6 +314,9 @@ __global__ __launch_bounds__(64 * TG_NW) void tridiag_glb_kernel(
 // Padding up to a multiple of eight: diagonal entries far above the spectrum,
 // not coupled, which add no eigenvalue below any shift and solve to zero.
 // --------------------------------------------------------------------------
+// uniform in (-1, 1): an xorshift-multiply mix of both numbers, with two prime
+// multipliers of xxHash and the rounds of Wellons' hash-prospector [15 2c1b3c6d
+// 12 297a2d39 15]
 __device__ __forceinline__ double hash_uniform(unsigned a, unsigned b) {
   unsigned h = a * 0x9E3779B1u ^ (b + 0x7F4A7C15u) * 0x85EBCA77u;
   h ^= h >> 15; h *= 0x2C1B3C6Du;
@@ -636,7 +639,7 @@ size_t tridiag_scratch_elems(int q) {
 
 void tridiag_vectors(const double* G, double* X, double* lam, int q, double* scratch,
                      hipStream_t s) {
-  ACETN_REQUIRE(q >= 1 && q <= kTridiagMaxQ, "tridiag_vectors: q out of range");
+  ACETN_REQUIRE(q > 32 && q <= kTridiagMaxQ, "tridiag_vectors: q out of range");
   double* U = scratch;
   double* tau = U + (size_t)q * q;
   double* d = tau + q;
@@ -645,7 +648,6 @@ void tridiag_vectors(const double* G, double* X, double* lam, int q, double* scr
 #define ACETN_TR(NB) \
   hipLaunchKernelGGL(tridiag_reg_kernel<NB>, dim3(1), dim3(TR_NT), 0, s, G, q, U, tau, d, e)
     switch ((q + 31) / 32) {
-      case 1: ACETN_TR(1); break;
       case 2: ACETN_TR(2); break;
       case 3: ACETN_TR(3); break;
       case 4: ACETN_TR(4); break;
@@ -655,10 +657,15 @@ void tridiag_vectors(const double* G, double* X, double* lam, int q, double* scr
 #undef ACETN_TR
   } else {
     const size_t lds = sizeof(double) * tridiag_ld(q) * (2 * kTgNB + TG_NW / 2 + 1);
-    static_assert(sizeof(double) * kTridiagMaxQ * (2 * kTgNB + TG_NW / 2 + 1) <= 156 * 1024,
+    constexpr size_t most = sizeof(double) * kTridiagMaxQ * (2 * kTgNB + TG_NW / 2 + 1);
+    static_assert(kTridiagMaxQ % 16 == 0 && most <= 156 * 1024,
                   "the panel of the largest matrix has to fit the LDS");
-    ACETN_HIP_CHECK(hipFuncSetAttribute((const void*)tridiag_glb_kernel,
-                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    static bool attr = false;
+    if (!attr) {
+      ACETN_HIP_CHECK(hipFuncSetAttribute((const void*)tridiag_glb_kernel,
+                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)most));
+      attr = true;
+    }
     hipLaunchKernelGGL(tridiag_glb_kernel, dim3(1), dim3(64 * TG_NW), lds, s, G, q, e + q, U, tau,
                        d, e);
   }

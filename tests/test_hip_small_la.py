@@ -375,3 +375,12 @@ def test_gemm_keeps_infinities_where_they_belong(hip, M, N, K, ta):
     C = run(Ai, B)
     assert np.array_equal(C[M - 1], np.sign(B[K - 1]) * -np.inf)
     assert np.isfinite(C[:M - 1]).all()
+
+
+@pytest.mark.parametrize("case", ["separate", "triples", "clusters", "graded"])
+@pytest.mark.parametrize("q", [47, 48, 64, 97, 128, 129, 161, 192, 385, 448, 449, 464, 465])
+def test_gram_svd_dispatch_lines(hip, q, case):
+    """The same at the lines of the tridiagonal route (48 to 464), of its
+    register kernel (192) and of its kernels by 32 and by 64 columns, those of
+    the largest sizes among them."""
+    test_gram_svd_spectra(hip, q, case)
