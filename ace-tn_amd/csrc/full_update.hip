@@ -404,14 +404,12 @@ using namespace acetn;
 
 namespace {
 
-// Scratch of acetn_hip_als_solve_noalloc: room for the system of the largest
-// problem it accepts (nD * D <= 128 rows, d <= 4; the elimination now keeps it in
-// registers and LDS), then the final cost and the sweep / flag words.  One copy
-// per device, held until the process ends; the kernel writes every element it
+// Scratch of acetn_hip_als_solve_noalloc: the final cost, then the sweep and flag
+// words (the elimination keeps its system in registers and LDS).  One copy per
+// device, held until the process ends; the kernel writes every element it
 // reads, so nothing has to start at zero.
-constexpr int kNoAllocMaxNR = 128;
-constexpr size_t kNoAllocWork = (size_t)kNoAllocMaxNR * kNoAllocMaxNR + (size_t)kNoAllocMaxNR * 4;
-constexpr size_t kNoAllocElems = kNoAllocWork + 4 + 4;
+constexpr int kNoAllocMaxNR = 128;  // rows of the largest problem it accepts
+constexpr size_t kNoAllocElems = 4 + 4;
 __device__ __align__(256) double scratch[kNoAllocElems];
 
 // the device address of ``scratch`` on each device, looked up once per
@@ -660,16 +658,13 @@ int acetn_hip_als_solve_noalloc(const double* n12, const double* a12g, double* a
                   "the device");
     ACETN_REQUIRE(niter >= 0, "als_solve_noalloc: negative niter");
     ACETN_REQUIRE(f.nD * f.D <= kNoAllocMaxNR && f.d <= 4,
-                  "als_solve_noalloc: nD * D must be at most 128 (the fixed scratch holds the "
-                  "system of D = 8, d = 2); use acetn_hip_als_solve for larger bonds");
-    ACETN_REQUIRE(als_work_elems((int)f.nD, (int)f.D, (int)f.d) <= kNoAllocWork,
-                  "als_solve_noalloc: problem exceeds the fixed scratch");
+                  "als_solve_noalloc: nD * D must be at most 128 (that of D = 8, d = 2) and d at "
+                  "most 4; use acetn_hip_als_solve for larger bonds");
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-    double* base = noalloc_scratch();
-    double* cost = base + kNoAllocWork;
-    int* info = reinterpret_cast<int*>(base + kNoAllocWork + 4);
-    als_solve_device(n12, a12g, a1r, a2r, (int)f.nD, (int)f.D, (int)f.d, niter, tol, epsilon, base,
-                     cost, info, st);
+    double* cost = noalloc_scratch();
+    int* info = reinterpret_cast<int*>(cost + 4);
+    als_solve_device(n12, a12g, a1r, a2r, (int)f.nD, (int)f.D, (int)f.d, niter, tol, epsilon,
+                     nullptr, cost, info, st);
     double hc = 0.0;
     int hi[2] = {0, 0};
     ACETN_HIP_CHECK(hipMemcpyAsync(&hc, cost, sizeof(double), hipMemcpyDeviceToHost, st));

@@ -391,10 +391,10 @@ int acetn_hip_als_solve_batch(const double* n12, const double* a12g, double* a1r
 /* acetn_hip_als_solve without a workspace argument, for callers that cannot
  * allocate device memory (code under stream capture, tight serving loops,
  * harnesses that forbid hipMalloc).  No counterpart in the reference.  Its
- * scratch is a fixed device array of the library (about 133 KB per device,
- * held until the process ends) sized for nD * D <= 128 (D = 8 at d = 2);
- * larger bonds return an error.  Calls that overlap on one device share that
- * array and race: serialise them. */
+ * results pass through a fixed device array of the library (64 bytes per
+ * device, held until the process ends).  Bonds above nD * D = 128 (that of D = 8
+ * at d = 2) or d = 4 return an error.  Calls that overlap on one device share
+ * that array and race: serialise them. */
 int acetn_hip_als_solve_noalloc(const double* n12, const double* a12g, double* a1r, double* a2r,
                                 int64_t nD, int64_t D, int64_t d, int niter, double tol,
                                 int method, double epsilon, int64_t* host_sweeps,
