@@ -384,3 +384,30 @@ def test_gram_svd_dispatch_lines(hip, q, case):
     register kernel (192) and of its kernels by 32 and by 64 columns, those of
     the largest sizes among them."""
     test_gram_svd_spectra(hip, q, case)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("D", [1, 2, 3, 4, 5, 6, 7, 8])
+def test_double_layer_absolute_values(hip, D, precision):
+    """The enlarged corner itself, no scale fitted: the engine applies none.  The
+    same bound as test_double_layer_shapes, through the oracle's corner times
+    the largest element that it divides by."""
+    from oracle import ctmrg as oc
+    rng = np.random.default_rng(D)
+    chi = 5
+    site = {"A": rng.standard_normal((D, D, D, D, 2)),
+            "C": [rng.standard_normal((chi, chi)) for _ in range(4)],
+            "E": [rng.standard_normal((chi, chi, D, D)) for _ in range(4)]}
+
+    def corner(s):
+        a = oc.bond_permute(s["A"], 1)
+        q = oc.ein("acuU,ealL->cuUelL", oc.ein("ab,bcuU->acuU", s["C"][1], s["E"][1]), s["E"][0])
+        q = oc.ein("lurdp,cuelRDp->crRedD", a, oc.ein("cuUelL,LURDp->cuelRDp", q, a))
+        return q.reshape(chi * D * D, -1)
+    dv = lambda t: torch.as_tensor(t, device="cuda")
+    got = hip.quarter_tensor((dv(site["A"]), [dv(t) for t in site["C"]],
+                              [dv(t) for t in site["E"]]), 1, precision=precision).cpu().numpy()
+    ref = corner(site)
+    mag = corner({k: np.abs(v) if k == "A" else [np.abs(t) for t in v] for k, v in site.items()})
+    ulp = 2.0 ** -52 if precision == "fp64" else 2.0 ** -23
+    assert np.all(np.abs(got - ref) <= 2 * ulp * (2 * chi + 2 * D ** 4) * mag)
