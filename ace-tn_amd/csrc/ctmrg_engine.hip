@@ -139,8 +139,9 @@ constexpr int kRecoverLevels = 3;
 
 // Sketch width from which the projector SVD is preconditioned through the
 // tridiagonal form: its twenty launches cost a small matrix more than the two
-// Jacobi solves take (one iteration at D=2, chi=20, q = 22: 8.3 ms with the
-// line at 17, 6.6 ms with it here; full-system D=3, chi=35: 22.2 and 20.5 ms).
+// Jacobi solves take (one iteration at D=2, chi=20, q = 22: 7.8 ms with the
+// line at 17, 6.8 ms with it here; at D=3 8.4 and 7.6 ms at chi=32, 8.5 and 7.6
+// at chi=45, q = 47, 14.0 and 12.4 ms full-system at chi=35).
 constexpr int kTridiagMinQ = 48;
 
 const double* orthonormalize(Ctx& c, double* Y, int64_t m, int64_t q, bool steer = false) {
@@ -198,7 +199,9 @@ const double* orthonormalize(Ctx& c, double* Y, int64_t m, int64_t q, bool steer
   // pass-1 ones), ``next`` receives those a level leaves dropped
   int* prev = dead;
   int* next = flags_a;
-  for (int level = 0; level < kRecoverLevels; ++level) {
+  // (the sizing pass sees one level: the others have the same products)
+  const int levels = c.run ? kRecoverLevels : 1;
+  for (int level = 0; level < levels; ++level) {
     const int* on = c.launch ? prev + q : nullptr;
     // the dropped columns (of the pass-0 output, then of the previous
     // level's residual), projected onto the complement of the columns Y
