@@ -5,8 +5,9 @@
 // shape (kind, M, N, K, operand flags) instead times each candidate (the
 // four tile shapes, each with split-K counts around its default that fit the
 // caller's scratch, and the pipelined and the small FP64 product where they take
-// it) on the caller's stream with HIP events, keeps the
-// fastest, and re-runs it so that the result is the chosen kernel's.  Later
+// it) on the caller's stream with HIP events, keeps the fastest (the pipelined
+// one unless another is 5 % faster), and re-runs it so that the result is the
+// chosen kernel's.  Later
 // products of that shape use the table; a CTMRG iteration repeats the same
 // shapes, so one warmup iteration tunes a whole run.  The table can be saved
 // to and loaded from a text file.  Tuning is skipped under stream capture
@@ -70,7 +71,7 @@ bool autotune_should_tune(const TuneKey& k, const GemmDesc& g, hipStream_t s) {
 }
 
 TuneChoice autotune_run(const TuneKey& k, const std::vector<TuneChoice>& cands, hipStream_t s,
-                        const std::function<void(const TuneChoice&)>& launch) {
+                        const std::function<void(const TuneChoice&)>& launch, float lead) {
   ACETN_REQUIRE(!cands.empty(), "autotune: no candidate");
   hipEvent_t e0 = nullptr, e1 = nullptr;
   ACETN_HIP_CHECK(hipEventCreate(&e0));
@@ -86,7 +87,7 @@ TuneChoice autotune_run(const TuneKey& k, const std::vector<TuneChoice>& cands, 
     ACETN_HIP_CHECK(hipEventSynchronize(e1));
     float ms = 0.f;
     ACETN_HIP_CHECK(hipEventElapsedTime(&ms, e0, e1));
-    if (i == 0 || ms < best) {
+    if (i == 0 || ms < (bi == 0 ? best * lead : best)) {
       best = ms;
       bi = i;
     }

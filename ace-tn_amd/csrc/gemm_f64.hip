@@ -327,7 +327,7 @@ __global__ void splitk_reduce_kernel(GemmDesc g, GemmBatch bt, int ksplit,
 //     empty.
 // Measured with the reduction of the parts, back to back, against the 64- and
 // 128-row tiles of gemm_f64_kernel: 5184 x 146 x 5184 (the range finder at
-// D=6, chi=144) 205 us against 295 (its matrix-core floor is 110 us at 72
+// D=6, chi=144) 200 us against 295 (its matrix-core floor is 110 us at 72
 // TFLOP/s: power holds the clock near 2.2 GHz, and the operands' way in costs
 // the rest), 2500 x 102 x 2500 47 against 74, 2592 x 74 x 2592 37 against 41,
 // 1024 x 66 x 1024 17 against 20.
@@ -619,7 +619,8 @@ int pipe_wn(const GemmDesc& g) {
 }
 // k parts: the fewest estimated microseconds of rounds of workgroups (two a CU,
 // 512 WN clocks a k-tile for the pair) and of the partial sums' way through
-// memory (about 4 TB/s, written and read).
+// memory (about 4 TB/s, written and read).  Only the proportions matter, so the
+// clock is the nominal 2.4 GHz, not the 2.2 that power leaves.
 int pipe_ksplit(const GemmDesc& g) {
   const int wn = pipe_wn(g), kt = (g.K + PP_BK - 1) / PP_BK;
   const int64_t tiles = (int64_t)((g.M + PP_BM - 1) / PP_BM) * ((g.N + 16 * wn - 1) / (16 * wn));
@@ -914,13 +915,19 @@ void gemm_f64(const GemmDesc& g, const GemmBatch& b, double* work, size_t work_e
   const bool listed = autotune_lookup(key, &ch) && fits(ch.ks) && (ch.var == 0 || lin) &&
                       (ch.wn != 1 || (ch.wm == 1 ? small : pipe));
   if (!listed && autotune_should_tune(key, g, s)) {
+    // The pipelined kernel leads: a tile that beats it by a few percent alone on
+    // the GPU gains nothing beside other streams (5184 x 5184 x 144 on 64 x 64
+    // tiles 199 us against 205; the FP64 iteration at D=6, chi=144 then 15.98 it/s
+    // against 16.00 - 16.07), one that is far ahead does (2500 x 2500 x 100: 46
+    // us against 59).
     std::vector<TuneChoice> cands;
-    if (small) cands.push_back(TuneChoice{1, 1, 1});
     if (pipe) {
       const int h = pipe_ksplit(g);
-      for (int k = 1; k <= h; k += std::max(1, h - 1))
-        if (fits(k)) cands.push_back(TuneChoice{4, 1, k});
+      if (fits(h)) cands.push_back(TuneChoice{4, 1, h});
+      if (h > 1) cands.push_back(TuneChoice{4, 1, 1});
     }
+    const float lead = cands.empty() ? 1.f : 0.95f;
+    if (small) cands.push_back(TuneChoice{1, 1, 1});
     const Tile tiles[8] = {{1, 5},    {2, 5},    {2, 2},    {4, 4},
                            {2, 5, 1}, {2, 5, 2}, {2, 5, 3}, {1, 5, 3}};
     for (const Tile& t : tiles) {
@@ -938,7 +945,7 @@ void gemm_f64(const GemmDesc& g, const GemmBatch& b, double* work, size_t work_e
         cands.push_back(c);
       }
     }
-    autotune_run(key, cands, s, launch_choice);
+    autotune_run(key, cands, s, launch_choice, lead);
     return;
   }
   if (!listed) {

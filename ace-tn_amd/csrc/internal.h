@@ -170,9 +170,10 @@ bool autotune_lookup(const TuneKey& k, TuneChoice* out);
 // whether this product should be tuned now (mode 1, shape not in the table,
 // beta == 0, stream not capturing)
 bool autotune_should_tune(const TuneKey& k, const GemmDesc& g, hipStream_t s);
-// times every candidate through ``launch`` on s, stores and re-runs the fastest
+// times every candidate through ``launch`` on s, stores and re-runs the fastest;
+// the first is kept unless another takes less than ``lead`` times its time
 TuneChoice autotune_run(const TuneKey& k, const std::vector<TuneChoice>& cands, hipStream_t s,
-                        const std::function<void(const TuneChoice&)>& launch);
+                        const std::function<void(const TuneChoice&)>& launch, float lead = 1.f);
 int64_t autotune_entries();
 void autotune_clear();
 void autotune_save(const char* path);
