@@ -500,14 +500,14 @@ size_t acetn_hip_svd_workspace(int64_t rows, int64_t cols);
 int acetn_hip_svd(const double* M, int64_t rows, int64_t cols, int64_t ldc, double* s, double* U,
                   int32_t* host_sweeps, void* workspace, size_t ws_bytes, void* stream);
 
-/* Symmetric eigen-decomposition (descending) of a q x q matrix (G is
- * overwritten).  Replaces torch.linalg.eigh at acetn/evolution/full_update.py:283. */
 /* The SVD behind the projectors: eigenvalues w (q, descending) of B B^T and
  * left singular vectors U (q x q, columns) of B given as BT = B^T (n x q). */
 size_t acetn_hip_gram_svd_workspace(int64_t n, int64_t q);
 int acetn_hip_gram_svd(const double* BT, int64_t n, int64_t q, double* w, double* U,
                        void* workspace, size_t workspace_bytes, void* stream);
 
+/* Symmetric eigen-decomposition (descending) of a q x q matrix (G is
+ * overwritten).  Replaces torch.linalg.eigh at acetn/evolution/full_update.py:283. */
 size_t acetn_hip_eigh_workspace(int64_t q);
 int acetn_hip_eigh(double* G, int64_t q, double* w, double* V, void* workspace,
                    size_t ws_bytes, void* stream);
