@@ -6,7 +6,7 @@
 // four tile shapes, each with split-K counts around its default that fit the
 // caller's scratch, and the pipelined and the small FP64 product where they take
 // it) on the caller's stream with HIP events, keeps the fastest (the pipelined
-// one unless another is 5 % faster), and re-runs it so that the result is the
+// one unless another is 10 % faster), and re-runs it so that the result is the
 // chosen kernel's.  Later
 // products of that shape use the table; a CTMRG iteration repeats the same
 // shapes, so one warmup iteration tunes a whole run.  The table can be saved

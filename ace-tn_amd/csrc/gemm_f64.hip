@@ -917,7 +917,7 @@ void gemm_f64(const GemmDesc& g, const GemmBatch& b, double* work, size_t work_e
   if (!listed && autotune_should_tune(key, g, s)) {
     // The pipelined kernel leads: a tile that beats it by a few percent alone on
     // the GPU gains nothing beside other streams (5184 x 5184 x 144 on 64 x 64
-    // tiles 199 us against 205; the FP64 iteration at D=6, chi=144 then 15.98 it/s
+    // tiles 194 - 199 us against 205; the FP64 iteration at D=6, chi=144 then 15.98 it/s
     // against 16.00 - 16.07), one that is far ahead does (2500 x 2500 x 100: 46
     // us against 59).
     std::vector<TuneChoice> cands;
@@ -926,7 +926,7 @@ void gemm_f64(const GemmDesc& g, const GemmBatch& b, double* work, size_t work_e
       if (fits(h)) cands.push_back(TuneChoice{4, 1, h});
       if (h > 1) cands.push_back(TuneChoice{4, 1, 1});
     }
-    const float lead = cands.empty() ? 1.f : 0.95f;
+    const float lead = cands.empty() ? 1.f : 0.9f;
     if (small) cands.push_back(TuneChoice{1, 1, 1});
     const Tile tiles[8] = {{1, 5},    {2, 5},    {2, 2},    {4, 4},
                            {2, 5, 1}, {2, 5, 2}, {2, 5, 3}, {1, 5, 3}};
